@@ -237,8 +237,7 @@ hs_status hs_op_gemm_i8(hs_device *dev, const int8_t *w, const int8_t *a, size_t
                         size_t k, int32_t *out);
 /* As hs_op_gemm_i8 with the K dimension cut into `splits` slices (1..=16; a slice holds at
  * least 64 of K, so fewer slices run when K is short) whose exact i32 partial products are
- * summed on the GPU (ops.rs:163-184 matmul_i8_split). The forward pass uses the same split for
- * decode-shaped products (at most 512 rows). */
+ * summed on the GPU (ops.rs:163-184 matmul_i8_split). */
 hs_status hs_op_gemm_i8_split(hs_device *dev, const int8_t *w, const int8_t *a, size_t m, size_t n,
                               size_t k, uint32_t splits, int32_t *out);
 /* out[i * n + r] = w[r] . a[i] for i16 activations a [m, k] (host pointers), exact i64: the two

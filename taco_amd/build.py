@@ -15,7 +15,8 @@ CXX = os.environ.get("CXX", "g++")
 # Host-only sources go through the host compiler; the HIP runtime calls and kernels through hipcc.
 HOST_SOURCES = {"common.cpp", "hsm.cpp", "taco/harness.cpp", "taco/tokenizer.cpp"}
 
-BACKEND_SOURCES = ["common.cpp", "hsm.cpp", "hs_api.cpp", "kernels.hip"]
+BACKEND_SOURCES = ["common.cpp", "hsm.cpp", "hs_api.cpp", "kernels.hip",
+                   "gemm_rows.hip"]
 HARNESS_SOURCES = ["taco/harness.cpp", "taco/tokenizer.cpp"]  # hs::fail, sha256: the backend's (one error state)
 
 LIB_BACKEND = os.path.join(HERE, "libhardshell_hip.so")

@@ -592,8 +592,6 @@ struct hs_batch {
     bool inflight = false;  // a pass returned with copies or kernels still queued on `st`
     void *split = nullptr;  // scratch of the split decode attention (grown on demand)
     size_t split_bytes = 0;
-    int32_t *gsplit = nullptr;  // i32 partials of the split-K decode products (grown on demand)
-    size_t gsplit_elems = 0;
     int8_t *d_a = nullptr, *d_qkv = nullptr, *d_att = nullptr, *d_g = nullptr, *d_af = nullptr;
     int64_t *d_logits = nullptr;
     uint16_t *d_d16 = nullptr;
@@ -628,7 +626,6 @@ struct hs_batch {
                         (void *)h_mix, (void *)h_stats, (void *)h_intervals2})
             if (p) (void)hipHostFree(p);
         if (split) (void)hipFree(split);
-        if (gsplit) (void)hipFree(gsplit);
         if (st) (void)hipStreamDestroy(st);
     }
     hipError_t event(hipEvent_t &e) {
@@ -1031,36 +1028,10 @@ hs_status run_pass(hs_batch &b, const std::vector<PassRow> &rows, Out out, const
             g.gelu_lo = gspan->gelu_lo; g.gelu_clo = gspan->gelu_clo; g.gelu_chi = gspan->gelu_chi;
             g.gelu_shift = gspan->gelu_shift; g.gelu_copy = gspan->gelu_copy;
         }
-        g.partials = b.gsplit; g.partials_cap = b.gsplit_elems;
         const uint64_t ops = 2ull * (uint64_t)rows_n * (uint64_t)lin.n * (uint64_t)lin.k;
         return b.launch(label, ops, [&] { return hs::launch_gemm(epi, g, st); });
     };
     const bool kv_fused = m.hd % 16 == 0 && m.d % 16 == 0;
-    // Decode-shaped passes (at most two 256-row tiles): the layer products split K where the
-    // launcher's plan says so; their partials need a scratch, grown here before any launch.
-    if (n <= 2 * hs::GEMM_BM) {
-        size_t need = 0;
-        auto want = [&](Epi e, const DevLinear &lin) {
-            const int sp = hs::gemm_split_plan(e, n, lin.n, lin.k_pad, 0);
-            if (sp > 1) need = std::max(need, hs::gemm_split_elems(n, lin.n, sp));
-        };
-        for (const DevBlock &blk : m.blocks) {
-            want(Epi::Act, blk.c_attn);
-            want(Epi::Residual, blk.c_proj);
-            want(blk.gelu16 ? Epi::GeluWide : Epi::Gelu, blk.c_fc);
-            if (!blk.gelu16) want(Epi::Residual, blk.mlp_proj);
-        }
-        if (need > b.gsplit_elems) {
-            if (b.gsplit) {
-                HIP_TRY(hipStreamSynchronize(st));
-                HIP_TRY(hipFree(b.gsplit));
-                b.gsplit = nullptr;
-                b.gsplit_elems = 0;
-            }
-            HIP_TRY(hipMalloc((void **)&b.gsplit, need * sizeof(int32_t)));
-            b.gsplit_elems = need;
-        }
-    }
     // Decode-shaped passes (short runs): attention split over key chunks when the scratch fits
     // (at most 1 GiB), else the row kernel.
     bool split_attn = false;
@@ -1098,7 +1069,6 @@ hs_status run_pass(hs_batch &b, const std::vector<PassRow> &rows, Out out, const
             g.ldo = 3 * m.d; g.fast32 = blk.c_attn.fast32;
             g.kv_rows = b.d_rows; g.kc = b.kc[l]; g.vc = b.vc[l];
             g.kv_d = m.d; g.kv_hd = m.hd; g.kv_h = m.H; g.kv_ctx = m.C;
-            g.partials = b.gsplit; g.partials_cap = b.gsplit_elems;
             const uint64_t ops = 2ull * (uint64_t)n * (uint64_t)blk.c_attn.n * (uint64_t)blk.c_attn.k;
             HIP_TRY(b.launch("gemm_qkv", ops, [&] { return hs::launch_gemm(Epi::Act, g, st); }));
         } else {
@@ -1447,8 +1417,7 @@ extern "C" void hs_op_gemm_layout(size_t m, size_t n, size_t k, size_t *m_pad, s
 
 namespace {
 
-// `splits`: 0 lets the launcher choose the K slices (as the forward pass does), 1 runs one
-// workgroup per tile over all of K, 2..16 forces that many slices.
+// `splits`: 2..16 sums that many slices of K in a second kernel (Raw); 0 and 1 do not split.
 hs_status gemm_host(hs_device *dev, Epi epi, const int8_t *w, const int8_t *a, const int32_t *bias,
                     const int32_t *mult, uint8_t shift, size_t m, size_t n, size_t k, void *out,
                     int splits = 0) {
@@ -1480,7 +1449,7 @@ hs_status gemm_host(hs_device *dev, Epi epi, const int8_t *w, const int8_t *a, c
     g.params_padded = 1;
     g.fast32 = fits_i32(k, bias, bias ? n : 0);
     g.splits = splits;
-    const int sp = hs::gemm_split_plan(epi, (int)m, (int)n, (int)kp, splits);
+    const int sp = hs::gemm_split_plan((int)kp, splits);
     if (sp > 1) {
         g.partials_cap = hs::gemm_split_elems((int)m, (int)n, sp);
         if ((s = mem.alloc(g.partials, g.partials_cap)) != HS_OK) return s;
@@ -1540,7 +1509,7 @@ extern "C" hs_status hs_op_gemm_i8_i16(hs_device *dev, const int8_t *w, const in
     hs::GemmArgs g;
     g.a = da; g.w = dw; g.m = (int)(2 * m); g.n = (int)n; g.k_pad = (int)kp;
     g.out = planes; g.ldo = (int)n; g.splits = (int)splits;
-    const int sp = hs::gemm_split_plan(Epi::Raw, g.m, g.n, g.k_pad, g.splits);
+    const int sp = hs::gemm_split_plan(g.k_pad, g.splits);
     if (sp > 1) {
         g.partials_cap = hs::gemm_split_elems(g.m, g.n, sp);
         if ((s = mem.alloc(g.partials, g.partials_cap)) != HS_OK) return s;
@@ -1572,18 +1541,6 @@ extern "C" hs_status hs_op_gemm_requant_i8_dev(hs_device *dev, const int8_t *w, 
     g.a = a; g.w = w; g.m = (int)m; g.n = (int)n; g.k_pad = (int)kp;
     g.bias = bias; g.mult = mult; g.shift = shift; g.out = out; g.ldo = (int)n;
     hipStream_t st = stream ? (hipStream_t)stream : dev->stream;
-    const int sp = hs::gemm_split_plan(Epi::Act, (int)m, (int)n, (int)kp, 0);
-    if (sp > 1) {  // the split-K partials in stream-ordered memory
-        g.partials_cap = hs::gemm_split_elems((int)m, (int)n, sp);
-        void *p = nullptr;
-        HIP_TRY(hipMallocAsync(&p, g.partials_cap * sizeof(int32_t), st));
-        g.partials = (int32_t *)p;
-        const hipError_t e = hs::launch_gemm(Epi::Act, g, st);
-        const hipError_t f = hipFreeAsync(p, st);
-        HIP_TRY(e);
-        HIP_TRY(f);
-        return HS_OK;
-    }
     HIP_TRY(hs::launch_gemm(Epi::Act, g, st));
     return HS_OK;
 }
@@ -1748,15 +1705,6 @@ extern "C" hs_status hs_op_gemm_requant_gpu_ns(hs_device *dev, const int8_t *w, 
     g.a = a; g.w = w; g.m = (int)m; g.n = (int)n; g.k_pad = (int)kp;
     g.bias = bias; g.mult = mult; g.shift = shift; g.out = out; g.ldo = (int)n;
     g.fast32 = fits_i32(k, hb.data(), n);
-    // the split-K scratch of decode-shaped products, as the forward pass has it (outside the
-    // timed launches)
-    const int sp = hs::gemm_split_plan(Epi::Act, (int)m, (int)n, (int)kp, 0);
-    DevMem mem;
-    if (sp > 1) {
-        g.partials_cap = hs::gemm_split_elems((int)m, (int)n, sp);
-        hs_status s = mem.alloc(g.partials, g.partials_cap);
-        if (s != HS_OK) return s;
-    }
     return time_reps(dev, reps, ns, [&] { return hs::launch_gemm(Epi::Act, g, dev->stream); });
 }
 

@@ -72,13 +72,11 @@ struct GemmArgs {
     const struct RowInfo *kv_rows = nullptr;
     int8_t *kc = nullptr, *vc = nullptr;
     int kv_d = 0, kv_hd = 0, kv_h = 0, kv_ctx = 0;
-    // Split-K (decode-shaped products: one or two M-tiles, few N tiles): when `partials` is set
-    // and the shape gains from it, the workgroups of a tile take slices of K and write exact i32
-    // partials, and an elementwise pass sums them and applies the epilogue. partials_cap is the
-    // scratch size in i32 elements (gemm_split_elems of the chosen split must fit).
+    // Split-K (Raw, on the caller's wish): K in `splits` slices (2..16) whose exact i32 partials
+    // go to `partials` (gemm_split_elems elements) and are summed by a second kernel.
     int32_t *partials = nullptr;
-    size_t partials_cap = 0;
-    int splits = 0;  // 0: chosen by gemm_split_plan; 1: no split; 2..16: that many slices
+    size_t partials_cap = 0;  // in i32 elements
+    int splits = 0;           // 0 or 1: no split
     int kslice = 0;  // set by the launcher: bytes of K per slice (a multiple of GEMM_BK)
 };
 
@@ -109,9 +107,9 @@ struct KernelResource {
 };
 int kernel_resources(KernelResource *out, int cap);
 
-// The split-K plan of a product: the number of K slices (1 = no split) for m rows, n columns and
-// k_pad bytes of K with the given epilogue, and the i32 partial elements it needs.
-int gemm_split_plan(Epi epi, int m, int n, int k_pad, int splits_wanted);
+// The K slices of a product whose caller wants `splits_wanted` (1: no split), and the i32 partial
+// elements they need.
+int gemm_split_plan(int k_pad, int splits_wanted);
 size_t gemm_split_elems(int m, int n, int splits);
 // out[i][r] = 256 planes[2i][r] + planes[2i + 1][r] + 128 wsum[r] (i64), planes [2m, n] i32.
 hipError_t launch_wide_combine(const int32_t *planes, const int32_t *wsum, int m, int n, int64_t *out,

@@ -4,7 +4,6 @@
 // Reductions are fixed-order wave/LDS trees, and the only atomics are the coder op's integer
 // histogram counts in LDS, whose sums do not depend on order: results do not depend on
 // scheduling.
-#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <map>
@@ -13,35 +12,19 @@
 
 #include "intmath.h"
 #include "kernels.h"
+#include "launch.h"
 
 namespace hs {
 
-// ---- kernel launches and their profiling events -------------------------------------------------
-// The caller of an op may hand it a pair of events (set_op_events): the first kernel the op
-// launches then records `start` as it begins and every one records `stop` as it ends (the
-// events ride on the dispatches, hipExtLaunchKernelGGL), so stop - start is the op's GPU time
-// with no event packets between its kernels.
-static thread_local hipEvent_t t_op_start = nullptr, t_op_stop = nullptr;
-static thread_local int t_op_launches = 0;
-
-void set_op_events(hipEvent_t start, hipEvent_t stop) {
-    t_op_start = start;
-    t_op_stop = stop;
-    t_op_launches = 0;
+// ---- kernel launches and their profiling events (launch.h) --------------------------------------
+OpEvents &op_events() {
+    static thread_local OpEvents ev;
+    return ev;
 }
 
-int op_launches() { return t_op_launches; }
+void set_op_events(hipEvent_t start, hipEvent_t stop) { op_events() = OpEvents{start, stop, 0}; }
 
-template <typename K, typename... Args>
-static inline void launch_k(K kernel, dim3 grid, dim3 block, size_t lds, hipStream_t stream, Args... args) {
-    if (t_op_stop) {
-        hipExtLaunchKernelGGL(kernel, grid, block, (uint32_t)lds, stream, t_op_launches == 0 ? t_op_start : nullptr,
-                              t_op_stop, 0u, args...);
-        t_op_launches++;
-    } else {
-        hipLaunchKernelGGL(kernel, grid, block, lds, stream, args...);
-    }
-}
+int op_launches() { return op_events().launches; }
 
 // ---- launch attributes, per kernel and device ---------------------------------------------------
 // A kernel's dynamic-LDS limit is raised on the current device before its first launch that needs
@@ -50,7 +33,7 @@ static inline void launch_k(K kernel, dim3 grid, dim3 block, size_t lds, hipStre
 // host threads at once (one batch per thread), so both caches sit behind one mutex.
 static std::mutex g_attr_mutex;
 
-static hipError_t allow_dynamic_lds(const void *fn, size_t bytes) {
+hipError_t allow_dynamic_lds(const void *fn, size_t bytes) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
@@ -88,8 +71,6 @@ static hipError_t resident_workgroups(const void *fn, int threads, size_t lds, i
     return hipSuccess;
 }
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-constexpr int32_t RES = (1 << 30) - 1;             // gpt2/mod.rs:116
 constexpr int64_t SCORE_LIMIT = (int64_t)1 << 40;  // gpt2/mod.rs:119
 
 __device__ __forceinline__ int32_t med3_i32(int32_t x, int32_t lo, int32_t hi) {
@@ -165,11 +146,11 @@ struct Flag {
 // BN = 128 (4 waves, 2 x 2) or 256 (8 waves, 2 x 4); every wave computes 128 x 64.
 // VEC: the output rows are 16-byte aligned (checked by the launcher); the four-columns epilogues
 // then stage and store 16-byte pieces, else they store each output on its own.
-// BM x BN tiles: 256 x 64 (2 x 1 waves), 256 x 128 (2 x 2), 256 x 256 (2 x 4, the full-line
-// loop), 128 x 192 (2 x 2 waves of 64 x 96) and 64 x 64 (2 x 1 waves of 32 x 64, decode
-// passes). Each wave computes a (BM / 2) x (BN / WN) sub-tile: TI x TJ tiles of 16 x 16.
+// BM x BN tiles: 256 x 128 (2 x 2 waves), 256 x 256 (2 x 4, the full-line
+// loop), 128 x 192 (2 x 2 waves of 64 x 96) and 64 x 64 (2 x 1 waves of 32 x 64, small
+// products). Each wave computes a (BM / 2) x (BN / WN) sub-tile: TI x TJ tiles of 16 x 16.
 constexpr int gemm_wn(int bn) { return bn == 192 ? 2 : bn / 64; }  // waves along N
-// The ring's stages: 3, or 6 for the 64 x 64 tiles of decode passes with K >= 1,024 (DEEP: their
+// The ring's stages: 3, or 6 for the 64 x 64 tiles with K >= 1,024 (DEEP: their
 // k-steps hold little MFMA work, so more k-steps of loads stay in flight; one workgroup per CU at
 // most there). Measured, GPT-2-medium unfold passes: c_attn and c_fc (K 1,024) 7-10% and
 // mlp.c_proj (K 4,096) 18% faster; the GPT-2-small c_attn (K 768) 6.0 -> 6.4 us, so it keeps 3.
@@ -352,7 +333,7 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
     const size_t pa = (size_t)g.a_rows * 64, pw = (size_t)g.w_rows * 64;  // bytes per panel
     // A load's address is a wave-uniform fragment base (scalar registers, recomputed by scalar
     // instructions each k-step) plus the lane's 32-bit offset inside the fragment, the same for
-    // every load (one vector add per load). The 64 x 64 tiles of decode passes, whose k-steps hold
+    // every load (one vector add per load). The 64 x 64 tiles, whose k-steps hold
     // 8 MFMAs per wave, keep a per-lane pointer per load instead: their loop is too short to hide
     // the scalar work (GPT-2-medium unfold GEMMs 2-4% slower with the shared form).
     const uint32_t lane_off = (uint32_t)((lane >> 2) * 64 + (((lane & 3) ^ sw(lane >> 2)) * 16));
@@ -738,7 +719,7 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
         // Act, Gelu, GeluWide: i8 outputs (GeluWide: the two planes of each i16 output), staged
         // per wave in LDS (the wave's rows x RS8 bytes) and stored as 16-byte row pieces. Gelu copies its
         // table's span (gelu_copy bytes from entry gelu_lo) into LDS first; the staging regions
-        // follow it. The 64 x 64 tiles of decode passes read the table through the caches instead
+        // follow it. The 64 x 64 tiles read the table through the caches instead
         // (a copy per workgroup would outweigh the 4,096 lookups of its tile).
         constexpr bool GELU_LDS = BM != 64;
         const int8_t *gspan = g.gelu + g.gelu_lo;  // entry gelu_lo: index 0 of the lookups
@@ -971,11 +952,17 @@ static hipError_t launch_gemm_t(const GemmArgs &ga, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// Decode-shaped products (at most two 256-row tiles of rows, K at most 4,096) take 64 x 64 tiles
-// over the whole of K (more workgroups than 128 x 192 tiles, no partials), or, when those tiles
-// are fewer than 128 and K is 2,048 or more, 64 x 64 partial tiles over slices of K
-// (gemm_split_plan); longer K splits in 256 x 64 partial tiles.
-static bool gemm_decode_tiles(int m, int k_pad) { return m <= 2 * GEMM_BM && k_pad <= 4096; }
+// The products that take 64 x 64 tiles over the whole of K: all of at most 512 rows, and larger ones
+// while their 64 x 64 tiles are few enough that the larger tiles would leave CUs idle (the narrow
+// layers of a few thousand rows). Measured against the larger tiles, us a launch: 1024 x 2304 x
+// 768 (576 tiles) 8.6 -> 6.9, 1536 x 2304 x 768 (864) 8.8 -> 7.5, 2048 x 2304 x 768 (1,152) 9.0
+// -> 9.5; residual 3400 x 768 x 768 (648) 13.9 -> 9.3, 2048 x 768 x 3072 (384) 24.6 -> 17.8,
+// 1536 x 1600 x 6400 (600) 42.3 -> 32.1, 2048 x 1600 x 6400 (800) 42.8 -> 51.7: the line lies
+// lower for long K, where the larger tiles' fewer loads per output count for more.
+static bool gemm_small_tiles(int m, int n, int k_pad) {
+    const long long tiles = ((m + 63) / 64) * (long long)((n + 63) / 64);
+    return m <= 2 * GEMM_BM || tiles <= (k_pad <= 1024 ? 900 : 640);
+}
 
 // 256 x 128 tiles (two workgroups per CU, so one's epilogue overlaps the other's main loop),
 // or 256 x 256 (below). Outputs whose rows are not 16-byte aligned take the per-output store
@@ -994,13 +981,9 @@ static hipError_t launch_gemm_w(const GemmArgs &g, hipStream_t stream) {
         constexpr bool PANEL_OUT = EPI == (int)Epi::Gelu || EPI == (int)Epi::GeluWide;
         const bool vec = ((uintptr_t)g.out & 15) == 0 && (PANEL_OUT || ((size_t)g.ldo * ES) % 16 == 0);
         if (!vec) return launch_gemm_t<EPI, NARROW, 128, false>(g, stream);
-        // Decode passes (at most two 256-row tiles of rows) with K up to 4,096: 64 x 64 tiles,
-        // two waves each (a 256-row pass of GPT-2 medium's c_attn: 192 workgroups instead of 24
-        // of 128 x 192 or 288 split-K slices and their summing pass; measured 16.0 -> 7.0 us,
-        // mlp.c_proj (K 4,096) 19.4 -> 16.1 us, the M 256 c_attn of GPT-2 small 10.2 -> 6.1 us).
         if constexpr (EPI == (int)Epi::Act || EPI == (int)Epi::Residual || EPI == (int)Epi::Gelu ||
                       EPI == (int)Epi::GeluWide || EPI == (int)Epi::Raw) {
-            if (gemm_decode_tiles(g.m, g.k_pad)) {
+            if (gemm_small_tiles(g.m, g.n, g.k_pad)) {
                 if (g.k_pad >= 1024) return launch_gemm_t<EPI, NARROW, 64, true, 64, true>(g, stream);
                 return launch_gemm_t<EPI, NARROW, 64, true, 64>(g, stream);
             }
@@ -1044,60 +1027,23 @@ static hipError_t launch_gemm_e(const GemmArgs &g, hipStream_t stream) {
     return launch_gemm_w<EPI, false>(g, stream);
 }
 
-// ---- Split-K for decode-shaped products ------------------------------------------------------
-// A pass of at most 512 rows has one or two 256-row M-tiles, so an N-tiled product launches
-// N / 128 workgroups, each walking all of K: a few dozen of the 256 CUs, each bound by the latency
-// of its k-steps (GPT-2 medium's mlp.c_proj: 8 workgroups x 64 k-steps). Here 64-column tiles
-// take slices of K (2 to 16 workgroups per tile), write exact i32 partials (|each| <= 2^30, and
-// i32 sums of them are exact in any order), and k_split_epi sums a tile's slices per output and
-// applies the epilogue's rule to the total: the epilogue is not linear, so it runs once, on the
-// exact product.
-
-constexpr int SPLIT_BN = 64;
-
+// ---- Split-K of a Raw product, on the caller's wish (matmul_i8_split, ops.rs:163-184) -------------
+// Slices of K in 64 x 64 tiles write exact i32 partials (|each| <= 2^30, and i32 sums of them are
+// exact in any order), and k_split_sum_raw adds a tile's slices. (The layers' products of few rows
+// split K inside a workgroup instead: gemm_rows.hip.)
 
 size_t gemm_split_elems(int m, int n, int splits) {
     return (size_t)splits * (size_t)m * (size_t)((n + 3) & ~3);
 }
 
-int gemm_split_plan(Epi epi, int m, int n, int k_pad, int wanted) {
-    const bool ok = epi == Epi::Raw || epi == Epi::Act || epi == Epi::Residual || epi == Epi::Gelu ||
-                    epi == Epi::GeluWide;
-    if (!ok || m <= 0 || n <= 0 || k_pad < 2 * GEMM_BK) return 1;
+int gemm_split_plan(int k_pad, int wanted) {
     const int nks = k_pad / GEMM_BK;
-    if (wanted >= 1) return wanted > nks ? nks : wanted;
-    if (gemm_decode_tiles(m, k_pad)) {
-        // 64 x 64 tiles over the whole of K, unless they are too few for the GPU and K is long:
-        // then 64 x 64 partials over slices of at least 16 k-steps (GPT-2 medium's mlp.c_proj in
-        // a 256-row pass: 256 workgroups of 16 k-steps instead of 64 of 64)
-        const int tiles64 = ((m + 63) / 64) * ((n + 63) / 64);
-        if (tiles64 >= 128 || k_pad < 2048) return 1;
-        int sp = (256 + tiles64 - 1) / tiles64;
-        sp = sp < nks / 16 ? sp : nks / 16;
-        sp = sp > 16 ? 16 : sp;
-        return sp < 2 ? 1 : sp;
-    }
-    const int gm = (m + GEMM_BM - 1) / GEMM_BM, tiles128 = gm * ((n + 127) / 128);
-    // enough workgroups without a split, or K too short for the partials to pay (measured: the
-    // c_attn product at M 256, K 768 takes 12.3 us whole and 13.5 us in three slices; at K 1,024
-    // and 4,096 the GPT-2-medium decode products take 1.9 instead of 3.2 ms per pass)
-    if (gm > 2 || tiles128 >= 96 || k_pad < 1024) return 1;
-    // about 256 workgroups of 64-column tiles, at least 4 k-steps each, and the partials
-    // (4 B per output and slice) at most about four times the weight bytes
-    const int tiles = gm * ((n + SPLIT_BN - 1) / SPLIT_BN);
-    int sp = (256 + tiles - 1) / tiles;
-    sp = sp < nks / 4 ? sp : nks / 4;
-    const int by_bytes = (int)((4ll * k_pad) / (4ll * gm * GEMM_BM));
-    sp = sp < by_bytes ? sp : by_bytes;
-    sp = sp > 16 ? 16 : sp;
-    return sp < 2 ? 1 : sp;
+    return wanted > nks ? nks : (wanted > 1 ? wanted : 1);
 }
 
-// Sums the `splits` partials of one output row x 4 columns and applies the epilogue rule of the
-// fused kernels to the exact product (Raw: the sum itself). A whole group of 4 columns whose
-// destination is 4-byte aligned (16-byte for the i32 outputs) is stored with one access.
-template <int EPI>
-__global__ __launch_bounds__(256) void k_split_epi(GemmArgs g, int splits, int ldp) {
+// Sums the `splits` partials of one output row x 4 columns. A whole group of 4 columns whose
+// destination is 16-byte aligned is stored with one access.
+__global__ __launch_bounds__(256) void k_split_sum_raw(GemmArgs g, int splits, int ldp) {
     const int groups = ldp / 4;
     const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
     const int m = (int)(idx / groups), n4 = (int)(idx % groups) * 4;
@@ -1114,80 +1060,13 @@ __global__ __launch_bounds__(256) void k_split_epi(GemmArgs g, int splits, int l
     }
     for (; sl < splits; sl++) acc += *(const v4i *)(src + sl * slice);
     const int cnt = g.n - n4 < 4 ? g.n - n4 : 4;
-    if (EPI == (int)Epi::Raw) {
-        int32_t *o = (int32_t *)g.out + (size_t)m * g.ldo + n4;
-        if (cnt == 4 && ((uintptr_t)o & 15) == 0) *(v4i *)o = acc;
-        else
-            for (int e = 0; e < cnt; e++) o[e] = acc[e];
-        return;
-    }
-    // rescale(a + bias, mult, shift) (int.rs:63-67): |a + bias| < 2^32, exact in i64
-    int64_t r[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++)
-        r[e] = e < cnt ? rescale_small((int64_t)acc[e] + g.bias[n4 + e], g.mult[n4 + e], (uint32_t)g.shift) : 0;
-    if (EPI == (int)Epi::Residual) {  // ops.rs:131-145: x = clamp(x + sat32(r), +-R)
-        int32_t *x = (int32_t *)g.out + (size_t)m * g.ldo + n4;
-        if (cnt == 4 && ((uintptr_t)x & 15) == 0) {
-            v4i v = *(const v4i *)x;
-#pragma unroll
-            for (int e = 0; e < 4; e++) v[e] = (int32_t)clamp64((int64_t)v[e] + clamp64(r[e], INT32_MIN, INT32_MAX), -RES, RES);
-            *(v4i *)x = v;
-        } else {
-            for (int e = 0; e < cnt; e++)
-                x[e] = (int32_t)clamp64((int64_t)x[e] + clamp64(r[e], INT32_MIN, INT32_MAX), -RES, RES);
-        }
-        return;
-    }
-    uint32_t b[4];  // the i8 outputs (GeluWide: the i16 values)
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        if (EPI == (int)Epi::Act) {  // ops.rs:123-130
-            b[e] = (uint32_t)clamp64(r[e], -127, 127);
-        } else {  // table[clamp(r, -off, off - 1) + off] (ops.rs:146-154, gelu.rs:58-62)
-            const int t = (int)clamp64(r[e], -g.gelu_off, g.gelu_off - 1) + g.gelu_off;
-            b[e] = EPI == (int)Epi::Gelu ? (uint32_t)g.gelu[t] : (uint32_t)g.gelu16[t];
-        }
-    }
-    auto store4 = [&](int8_t *o, auto byte) {
-        if (cnt == 4 && ((uintptr_t)o & 3) == 0) {
-            *(uint32_t *)o = (byte(0) & 255) | ((byte(1) & 255) << 8) | ((byte(2) & 255) << 16) | ((byte(3) & 255) << 24);
-        } else {
-            for (int e = 0; e < cnt; e++) o[e] = (int8_t)byte(e);
-        }
-    };
-    if (EPI == (int)Epi::Act) {
-        if (g.kv_rows && n4 >= g.kv_d) {
-            // K or V of the row into the cache: kv_d and kv_hd are multiples of 4, so the group
-            // lies in one head of one part; the columns past 3 kv_d are padding
-            if (n4 >= 3 * g.kv_d) return;
-            const RowInfo ri = g.kv_rows[m];
-            const int part = n4 >= 2 * g.kv_d, c = n4 - (part + 1) * g.kv_d;
-            const int hh = c / g.kv_hd, cc = c - hh * g.kv_hd;
-            store4((part ? g.vc : g.kc) + (((size_t)ri.slot * g.kv_h + hh) * g.kv_ctx + ri.pos) * g.kv_hd + cc,
-                   [&](int e) { return b[e]; });
-        } else {
-            store4((int8_t *)g.out + (size_t)m * g.ldo + n4, [&](int e) { return b[e]; });
-        }
-    } else if (EPI == (int)Epi::Gelu) {  // the operand of the next product, in panels
-        store4((int8_t *)g.out + panel_off(m, n4, g.out_rows), [&](int e) { return b[e]; });
-    } else {  // GeluWide: the two planes of each i16 output, hi = v >> 8, lo = (v & 255) - 128
-        store4((int8_t *)g.out + panel_off(2 * (size_t)m, n4, g.out_rows),
-               [&](int e) { return (uint32_t)((int32_t)(int16_t)b[e] >> 8); });
-        store4((int8_t *)g.out + panel_off(2 * (size_t)m + 1, n4, g.out_rows),
-               [&](int e) { return (uint32_t)(((int32_t)(int16_t)b[e] & 255) - 128); });
-    }
+    int32_t *o = (int32_t *)g.out + (size_t)m * g.ldo + n4;
+    if (cnt == 4 && ((uintptr_t)o & 15) == 0) *(v4i *)o = acc;
+    else
+        for (int e = 0; e < cnt; e++) o[e] = acc[e];
 }
 
-template <int EPI>
-static hipError_t launch_split_epi(const GemmArgs &g, int splits, int ldp, hipStream_t stream) {
-    const long long threads = (long long)g.m * (ldp / 4);
-    launch_k(k_split_epi<EPI>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, g,
-                       splits, ldp);
-    return hipGetLastError();
-}
-
-static hipError_t launch_gemm_split(Epi epi, const GemmArgs &ga, int splits, hipStream_t stream) {
+static hipError_t launch_gemm_split(const GemmArgs &ga, int splits, hipStream_t stream) {
     if (ga.group < 1 || ga.group > (ga.m + GEMM_BM - 1) / GEMM_BM || splits < 2 || splits > 16)
         return hipErrorInvalidValue;
     GemmArgs p = ga;  // the partial products: Raw into the scratch, [splits][m][ldp]
@@ -1197,42 +1076,17 @@ static hipError_t launch_gemm_split(Epi epi, const GemmArgs &ga, int splits, hip
     splits = (ga.k_pad + p.kslice - 1) / p.kslice;  // every slice holds at least one k-step
     p.out = ga.partials;
     p.ldo = ldp;
-    constexpr int EPI_RAW = (int)Epi::Raw;
-    if (gemm_decode_tiles(ga.m, ga.k_pad)) {
-        // decode-shaped: the partials in 64 x 64 tiles (two waves), with the 6-stage ring for
-        // slices of 1,024 or more (as the whole-K 64 x 64 tiles)
-        const int gm = (ga.m + 63) / 64, gn = (ga.n + 63) / 64;
-        p.group = 4 * ga.group < gm ? 4 * ga.group : gm;
-        auto run = [&](auto kernel, int stages) -> hipError_t {
-            const size_t lds = (size_t)stages * 8 * 1024;
-            const hipError_t e = allow_dynamic_lds((const void *)kernel, lds);
-            if (e != hipSuccess) return e;
-            launch_k(kernel, dim3(gm * gn, splits), dim3(64 * gemm_waves(64)), lds, stream, p);
-            return hipGetLastError();
-        };
-        const hipError_t e = p.kslice >= 1024 ? run(k_gemm<EPI_RAW, false, 64, true, 64, true>, gemm_stages(64, true))
-                                              : run(k_gemm<EPI_RAW, false, 64, true, 64>, gemm_stages(64, false));
-        if (e != hipSuccess) return e;
-    } else {
-        constexpr size_t lds = (size_t)GEMM_STAGES * (GEMM_BM / 16 + SPLIT_BN / 16) * 1024;
-        {
-            const hipError_t e = allow_dynamic_lds((const void *)k_gemm<EPI_RAW, false, SPLIT_BN, true>, lds);
-            if (e != hipSuccess) return e;
-        }
-        const int gm = (ga.m + GEMM_BM - 1) / GEMM_BM, gn = (ga.n + SPLIT_BN - 1) / SPLIT_BN;
-        launch_k((k_gemm<EPI_RAW, false, SPLIT_BN, true>), dim3(gm * gn, splits), dim3(64 * gemm_waves(SPLIT_BN)),
-                 lds, stream, p);
-    }
-    hipError_t e = hipGetLastError();
+    const int gm = (ga.m + 63) / 64, gn = (ga.n + 63) / 64;
+    p.group = 4 * ga.group < gm ? 4 * ga.group : gm;
+    constexpr size_t lds = (size_t)gemm_stages(64, false) * 8 * 1024;
+    hipError_t e = allow_dynamic_lds((const void *)k_gemm<(int)Epi::Raw, false, 64, true, 64>, lds);
     if (e != hipSuccess) return e;
-    switch (epi) {
-        case Epi::Raw: return launch_split_epi<0>(ga, splits, ldp, stream);
-        case Epi::Act: return launch_split_epi<1>(ga, splits, ldp, stream);
-        case Epi::Residual: return launch_split_epi<2>(ga, splits, ldp, stream);
-        case Epi::Gelu: return launch_split_epi<3>(ga, splits, ldp, stream);
-        case Epi::GeluWide: return launch_split_epi<6>(ga, splits, ldp, stream);
-        default: return hipErrorInvalidValue;
-    }
+    launch_k((k_gemm<(int)Epi::Raw, false, 64, true, 64>), dim3(gm * gn, splits), dim3(64 * gemm_waves(64)), lds,
+             stream, p);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    const long long threads = (long long)ga.m * (ldp / 4);
+    launch_k(k_split_sum_raw, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, ga, splits, ldp);
+    return hipGetLastError();
 }
 
 // The i16-activation product from its plane rows (matvec_i8_i16, ADR 0004 addendum B):
@@ -1269,13 +1123,15 @@ hipError_t launch_gemm(Epi epi, const GemmArgs &ga, hipStream_t stream) {
     if ((epi == Epi::Gelu && g.out_rows < g.m) || (epi == Epi::GeluWide && g.out_rows < 2 * g.m))
         return hipErrorInvalidValue;
     g.kslice = 0;
-    if (g.partials) {
-        const int sp = gemm_split_plan(epi, g.m, g.n, g.k_pad, g.splits);
+    if (g.splits > 1) {
+        const int sp = gemm_split_plan(g.k_pad, g.splits);
         if (sp > 1) {
-            if (gemm_split_elems(g.m, g.n, sp) > g.partials_cap) return hipErrorInvalidValue;
-            return launch_gemm_split(epi, g, sp, stream);
+            if (epi != Epi::Raw || !g.partials || gemm_split_elems(g.m, g.n, sp) > g.partials_cap)
+                return hipErrorInvalidValue;
+            return launch_gemm_split(g, sp, stream);
         }
     }
+    if (gemm_rows_fits(epi, g)) return launch_gemm_rows(epi, g, stream);
     switch (epi) {
         case Epi::Raw: return launch_gemm_w<0, false>(g, stream);
         case Epi::Act: return launch_gemm_e<1>(g, stream);
@@ -4314,14 +4170,13 @@ int kernel_resources(KernelResource *out, int cap) {
         {"k_gemm<GeluWide, 256x128>", (const void *)k_gemm<6, false, 128, true>},
         {"k_gemm<ResidualWide, 256x128>", (const void *)k_gemm<7, false, 128, true>},
         {"k_gemm<LogitsCompactWide, 256x128>", (const void *)k_gemm<9, false, 128, true>},
-        {"k_gemm<Raw, split-K partials, 256x64>", (const void *)k_gemm<0, false, 64, true>},
+        {"k_gemm<Raw, split-K partials, 64x64>", (const void *)k_gemm<0, false, 64, true, 64>},
         {"k_gemm<Act, narrow, 128x192>", (const void *)k_gemm<1, true, 192, true, 128>},
         {"k_gemm<Residual, narrow, 128x192>", (const void *)k_gemm<2, true, 192, true, 128>},
-        {"k_gemm<Act, narrow, 64x64 decode>", (const void *)k_gemm<1, true, 64, true, 64>},
-        {"k_gemm<Residual, narrow, 64x64 decode>", (const void *)k_gemm<2, true, 64, true, 64>},
-        {"k_gemm<Gelu, narrow, 64x64 decode>", (const void *)k_gemm<3, true, 64, true, 64>},
-        {"k_split_epi<Act>", (const void *)k_split_epi<1>},
-        {"k_split_epi<Residual>", (const void *)k_split_epi<2>},
+        {"k_gemm<Act, narrow, 64x64>", (const void *)k_gemm<1, true, 64, true, 64>},
+        {"k_gemm<Residual, narrow, 64x64>", (const void *)k_gemm<2, true, 64, true, 64>},
+        {"k_gemm<Gelu, narrow, 64x64>", (const void *)k_gemm<3, true, 64, true, 64>},
+        {"k_split_sum_raw", (const void *)k_split_sum_raw},
         {"k_embed", (const void *)k_embed},
         {"k_embed4", (const void *)k_embed4},
         {"k_layernorm", (const void *)k_layernorm},
