@@ -954,6 +954,7 @@ hs_status run_pass(hs_batch &b, const std::vector<PassRow> &rows, Out out, const
     owner.clear();
     owner.reserve(n);
     int n_out = 0;
+    uint32_t kinds = 0;  // nonzero: a Decode query among them
     for (int r = 0; r < n; r++) {
         info[r] = RowInfo{(int32_t)rows[r].slot, (int32_t)rows[r].token, (int32_t)rows[r].pos, -1};
         if (rows[r].input >= 0) {
@@ -963,6 +964,7 @@ hs_status run_pass(hs_batch &b, const std::vector<PassRow> &rows, Out out, const
             if (out == Out::Intervals) {
                 q[2 * n_out] = queries[2 * rows[r].input];
                 q[2 * n_out + 1] = queries[2 * rows[r].input + 1];
+                kinds |= q[2 * n_out];
             }
             n_out++;
         }
@@ -1138,6 +1140,7 @@ hs_status run_pass(hs_batch &b, const std::vector<PassRow> &rows, Out out, const
             ca.d16 = b.d_d16; ca.ld16 = m.ld16; ca.tmax = b.d_tmax; ca.ntiles = m.ntiles; ca.vocab = m.V;
             ca.table = m.logits_exp; ca.table_len = (int)m.host.logits_exp.size(); ca.d0 = m.d0;
             ca.zcut = m.zcut;
+            ca.decode = kinds != 0;
             ca.queries = out == Out::Intervals ? b.d_queries + 2 * c0 : nullptr;
             ca.bits = (int)bits;
             ca.intervals = out == Out::Intervals ? b.d_intervals + 3 * (size_t)c0 : nullptr;
@@ -1991,6 +1994,7 @@ hs_status coder_on_logits(hs_device *dev, const int64_t *logits, size_t rows, si
         while (zcut > 1 && table[zcut - 1] == 0) zcut--;
         cca.d16 = d16; cca.ld16 = (int)ld16; cca.tmax = dtm; cca.ntiles = (int)nt; cca.vocab = (int)vocab;
         cca.table = dt; cca.table_len = (int)len; cca.d0 = d0; cca.zcut = zcut; cca.queries = dq;
+        for (size_t r = 0; r < rows; r++) cca.decode |= queries[r].kind != 0;
         cca.bits = (int)freq_bits; cca.intervals = di; cca.mix = dm; cca.stats = dst;
         launch = [&](int what) {
             if (what == 0) return hs::launch_mix_stats_compact(cca, (int)rows, st);

@@ -250,6 +250,7 @@ struct CompactCoderArgs {
     int d0 = 0;    // the largest d with table[d] == table[0]
     int zcut = 0;  // every table[d] with d >= zcut is 0 (1 <= zcut <= table_len)
     const uint32_t *queries = nullptr;
+    int decode = 0;  // 1: a query may be a Decode one (0 promises Encode queries only)
     int bits = 32;
     uint64_t *intervals = nullptr;
     uint64_t *weights = nullptr;

@@ -6,6 +6,7 @@
 // scheduling.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -3426,30 +3427,35 @@ __device__ __forceinline__ uint64_t block_sum64(uint64_t v, uint64_t *s, int tid
     return v;
 }
 
-// Reductions over a 256-thread block through wave shuffles and one LDS slot per wave.
-__device__ __forceinline__ int64_t block_max64w(int64_t v, int64_t *s4, int tid) {
+// Reductions over a block of NW waves through wave shuffles and one LDS slot per wave.
+template <int NW = 4>
+__device__ __forceinline__ int64_t block_max64w(int64_t v, int64_t *slots, int tid) {
     v = wave_max64(v);
-    if ((tid & 63) == 0) s4[tid >> 6] = v;
+    if ((tid & 63) == 0) slots[tid >> 6] = v;
     __syncthreads();
-    int64_t r = s4[0];
+    int64_t r = slots[0];
 #pragma unroll
-    for (int w = 1; w < 4; w++) r = s4[w] > r ? s4[w] : r;
+    for (int w = 1; w < NW; w++) r = slots[w] > r ? slots[w] : r;
     __syncthreads();
     return r;
 }
 
-__device__ __forceinline__ uint64_t block_sum64w(uint64_t v, uint64_t *s4, int tid) {
+template <int NW = 4>
+__device__ __forceinline__ uint64_t block_sum64w(uint64_t v, uint64_t *slots, int tid) {
     v = (uint64_t)wave_sum64((int64_t)v);
-    if ((tid & 63) == 0) s4[tid >> 6] = v;
+    if ((tid & 63) == 0) slots[tid >> 6] = v;
     __syncthreads();
-    const uint64_t r = s4[0] + s4[1] + s4[2] + s4[3];
+    uint64_t r = slots[0];
+#pragma unroll
+    for (int w = 1; w < NW; w++) r += slots[w];
     __syncthreads();
     return r;
 }
 
-// Exclusive prefix sum over a 256-thread block in thread order, and the block total: wave scans
-// through shuffles, then the four wave totals through one LDS slot per wave.
-__device__ __forceinline__ uint64_t block_scan64w(uint64_t v, uint64_t *s4, int tid, uint64_t &total) {
+// Exclusive prefix sum over a block of NW waves in thread order, and the block total: wave scans
+// through shuffles, then the wave totals through one LDS slot per wave.
+template <int NW = 4>
+__device__ __forceinline__ uint64_t block_scan64w(uint64_t v, uint64_t *slots, int tid, uint64_t &total) {
     const int lane = tid & 63, w = tid >> 6;
     int64_t x = (int64_t)v;
 #pragma unroll
@@ -3457,18 +3463,56 @@ __device__ __forceinline__ uint64_t block_scan64w(uint64_t v, uint64_t *s4, int 
         const int64_t u = __shfl_up(x, o, 64);
         if (lane >= o) x += u;
     }
-    if (lane == 63) s4[w] = (uint64_t)x;
+    if (lane == 63) slots[w] = (uint64_t)x;
     __syncthreads();
     uint64_t before = 0, all = 0;
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const uint64_t t = s4[k];
+    for (int k = 0; k < NW; k++) {
+        const uint64_t t = slots[k];
         before += k < w ? t : 0;
         all += t;
     }
     __syncthreads();
     total = all;
     return before + (uint64_t)x - v;
+}
+
+// The weights of rows of compact logits (run_weights): 2,048 symbols per workgroup, so that the
+// 402 KB a row of GPT-2's vocabulary writes come from 25 CUs (one workgroup per row took 100 us
+// for a row; the row max is redone per workgroup, 6 KB of tile maxes from the caches).
+__global__ __launch_bounds__(256) void k_weights_compact(CompactCoderArgs a) {
+    __shared__ int64_t slots[4];
+    const int row = blockIdx.y, tid = threadIdx.x, V = a.vocab, last = a.table_len - 1;
+    const uint16_t *d16 = a.d16 + (size_t)row * a.ld16;
+    const int64_t *tm = a.tmax + (size_t)row * a.ntiles;
+    const int j0 = blockIdx.x * 2048 + tid;
+    int64_t t8[8];
+    uint16_t d8[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) {  // no branch around the loads: a symbol past the row reads the last one
+        const int j = j0 + 256 * u < V ? j0 + 256 * u : V - 1;
+        t8[u] = tm[j >> 6];
+        d8[u] = d16[j];
+    }
+    int64_t mx = INT64_MIN;
+    for (int t = tid; t < a.ntiles; t += 1024) {
+        int64_t v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = tm[min(t + 256 * u, a.ntiles - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; u++) mx = v[u] > mx ? v[u] : mx;
+    }
+    const int64_t M = block_max64w(mx, slots, tid);
+    uint64_t w8[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+        const int64_t d = M - t8[u] + d8[u];
+        w8[u] = a.table[d < last ? d : last];
+    }
+    uint64_t *out = a.weights + (size_t)row * V;
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+        if (j0 + 256 * u < V) out[j0 + 256 * u] = w8[u];
 }
 
 // One row per workgroup. The histogram counts the symbols of each table index d < zcut (the
@@ -3481,9 +3525,20 @@ __device__ __forceinline__ uint64_t block_scan64w(uint64_t v, uint64_t *s4, int 
 // PACKED: V < 2^16 (the launch picks the form). The histogram is the only sizeable LDS of the
 // workgroup (4 (zcut + 64) bytes); with at most 128 registers four rows share a CU, so a chunk
 // of 2,048 rows runs in two full rounds of 1,024.
-template <bool STATS, bool PACKED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_coder_compact(CompactCoderArgs a) {
-    // LDS: the histogram from address 0 (a bin's byte address is 4 d), then the reduction slots
+// FIND: queries may be Decode ones (a template parameter, so that the fold's Encode launches keep
+// the registers and the S pass they had: 58.6 against 55.2 us per 2,048 rows otherwise). A Decode
+// query finds its symbol from the sums of f over segments of 64 symbols (more for
+// vocabularies above 65,536): f = 1 + q of a symbol's bin by one LDS lookup (the S pass leaves q in
+// the histogram's place), a scan over the segment sums, and one wave's scan of the segment that
+// holds the target. (A scan of the whole row in symbol order, with the quotients formed again,
+// took 65 us of an 88 us launch.)
+constexpr int CODER_SEGS = 1024;  // at most this many segments
+
+template <bool STATS, bool PACKED, bool FIND, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_coder_compact(CompactCoderArgs a) {
+    constexpr int NW = NT / 64;
+    // LDS: the histogram from address 0 (a bin's byte address is 4 d), then the reduction slots and
+    // the segment sums of a Decode query
     extern __shared__ uint4 lds4[];
     uint32_t *hist = (uint32_t *)lds4;
     const int V = a.vocab, len = a.table_len, last = len - 1;
@@ -3491,7 +3546,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     constexpr bool packed = PACKED;
     const int n4 = ((packed ? zc + 64 : 2 * zc) + 3) >> 2;  // histogram words in uint4
     int64_t *s_i = (int64_t *)(lds4 + n4);
-    uint64_t *s_u = (uint64_t *)(lds4 + n4 + 2);
+    uint64_t *s_u = (uint64_t *)s_i + NW;
+    uint32_t *seg = (uint32_t *)(s_u + 2 * NW);
     const int row = blockIdx.x, tid = threadIdx.x;
     const uint16_t *d16 = a.d16 + (size_t)row * a.ld16;
     const int64_t *tm = a.tmax + (size_t)row * a.ntiles;
@@ -3514,12 +3570,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     // steps in turn, each step's loads issued one step ahead (the first before the row max). A
     // group past the row loads the row's last group instead (no branch around the loads, so a
     // step waits only for its own loads).
-    constexpr int STEP = 4 * 256 * 8;
+    constexpr int STEP = 4 * NT * 8;
     const int last_group = (V - 1) & ~7;
     auto fetch = [&](uint4 (&raw)[4], int64_t (&tmv)[4], int g0) {
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-            const int gq = g0 + u * 256 * 8;
+            const int gq = g0 + u * NT * 8;
             const int gc = gq < V ? gq : last_group;
             raw[u] = *(const uint4 *)(d16 + gc);
             tmv[u] = tm[gc >> 6];
@@ -3531,28 +3587,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     // no branch), so the max waits for them alone while the first step's groups arrive; the
     // histogram is cleared meanwhile (the barriers of the max order it before the symbol pass).
     int64_t mx = INT64_MIN;
-    for (int t = tid; t < a.ntiles; t += 1024) {
+    for (int t = tid; t < a.ntiles; t += 4 * NT) {
         int64_t v[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) v[u] = tm[min(t + 256 * u, a.ntiles - 1)];
+        for (int u = 0; u < 4; u++) v[u] = tm[min(t + NT * u, a.ntiles - 1)];
 #pragma unroll
         for (int u = 0; u < 4; u++) mx = v[u] > mx ? v[u] : mx;
     }
     fetch(ra, ta, tid * 8);
-    for (int k = tid; k < n4; k += 256) lds4[k] = make_uint4(0, 0, 0, 0);
-    const int64_t M = block_max64w(mx, s_i, tid);
+    for (int k = tid; k < n4; k += NT) lds4[k] = make_uint4(0, 0, 0, 0);
+    const int64_t M = block_max64w<NW>(mx, s_i, tid);
     uint64_t tok_w = 0;
     if (tok_lead) {
         const int64_t dt = M - tok_tm + tok_off;
         tok_w = a.table[dt < last ? dt : last];
     }
-    if (!STATS && a.weights) {  // the weights themselves (run_weights)
-        for (int j = tid; j < V; j += 256) {
-            const int64_t dd = M - tm[j >> 6] + d16[j];
-            a.weights[(size_t)row * V + j] = a.table[dd < last ? dd : last];
-        }
-    }
-
     int64_t first = INT64_MAX;  // the first symbol with weight table[0] (d <= d0)
     // A symbol's index is min(d, last) (logits.rs:62-72). tail0: the table ends in zeros, so
     // every d >= zcut weighs 0 (no count needed); else (zcut = len) every d >= last weighs
@@ -3565,7 +3614,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     auto process = [&](const uint4 (&cur)[4], const int64_t (&tmv)[4], int g0) {
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-            const int gq = g0 + u * 256 * 8;
+            const int gq = g0 + u * NT * 8;
             // with tail0, a group whose tile max is zcut or more below M has only weight-0
             // symbols; else its symbols' indexes start at min(M - tile max, last)
             if (gq >= V) continue;
@@ -3641,41 +3690,41 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     }
     __syncthreads();
 
-    // The weighted bins of this thread: d = tid + 256 k. The first KB (zcut up to 8,192) take
+    // The weighted bins of this thread: d = tid + NT k. The first KB (zcut up to 8,192) take
     // their table entries in one batch of loads (the table holds CODER_TABLE_READ entries; a bin
     // past zcut has count 0), kept in registers for the S pass; bins from 8,192 on go 8 at a
     // time, loaded in each pass.
     // c t = c t_lo + 2^32 c t_hi with t <= 2^40: the low parts accumulate in 64 bits (one
     // multiply-add each), the high parts (c t_hi <= V 2^8 summed over a thread's bins) in 32.
-    constexpr int KB = 32, BU = 8;
-    static_assert(256 * KB <= CODER_TABLE_READ, "the first bins' entries are read without bounds tests");
-    const int kept = zc < 256 * KB ? zc : 256 * KB;
+    constexpr int KB = 8192 / NT, BU = 8;
+    static_assert(NT * KB <= CODER_TABLE_READ, "the first bins' entries are read without bounds tests");
+    const int kept = zc < NT * KB ? zc : NT * KB;
     uint64_t tk[KB];
 #pragma unroll
     for (int k = 0; k < KB; k++) {
-        const int d = tid + 256 * k;
+        const int d = tid + NT * k;
         tk[k] = a.table[d];
     }
     uint64_t W = 0;
     uint32_t w_hi = 0;
 #pragma unroll
     for (int k = 0; k < KB; k++) {
-        const int d = tid + 256 * k;
+        const int d = tid + NT * k;
         const uint32_t h = d < kept ? hist[d] : 0;
         const uint32_t c = packed ? (h & 0xffffu) : h;
         W += (uint64_t)c * (uint32_t)tk[k];
         w_hi += c * (uint32_t)(tk[k] >> 32);
     }
-    for (int d0 = tid + 256 * KB; d0 < zc; d0 += 256 * BU) {
+    for (int d0 = tid + NT * KB; d0 < zc; d0 += NT * BU) {
         uint32_t c[BU];
         uint64_t t[BU];
 #pragma unroll
         for (int u = 0; u < BU; u++) {
-            const int d = d0 + 256 * u;
+            const int d = d0 + NT * u;
             c[u] = d < zc ? (packed ? (hist[d] & 0xffffu) : hist[d]) : 0;
         }
 #pragma unroll
-        for (int u = 0; u < BU; u++) t[u] = c[u] ? a.table[d0 + 256 * u] : 0;
+        for (int u = 0; u < BU; u++) t[u] = c[u] ? a.table[d0 + NT * u] : 0;
 #pragma unroll
         for (int u = 0; u < BU; u++) {
             W += (uint64_t)c[u] * (uint32_t)t[u];
@@ -3691,10 +3740,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         s_i[tid >> 6] = first;
     }
     __syncthreads();
-    W = s_u[0] + s_u[1] + s_u[2] + s_u[3];
+    W = s_u[0];
     int64_t largest = s_i[0];
 #pragma unroll
-    for (int w = 1; w < 4; w++) largest = s_i[w] < largest ? s_i[w] : largest;
+    for (int w = 1; w < NW; w++) {
+        W += s_u[w];
+        largest = s_i[w] < largest ? s_i[w] : largest;
+    }
     __syncthreads();
     if (STATS) {  // mixer.rs:278-288 (W >= table[0] >= 1, so top is the largest)
         if (tid == 0) {
@@ -3744,11 +3796,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         close = !(fabs(dl) >= 0x1p-18);
         return (uint32_t)bits - (dl < 0.0 ? 1u : 0u);
     };
+    const bool find = FIND && kind != 0;  // a Decode query: each counted bin keeps its q in the histogram's place
     uint64_t S = 0, Slo = 0;
-    uint32_t exact = 0;  // bit k: bin tid + 256 k needs the exact quotient
+    uint32_t exact = 0;  // bit k: bin tid + NT k needs the exact quotient
 #pragma unroll
     for (int k = 0; k < KB; k++) {
-        const int d = tid + 256 * k;
+        const int d = tid + NT * k;
         const uint32_t h = d < kept ? hist[d] : 0;
         const uint32_t c = packed ? (h & 0xffffu) : h;
         const uint32_t clo = packed ? (h >> 16) : (c ? hist[zc + d] : 0);
@@ -3759,6 +3812,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         } else {
             S += (uint64_t)c * q;
             Slo += (uint64_t)clo * q;
+            if (find && c) hist[d] = q;
         }
     }
     auto add_exact = [&](int d) {
@@ -3768,24 +3822,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         const uint64_t q = quotient(a.table[d], spare, W, W >= ((uint64_t)1 << 32) ? coder_frac(spare, W) : 0);
         S += (uint64_t)c * q;
         Slo += (uint64_t)clo * q;
+        if (find) hist[d] = (uint32_t)q;  // q < 2^32: the weight is at most W
     };
     while (exact) {
         const int k = __builtin_ctz(exact);
         exact &= exact - 1;
-        add_exact(tid + 256 * k);
+        add_exact(tid + NT * k);
     }
-    for (int d0 = tid + 256 * KB; d0 < zc; d0 += 256 * BU) {
+    for (int d0 = tid + NT * KB; d0 < zc; d0 += NT * BU) {
         uint32_t c[BU], clo[BU];
         uint64_t td[BU];
 #pragma unroll
         for (int u = 0; u < BU; u++) {
-            const int d = d0 + 256 * u;
+            const int d = d0 + NT * u;
             const uint32_t h = d < zc ? hist[d] : 0;
             c[u] = packed ? (h & 0xffffu) : h;
             clo[u] = packed ? (h >> 16) : (c[u] ? hist[zc + d] : 0);
         }
 #pragma unroll
-        for (int u = 0; u < BU; u++) td[u] = c[u] ? a.table[d0 + 256 * u] : 0;
+        for (int u = 0; u < BU; u++) td[u] = c[u] ? a.table[d0 + NT * u] : 0;
         uint32_t ex = 0;
 #pragma unroll
         for (int u = 0; u < BU; u++) {
@@ -3796,12 +3851,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
             } else {
                 S += (uint64_t)c[u] * q;
                 Slo += (uint64_t)clo[u] * q;
+                if (find && c[u]) hist[d0 + NT * u] = q;
             }
         }
         while (ex) {
             const int u = __builtin_ctz(ex);
             ex &= ex - 1;
-            add_exact(d0 + 256 * u);
+            add_exact(d0 + NT * u);
         }
     }
     // S and Slo in one round
@@ -3809,11 +3865,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     Slo = (uint64_t)wave_sum64((int64_t)Slo);
     if ((tid & 63) == 0) {
         s_u[tid >> 6] = S;
-        s_u[4 + (tid >> 6)] = Slo;
+        s_u[NW + (tid >> 6)] = Slo;
     }
     __syncthreads();
-    S = s_u[0] + s_u[1] + s_u[2] + s_u[3];
-    Slo = s_u[4] + s_u[5] + s_u[6] + s_u[7];
+    S = s_u[0];
+    Slo = s_u[NW];
+#pragma unroll
+    for (int w = 1; w < NW; w++) {
+        S += s_u[w];
+        Slo += s_u[NW + w];
+    }
     __syncthreads();
     const uint64_t rem = total - ((uint64_t)V + S);
     uint64_t *out = a.intervals ? a.intervals + 3 * (size_t)row : nullptr;
@@ -3827,53 +3888,101 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         }
         return;
     }
-    // Decode: the largest i with start_i <= target, in symbol order, 2048 symbols per step.
+    if constexpr (!FIND) return;
+    // Decode: the symbol whose interval [start, start + f) holds the target (every f is at least 1
+    // and their sum is the total, so there is one).
     const uint64_t target = value;
-    uint64_t run = 0;
-    int64_t cand = -1;
-    uint64_t cstart = 0, cfreq = 0;
-    for (int b = 0; b < V; b += 2048) {
-        uint64_t f[8];
-        uint64_t local = 0;
-        const int j0 = b + tid * 8;
-        if (j0 < V) {
-            const uint4 raw = *(const uint4 *)(d16 + j0);
-            const uint16_t *dv = (const uint16_t *)&raw;
-            const int64_t base = M - tm[j0 >> 6];
+    int shift = 6;  // a segment is 2^shift symbols
+    while (((V - 1) >> shift) >= CODER_SEGS) shift++;
+    const int nseg = ((V - 1) >> shift) + 1;
+    for (int k = tid; k < CODER_SEGS; k += NT) seg[k] = 0;
+    if (packed && tid < 64) hist[zc + tid] = 0;  // the spare bins: weight 0
+    __syncthreads();
+    auto q_at = [&](int64_t d) -> uint32_t {  // q of a symbol at distance d (d >= zc: weight 0)
+        const int dd = (int)(d < last ? d : last);
+        return dd < zc ? hist[dd] : 0;
+    };
+    // The sums of q over the 8 symbols of a thread's group, then over the eight threads of a tile of
+    // 64, in 32 bits: all the q of a row add up to at most spare < 2^32.
+    auto tiles = [&](const uint4 (&cur)[4], const int64_t (&tmv)[4], int g0) {
 #pragma unroll
-            for (int q = 0; q < 8; q++) {
-                const int j = j0 + q;
-                f[q] = 0;
-                if (j < V) {
-                    const int64_t dd = base + dv[q];
-                    const int d = (int)(dd < last ? dd : last);
-                    f[q] = 1 + q_of(a.table[d]) + (j == largest ? rem : 0);
-                    local += f[q];
+        for (int u = 0; u < 4; u++) {
+            const int gq = g0 + u * NT * 8;
+            uint32_t sum = 0;
+            const int64_t b64 = M - tmv[u];
+            if (gq < V && !(tail0 && b64 >= zc)) {
+                if (packed && addr16 && gq + 8 <= V) {  // bin addresses as in the symbol pass
+                    const unsigned short base = (unsigned short)(b64 < last ? b64 : last);
+                    const us2 bb = {base, base}, zz = {zl, zl};
+                    const uint32_t *wv = (const uint32_t *)&cur[u];
+                    const uint8_t *hb = (const uint8_t *)hist;
+#pragma unroll
+                    for (int p = 0; p < 4; p++) {
+                        us2 v;
+                        __builtin_memcpy(&v, &wv[p], 4);
+                        v = __builtin_elementwise_min(__builtin_elementwise_add_sat(v, bb), zz) << (unsigned short)2;
+                        sum += *(const uint32_t *)(hb + v.x) + *(const uint32_t *)(hb + v.y);
+                    }
+                } else {
+                    const uint16_t *dv = (const uint16_t *)&cur[u];
+#pragma unroll
+                    for (int q = 0; q < 8; q++)
+                        if (gq + q < V) sum += q_at(b64 + dv[q]);
                 }
             }
-        }
-        uint64_t step_total;
-        uint64_t start = run + block_scan64w(local, s_u, tid, step_total);
-        if (j0 < V) {
 #pragma unroll
-            for (int q = 0; q < 8; q++) {
-                const int j = j0 + q;
-                if (j >= V) break;
-                if (start <= target) {
-                    cand = j;
-                    cstart = start;
-                    cfreq = f[q];
-                }
-                start += f[q];
-            }
+            for (int o = 1; o < 8; o <<= 1) sum += __shfl_xor(sum, o, 64);
+            if ((tid & 7) == 0 && sum) atomicAdd(&seg[gq >> shift], sum);
         }
-        run += step_total;
+    };
+    for (int s0 = 0; s0 < V; s0 += STEP) {  // uniform trip count; groups past V add nothing
+        fetch(ra, ta, s0 + tid * 8);
+        tiles(ra, ta, s0 + tid * 8);
     }
-    const int64_t best = block_max64w(cand, s_i, tid);
-    if (cand >= 0 && cand == best) {
-        out[0] = (uint64_t)cand;
-        out[1] = cstart;
-        out[2] = cfreq;
+    __syncthreads();
+    // the segment that holds the target: each thread scans SP consecutive segments
+    constexpr int SP = CODER_SEGS / NT;
+    const int lseg = (int)(largest >> shift);
+    uint64_t mine[SP], local = 0, all;
+#pragma unroll
+    for (int u = 0; u < SP; u++) {
+        const int k = tid * SP + u;
+        const int count = min(V - (k << shift), 1 << shift);  // the segment's symbols (k < nseg)
+        mine[u] = k < nseg ? (uint64_t)seg[k] + (uint64_t)count + (k == lseg ? rem : 0) : 0;
+        local += mine[u];
+    }
+    uint64_t at = block_scan64w<NW>(local, s_u, tid, all);
+#pragma unroll
+    for (int u = 0; u < SP; u++) {
+        if (at <= target && target - at < mine[u]) {
+            s_u[0] = (uint64_t)(tid * SP + u);
+            s_u[1] = at;
+        }
+        at += mine[u];
+    }
+    __syncthreads();
+    if (tid >= 64) return;
+    const int j_end = min(V, (int)(s_u[0] + 1) << shift);
+    uint64_t start = s_u[1];
+    for (int j0 = (int)s_u[0] << shift; j0 < j_end; j0 += 64) {  // one tile at a time
+        const int j = j0 + tid;
+        uint64_t f = 0;
+        if (j < V) f = 1 + (uint64_t)q_at(M - tm[j >> 6] + d16[j]) + (j == largest ? rem : 0);
+        uint64_t end = f;  // inclusive scan
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint64_t v = __shfl_up(end, o, 64);
+            if (tid >= o) end += v;
+        }
+        const uint64_t mystart = start + end - f;
+        const bool here = mystart <= target && target - mystart < f;
+        if (here) {
+            out[0] = (uint64_t)j;
+            out[1] = mystart;
+            out[2] = f;
+        }
+        if (__any(here)) return;
+        start += __shfl(end, 63, 64);
     }
 }
 
@@ -4119,35 +4228,64 @@ __global__ __launch_bounds__(256) void k_coder_compact_mixed(CompactCoderArgs a)
 }
 
 template <typename K>
-static hipError_t launch_compact(K kernel, const CompactCoderArgs &a, int n_rows, hipStream_t stream) {
+static hipError_t launch_compact(K kernel, int threads, size_t extra, const CompactCoderArgs &a, int n_rows,
+                                 hipStream_t stream) {
     if (n_rows <= 0) return hipSuccess;
     // packed counts: zcut bins and 64 spare bins of the weight-0 symbols; else two arrays;
-    // rounded up to whole 16-byte words (the kernels clear them so)
-    // (k_coder_compact puts 128 bytes of reduction slots after them)
+    // rounded up to whole 16-byte words (the kernels clear them so), and `extra` bytes after them
     const size_t words = a.vocab < 65536 ? (size_t)a.zcut + 64 : 2 * (size_t)a.zcut;
-    const size_t lds = sizeof(uint32_t) * ((words + 3) & ~(size_t)3) + 128;
+    const size_t lds = sizeof(uint32_t) * ((words + 3) & ~(size_t)3) + extra;
     {
         const hipError_t e = allow_dynamic_lds((const void *)kernel, lds);
         if (e != hipSuccess) return e;
     }
-    launch_k(kernel, dim3(n_rows), dim3(256), lds, stream, a);
+    launch_k(kernel, dim3(n_rows), dim3(threads), lds, stream, a);
     return hipGetLastError();
 }
 
+// The reduction slots (three per wave) and the segment sums after the histogram.
+constexpr size_t coder_extra(int nt, bool find) { return (size_t)(3 * nt / 64) * 8 + (find ? CODER_SEGS * 4 : 0); }
+static_assert(2 * 4 * CODER_MAX_TABLE + coder_extra(1024, true) <= 160 * 1024, "LDS of one workgroup");
+
+template <bool STATS, bool FIND, int NT>
+static hipError_t launch_coder_compact_t(const CompactCoderArgs &a, int n_rows, hipStream_t stream) {
+    const size_t extra = coder_extra(NT, FIND);
+    return a.vocab < 65536 ? launch_compact(k_coder_compact<STATS, true, FIND, NT>, NT, extra, a, n_rows, stream)
+                           : launch_compact(k_coder_compact<STATS, false, FIND, NT>, NT, extra, a, n_rows, stream);
+}
+
 hipError_t launch_coder_compact(const CompactCoderArgs &a, int n_rows, hipStream_t stream) {
-    return a.vocab < 65536 ? launch_compact(k_coder_compact<false, true>, a, n_rows, stream)
-                           : launch_compact(k_coder_compact<false, false>, a, n_rows, stream);
+    if (a.weights && n_rows > 0) {
+        for (int r0 = 0; r0 < n_rows; r0 += 32768) {  // the grid's y dimension
+            CompactCoderArgs c = a;
+            c.d16 += (size_t)r0 * a.ld16;
+            c.tmax += (size_t)r0 * a.ntiles;
+            c.weights += (size_t)r0 * a.vocab;
+            launch_k(k_weights_compact, dim3((a.vocab + 2047) / 2048, std::min(n_rows - r0, 32768)), dim3(256), 0,
+                     stream, c);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+        }
+    }
+    if (!a.intervals) return hipSuccess;
+    // up to one row per CU: 1,024 threads a row (64 rows 18.0 -> 13.9 us, 42 -> 20 us with Decode
+    // queries); past that four rows of 256 threads share a CU (383 rows 20.5 us against 26.5)
+    if (n_rows <= 256) {
+        return a.decode ? launch_coder_compact_t<false, true, 1024>(a, n_rows, stream)
+                        : launch_coder_compact_t<false, false, 1024>(a, n_rows, stream);
+    }
+    return a.decode ? launch_coder_compact_t<false, true, 256>(a, n_rows, stream)
+                    : launch_coder_compact_t<false, false, 256>(a, n_rows, stream);
 }
 
 hipError_t launch_mix_stats_compact(const CompactCoderArgs &a, int n_rows, hipStream_t stream) {
     if (!a.mix || !a.stats) return hipErrorInvalidValue;
-    return a.vocab < 65536 ? launch_compact(k_coder_compact<true, true>, a, n_rows, stream)
-                           : launch_compact(k_coder_compact<true, false>, a, n_rows, stream);
+    return launch_coder_compact_t<true, false, 256>(a, n_rows, stream);
 }
 
 hipError_t launch_coder_compact_mixed(const CompactCoderArgs &a, int n_rows, hipStream_t stream) {
     if (!a.mix) return hipErrorInvalidValue;
-    return launch_compact(k_coder_compact_mixed, a, n_rows, stream);
+    return launch_compact(k_coder_compact_mixed, 256, 128, a, n_rows, stream);
 }
 
 // ---- kernel resources (CudaDevice::kernel_resources, crates/hardshell-cuda/src/device.rs:65-74) --
@@ -4193,7 +4331,9 @@ int kernel_resources(KernelResource *out, int cap) {
         {"k_attend_decode_wave<noclamp, 4>", (const void *)k_attend_decode_wave<true, 4>},
         {"k_split_dots<64>", (const void *)k_split_dots<64>},
         {"k_split_pv<noclamp>", (const void *)k_split_pv<true>},
-        {"k_coder_compact", (const void *)k_coder_compact<false, true>},
+        {"k_coder_compact", (const void *)k_coder_compact<false, true, false, 256>},
+        {"k_coder_compact, few rows with Decode", (const void *)k_coder_compact<false, true, true, 1024>},
+        {"k_weights_compact", (const void *)k_weights_compact},
         {"k_coder_compact_mixed", (const void *)k_coder_compact_mixed},
         {"k_read_bw", (const void *)k_read_bw},
     };
