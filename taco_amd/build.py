@@ -16,7 +16,7 @@ CXX = os.environ.get("CXX", "g++")
 HOST_SOURCES = {"common.cpp", "hsm.cpp", "taco/harness.cpp", "taco/tokenizer.cpp"}
 
 BACKEND_SOURCES = ["common.cpp", "hsm.cpp", "hs_api.cpp", "kernels.hip",
-                   "gemm_rows.hip"]
+                   "gemm_rows.hip", "layernorm.hip"]
 HARNESS_SOURCES = ["taco/harness.cpp", "taco/tokenizer.cpp"]  # hs::fail, sha256: the backend's (one error state)
 
 LIB_BACKEND = os.path.join(HERE, "libhardshell_hip.so")

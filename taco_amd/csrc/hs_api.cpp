@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <memory>
 #include <mutex>
@@ -19,6 +20,7 @@
 #include "common.h"
 #include "hardshell_hip.h"
 #include "hsm.h"
+#include "intmath.h"
 #include "kernels.h"
 
 #ifndef HS_SOURCE_SHA256
@@ -164,7 +166,10 @@ struct DevLn {
     int32_t *b = nullptr;
     int32_t m = 0;
     int s = 0;
-    bool beta_small = false;  // every |b[j]| <= 256
+    // the single-precision element rule (LnArgs::gf ..), where it holds for this LayerNorm
+    float *gf = nullptr, *bf = nullptr;
+    float margin = 0;
+    double mk = 0, inv_d = 0;
 };
 
 struct DevBlock {
@@ -220,7 +225,7 @@ hs_status upload_linear(DevMem &mem, const hs::HostLinear &l, DevLinear &o) {
     return st;
 }
 
-hs_status upload_ln(DevMem &mem, const hs::HostLayerNorm &l, DevLn &o) {
+hs_status upload_ln(DevMem &mem, const hs::HostLayerNorm &l, int beta_frac, DevLn &o) {
     std::vector<int64_t> gm(l.g.size());
     for (size_t j = 0; j < gm.size(); j++) gm[j] = (int64_t)l.g[j] * (int64_t)l.m;
     hs_status st = mem.upload(o.g, l.g.data(), l.g.size());
@@ -228,8 +233,19 @@ hs_status upload_ln(DevMem &mem, const hs::HostLayerNorm &l, DevLn &o) {
     if (st == HS_OK) st = mem.upload(o.b, l.b.data(), l.b.size());
     o.m = l.m;
     o.s = l.s;
-    o.beta_small = true;
-    for (int32_t v : l.b) o.beta_small = o.beta_small && v >= -256 && v <= 256;
+    // single precision needs |beta| <= 256 (beta is b 2^-beta_frac), a shift that rounds (s <= 126)
+    // and a fraction inside it; 128 + beta is then exact (at most 9 + beta_frac <= 24 bits)
+    double most = 0;
+    for (int32_t v : l.b) most = std::max(most, std::ldexp(std::fabs((double)v), -beta_frac));
+    if (st == HS_OK && most <= 256 && beta_frac >= 0 && beta_frac <= 15 && l.s <= 126 && l.s >= beta_frac) {
+        std::vector<float> gf(l.g.begin(), l.g.end()), bf(l.b.size());
+        for (size_t j = 0; j < bf.size(); j++) bf[j] = 128.0f + (float)std::ldexp((double)l.b[j], -beta_frac);
+        st = mem.upload(o.gf, gf.data(), gf.size());
+        if (st == HS_OK) st = mem.upload(o.bf, bf.data(), bf.size());
+        o.margin = hs::ln_margin((float)most);
+        o.mk = std::ldexp((double)l.m, -(int)l.s);
+        o.inv_d = 1.0 / (double)l.g.size();
+    }
     return st;
 }
 
@@ -393,8 +409,8 @@ hs_status upload_model(hs_device *dev, std::unique_ptr<hs_model> &m, hs_model **
     for (int l = 0; l < m->L; l++) {
         const hs::HostBlock &hb = h.blocks[l];
         DevBlock &b = m->blocks[l];
-        if ((st = upload_ln(mem, hb.ln1, b.ln1)) != HS_OK) return st;
-        if ((st = upload_ln(mem, hb.ln2, b.ln2)) != HS_OK) return st;
+        if ((st = upload_ln(mem, hb.ln1, (int)h.ln_beta_frac, b.ln1)) != HS_OK) return st;
+        if ((st = upload_ln(mem, hb.ln2, (int)h.ln_beta_frac, b.ln2)) != HS_OK) return st;
         if ((st = upload_linear(mem, hb.c_attn, b.c_attn)) != HS_OK) return st;
         if ((st = upload_linear(mem, hb.c_proj, b.c_proj)) != HS_OK) return st;
         if ((st = upload_linear(mem, hb.c_fc, b.c_fc)) != HS_OK) return st;
@@ -426,7 +442,7 @@ hs_status upload_model(hs_device *dev, std::unique_ptr<hs_model> &m, hs_model **
             b.gelu_copy = end16 - lo16;
         }
     }
-    if ((st = upload_ln(mem, h.ln_f, m->ln_f)) != HS_OK) return st;
+    if ((st = upload_ln(mem, h.ln_f, (int)h.ln_beta_frac, m->ln_f)) != HS_OK) return st;
     // padded to a multiple of 256 entries: the prefill attention loads it in 1 KiB chunks
     if ((st = mem.upload(m->attn_exp, h.attn_exp.data(), h.attn_exp.size(), (h.attn_exp.size() + 255) / 256 * 256)) != HS_OK) return st;
     {  // the zero tail of attn_exp: the short prefill kernel copies only the entries before it
@@ -1007,7 +1023,8 @@ hs_status run_pass(hs_batch &b, const std::vector<PassRow> &rows, Out out, const
         a.x = b.d_x; a.d = m.d; a.gamma = l.g; a.beta = l.b; a.m = l.m; a.s = l.s;
         a.beta_frac = m.host.ln_beta_frac; a.k = m.host.ln_k; a.j = m.host.ln_j; a.eps = m.host.ln_eps;
         a.out = dst; a.out_rows = (out_bits == 16 ? 2 : 1) * RP;
-        a.src = src_rows; a.gm = l.gm; a.beta_small = l.beta_small;
+        a.src = src_rows; a.gm = l.gm;
+        a.gf = l.gf; a.bf = l.bf; a.margin = l.margin; a.mk = l.mk; a.inv_d = l.inv_d;
         return b.launch("layer_norm", 0, [&] { return hs::launch_layernorm(a, rows_n, st); });
     };
     // The LM head: the rows of a chunk (at most a few MB of A) stay in every XCD's L2 while

@@ -172,23 +172,38 @@ HS_HD int64_t shift_round_hi(int64_t t, int64_t g, uint32_t s) {
     return (hi + ((int64_t)1 << (u - 1))) >> u;
 }
 
-// The LayerNorm element rule in single precision for 8-bit outputs with |beta| <= 256:
-// clamp(floor(X + 1/2) + beta, +-127) for X = c inv m gamma 2^-s, from y = c k + b with
-// k = float(inv m 2^-s) gamma (two roundings) and b = 1/2 + beta (exact), one fused
-// multiply-add. |y - (X + b)| <= 3.0001 2^-24 |X| + 2^-24 |y|. y is clamped to [-126.5, 127.5]:
-// inside, |X| < 458 and the error is below 1575 2^-24 < 2^-13, so floor(y) is exact when y lies
-// at least 2^-13 from an integer, and it lies in [-127, 127] (no output clamp); outside, y has
-// the sign and size of X + b (relative error below 2^-21), so floor(X + b) is at least 127 or at
-// most -127 and the output clamp gives the floor of the clamped y, whose fraction is 1/2.
-// |k| <= 2^110 keeps y finite or an infinity of the sign of c k (never NaN). Returns false
-// (declines) near an integer; *out is then unused.
+// The LayerNorm element rule in single precision for 8-bit outputs: clamp(floor(X + beta + 1/2), +-127)
+// for X = c inv m gamma 2^-s, from z = X + (beta + 128) by one fused multiply-add c k + b with
+// k = float(inv m 2^-s) gamma (two roundings) and b = 128 + beta (exact; beta may have a
+// fraction): |z - exact| <= 3.0001 2^-24 |X| + 2^-24 |z|. The output plus 128 is z rounded to the
+// nearest integer and clamped to [1, 255], exactly so when z lies further than the error from
+// a half: inside the clamp |X| <= 128 + |beta| and |z| <= 256, so `margin` =
+// 2^-24 (3.01 (128 + max |beta|) + 257) bounds it; outside, z has the sign and size of the exact
+// value and the clamp decides. |k| <= 2^110 keeps z finite or an infinity of the sign of c k.
+// Returns z clamped; the caller rounds it and takes another rule when ln_half_dist is below margin.
+HS_HD float ln_elem_z(int32_t c, float k, float b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_fmed3f(fmaf((float)c, k, b), 1.0f, 255.0f);
+#else
+    const float z = fmaf((float)c, k, b);
+    return z < 1.0f ? 1.0f : (z > 255.0f ? 255.0f : z);
+#endif
+}
+// The distance of z >= 0 from the nearest half (n + 1/2), as a signed difference.
+HS_HD float ln_half_dist(float z) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_fractf(z) - 0.5f;
+#else
+    return (z - floorf(z)) - 0.5f;
+#endif
+}
+HS_HD float ln_margin(float max_beta) { return (3.01f * (128.0f + max_beta) + 257.0f) * 0x1p-24f; }
+// One element as an integer, from b = 1/2 + beta with |beta| <= 256 (ln_margin(256) < 2^-13).
+// Returns false (declines) near a half; *out is then unused.
 HS_HD bool ln_elem_f32(int32_t c, float k, float b, int32_t *out) {
-    const float y = fmaf((float)c, k, b);
-    const float yc = fminf(fmaxf(y, -126.5f), 127.5f);
-    const float fl = floorf(yc);
-    const float f = yc - fl;
-    *out = (int32_t)fl;
-    return fabsf(f - 0.5f) <= 0.5f - 0x1p-13f;
+    const float z = ln_elem_z(c, k, b + 127.5f);
+    *out = (int32_t)rintf(z) - 128;
+    return fabsf(ln_half_dist(z)) >= 0x1p-13f;
 }
 
 // floor((c inv gamma m + 2^(s - 1)) / 2^s) (the LayerNorm element rule, layernorm.rs:66-108,
@@ -260,6 +275,75 @@ HS_HD uint64_t ln_inv_est(u128 sq, uint32_t n, uint32_t k, uint32_t j, uint64_t 
     const uint64_t var = div_u128_est(sq, n, inv_n);
     const uint64_t r = isqrt_est(((u128)var << (2 * j)) + (u128)eps);
     return pow2_div_est(k, r > 0 ? r : 1);
+}
+
+// The mean and scale of a LayerNorm row in 64-bit arithmetic, for rows with |x| <= 2^24 and
+// n <= 2,048 values: sum = sum x, Q = sum x^2 (below 2^59). With r = sum - n mean (0 <= r < n),
+// sum (x - mean)^2 = Q - mean (sum + r), below 2^59; var, t = var 2^(2j) + eps, the root of t and
+// 2^k / root each come from a double-precision estimate (inv_n = 1.0 / n, a reciprocal square
+// root, a reciprocal, refined once), are moved by at most one by the exact remainder, and the
+// remainder is then checked, so ok = true means the exact floors whatever the estimates were.
+// ok = false (a value outside 64 bits or an estimate further off): the caller takes ln_inv_est.
+struct LnTerms {
+    int32_t mean;
+    uint32_t inv;
+    bool ok;
+};
+HS_HD double rsq_approx(double x) {  // at least 20 bits
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_rsq(x);
+#else
+    return 1.0 / __builtin_sqrt(x);
+#endif
+}
+HS_HD double rcp_approx(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_rcp(x);
+#else
+    return 1.0 / x;
+#endif
+}
+HS_HD LnTerms ln_terms_small(int64_t sum, uint64_t Q, int32_t n, double inv_n, uint32_t k, uint32_t j,
+                             uint64_t eps) {
+    LnTerms o;
+    // |sum| <= 2^35: exact in double, the estimate within one of the quotient
+    int32_t mean = (int32_t)__builtin_floor((double)sum * inv_n);
+    int64_t r = sum - (int64_t)mean * n;
+    if (r < 0) mean--, r += n;
+    if (r >= n) mean++, r -= n;
+    bool ok = r >= 0 && r < n;
+    const uint64_t sq = Q - (uint64_t)((int64_t)mean * (sum + r));
+    // var < 2^48: the estimate within one
+    const double vd = __builtin_floor((double)sq * inv_n);
+    const uint32_t vh = (uint32_t)(vd * 0x1p-32);
+    uint64_t var = ((uint64_t)vh << 32) + (uint32_t)fma((double)vh, -0x1p32, vd);
+    int64_t rem = (int64_t)(sq - var * (uint32_t)n);
+    if (rem < 0) var--, rem += n;
+    if (rem >= n) var++, rem -= n;
+    ok = ok && rem >= 0 && rem < n && j <= 15 && (var >> (62 - 2 * j)) == 0 && eps >> 62 == 0;
+    const uint64_t t = (var << (2 * (j & 15))) + eps;  // below 2^63
+    const double td = (double)t, rs = rsq_approx(td);
+    double y = td * rs;
+    y = fma(fma(-y, y, td), 0.5 * rs, y);
+    uint32_t root = (uint32_t)y;
+    int64_t rt = (int64_t)(t - (uint64_t)root * root);
+    if (rt < 0) root--, rt += 2 * (int64_t)root + 1;
+    if (rt > 2 * (int64_t)root) rt -= 2 * (int64_t)root + 1, root++;
+    ok = ok && rt >= 0 && rt <= 2 * (int64_t)root && root > 0;
+    const uint64_t num = (uint64_t)1 << (k & 63);  // k <= 48
+    ok = ok && k <= 62 && (num >> 32) < root;      // the quotient is below 2^32
+    const double rd = (double)root;
+    double rc = rcp_approx(rd);
+    rc = fma(fma(-rd, rc, 1.0), rc, rc);
+    uint32_t inv = (uint32_t)((double)num * rc);
+    int64_t ri = (int64_t)(num - (uint64_t)inv * root);
+    if (ri < 0) inv--, ri += root;
+    if (ri >= (int64_t)root) inv++, ri -= root;
+    ok = ok && ri >= 0 && ri < (int64_t)root;
+    o.mean = mean;
+    o.inv = inv;
+    o.ok = ok;
+    return o;
 }
 
 // The softmax weight p = floor(e 2^P / S) (softmax.rs:78-104) of a table entry e <= S, e < 2^31,

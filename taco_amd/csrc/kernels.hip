@@ -1533,18 +1533,14 @@ __global__ __launch_bounds__(256) void k_layernorm_rows(LnArgs a, int n_rows) {
 // column past d the last group; neither value is used): no branch around the loads.
 // The input is the residual stream (|x| <= RES = 2^30 - 1): every square is below 2^60, so the
 // four of a group sum in i64 without a carry.
-// F32 (8-bit outputs, beta_frac 0, |beta| <= 256): each element takes the single-precision rule
-// (ln_elem_f32, with beta folded into the addend); declined groups take the integer rule, as in
-// the double-precision form.
+// (8-bit outputs with |beta| <= 256 take k_layernorm_f32 instead: layernorm.hip.)
 constexpr int LN_WAVES = 16;
 
-template <int NG, bool F32>
+template <int NG>
 __global__ __launch_bounds__(64 * LN_WAVES) void k_layernorm_rows4(LnArgs a, int n_rows) {
     constexpr int NT = 64 * LN_WAVES, CI = (64 * NG + NT - 1) / NT, RW = 4 * LN_WAVES;
     __shared__ __attribute__((aligned(16))) int32_t s_beta[64 * NG];
-    __shared__ __attribute__((aligned(16))) double s_gamma[F32 ? 1 : 64 * NG];
-    __shared__ __attribute__((aligned(16))) float s_gammaf[F32 ? 64 * NG : 1];
-    __shared__ __attribute__((aligned(16))) float s_betaf[F32 ? 64 * NG : 1];  // 1/2 + beta
+    __shared__ __attribute__((aligned(16))) double s_gamma[64 * NG];
     // per row of the workgroup: the sums, then the rule's terms
     __shared__ int64_t s_sum[RW];
     __shared__ uint64_t s_lo[RW], s_hi[RW];
@@ -1567,16 +1563,11 @@ __global__ __launch_bounds__(64 * LN_WAVES) void k_layernorm_rows4(LnArgs a, int
         xv[t] = *(const v4i *)(x + (j < d ? j : d - 4));
     }
 #pragma unroll
-    for (int i = 0; i < CI; i++) {  // gamma as doubles or floats (exact)
+    for (int i = 0; i < CI; i++) {  // gamma as doubles (exact)
         const int c = threadIdx.x + NT * i;
         if (c >= d) continue;
         s_beta[c] = a.beta[c];
-        if (F32) {
-            s_gammaf[c] = (float)a.gamma[c];
-            s_betaf[c] = 0.5f + (float)a.beta[c];  // exact: |beta| <= 256
-        } else {
-            s_gamma[c] = (double)a.gamma[c];
-        }
+        s_gamma[c] = (double)a.gamma[c];
     }
     // squares: the four of a group to an i64 partial (each < 2^60), the partials into a 128-bit
     // lo/hi with carries
@@ -1670,22 +1661,7 @@ __global__ __launch_bounds__(64 * LN_WAVES) void k_layernorm_rows4(LnArgs a, int
         if (wide) *at(1, j) = packed_lo;
     };
     uint32_t redo = fpath ? 0u : ~0u;  // bit t: group t takes the integer rule
-    if (F32) {
-        const float krf = (float)kr;
-#pragma unroll
-        for (int t = 0; t < NG; t++) {
-            const int j = 4 * (q + 16 * t);
-            if (j >= d) continue;
-            int32_t y[4];
-            bool all = true;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                all &= ln_elem_f32(xv[t][e] - mean32, krf * s_gammaf[j + e], s_betaf[j + e], &y[e]);
-            }
-            put(j, y);
-            redo |= all ? 0u : 1u << t;
-        }
-    } else if (fpath) {
+    if (fpath) {
 #pragma unroll
         for (int t = 0; t < NG; t++) {
             const int j = 4 * (q + 16 * t);
@@ -1738,23 +1714,17 @@ __global__ __launch_bounds__(64 * LN_WAVES) void k_layernorm_rows4(LnArgs a, int
 hipError_t launch_layernorm(const LnArgs &a, int n_rows, hipStream_t stream) {
     if (n_rows <= 0) return hipSuccess;
     const dim3 grid((n_rows + 3) / 4);
+    if (layernorm_f32_fits(a)) return launch_layernorm_f32(a, n_rows, stream);
     // the vector forms need d a multiple of 4 (4-byte groups of a row lie in one panel)
-    // the single-precision element rule: 8-bit outputs, integer beta with |beta| <= 256
-    const bool f32 = a.bits == 8 && a.beta_frac == 0 && a.beta_small && a.s <= 126;
-    // Fewer than 4,096 rows (decode passes): a one-wave workgroup per row, spread over the CUs;
-    // the 16-lane form would leave most of them idle (256 rows: 16 workgroups)
+    // Fewer than 4,096 rows: a one-wave workgroup per row, spread over the CUs; the 16-lane form
+    // would leave most of them idle (256 rows: 16 workgroups)
     if (n_rows < 4096 && a.d % 4 == 0 && a.d <= 2048) {
         if (a.d <= 1024) launch_k(k_layernorm_rows<4>, dim3(n_rows), dim3(64), 0, stream, a, n_rows);
         else launch_k(k_layernorm_rows<8>, dim3(n_rows), dim3(64), 0, stream, a, n_rows);
     } else if (a.d % 4 == 0 && a.d <= 1024) {
         const dim3 g4((n_rows + 4 * LN_WAVES - 1) / (4 * LN_WAVES)), b4(64 * LN_WAVES);
-        if (a.d <= 768) {
-            if (f32) launch_k((k_layernorm_rows4<12, true>), g4, b4, 0, stream, a, n_rows);
-            else launch_k((k_layernorm_rows4<12, false>), g4, b4, 0, stream, a, n_rows);
-        } else {
-            if (f32) launch_k((k_layernorm_rows4<16, true>), g4, b4, 0, stream, a, n_rows);
-            else launch_k((k_layernorm_rows4<16, false>), g4, b4, 0, stream, a, n_rows);
-        }
+        if (a.d <= 768) launch_k(k_layernorm_rows4<12>, g4, b4, 0, stream, a, n_rows);
+        else launch_k(k_layernorm_rows4<16>, g4, b4, 0, stream, a, n_rows);
     } else if (a.d % 4 == 0 && a.d <= 2048) {
         launch_k(k_layernorm_rows<8>, grid, dim3(256), 0, stream, a, n_rows);
     } else {
@@ -4320,8 +4290,8 @@ int kernel_resources(KernelResource *out, int cap) {
         {"k_layernorm", (const void *)k_layernorm},
         {"k_layernorm_rows<4>", (const void *)k_layernorm_rows<4>},
         {"k_layernorm_rows<8>", (const void *)k_layernorm_rows<8>},
-        {"k_layernorm_rows4<12, f32>", (const void *)k_layernorm_rows4<12, true>},
-        {"k_layernorm_rows4<16, f32>", (const void *)k_layernorm_rows4<16, true>},
+        {"k_layernorm_rows4<12>", (const void *)k_layernorm_rows4<12>},
+        {"k_layernorm_rows4<16>", (const void *)k_layernorm_rows4<16>},
         {"k_kv_store", (const void *)k_kv_store},
         {"k_attend", (const void *)k_attend},
         {"k_attend_short<4>", (const void *)k_attend_short<4>},
