@@ -113,28 +113,6 @@ __device__ __forceinline__ int64_t wave_sum64(int64_t v) {
 constexpr int GEMM_STAGES = 3;
 static_assert(GEMM_BM == 256 && GEMM_BK == 64 && GEMM_NPAD % 256 == 0, "tile shape of k_gemm");
 
-typedef __attribute__((address_space(3))) void lds_void;
-typedef int v2i __attribute__((ext_vector_type(2)));
-typedef unsigned short us2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) v2i lds_v2i;
-
-// s_waitcnt vmcnt(N) with the other counters left at their maximum (gfx9 encoding).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-
-// A workgroup barrier for LDS data only: this wave's LDS operations complete (lgkmcnt 0), then
-// s_barrier, without the wait for every outstanding global load that the release fence of
-// __syncthreads brings. Global data read after it must not depend on other waves' stores.
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0); vmcnt 63 and expcnt 7 leave those alone
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
 // A compile-time flag for the steps of an unrolled loop (the first k-step differs).
 template <bool B>
 struct Flag {
@@ -1773,10 +1751,6 @@ __device__ __forceinline__ int32_t dot_key(const int *q4, const int8_t *k, int h
 // The output of row r at column col: row-major (ldo) for the op entries, or the operand panels
 // of the next product (out_rows > 0). Groups of up to 16 columns from a multiple of 16 (of 4
 // for 4-byte groups) lie in one panel.
-__device__ __forceinline__ int8_t *attn_out(const AttnArgs &a, int r, int col) {
-    return a.out + (a.out_rows ? panel_off(r, col, a.out_rows) : (size_t)r * a.ldo + col);
-}
-
 __global__ __launch_bounds__(256) void k_attend(AttnArgs a, int n_tasks) {
     __shared__ __attribute__((aligned(16))) int s_q[4][64];  // hd <= 256 bytes per wave
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -2481,18 +2455,6 @@ constexpr int AT_ST = 80;               // LDS row stride in bytes (64 + 16)
 constexpr int AT_SB = 4;                // key blocks of 64 held in registers
 constexpr int ATTN_LDS_TABLE = 16384;   // attn_exp entries kept in LDS (64 KiB)
 
-// 4 x 4 byte transpose: out[k] holds byte k of w0, w1, w2, w3 (in that order).
-__device__ __forceinline__ void byte_transpose(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3,
-                                               uint32_t out[4]) {
-    const uint32_t t0 = __builtin_amdgcn_perm(w1, w0, 0x05010400u);
-    const uint32_t t1 = __builtin_amdgcn_perm(w1, w0, 0x07030602u);
-    const uint32_t t2 = __builtin_amdgcn_perm(w3, w2, 0x05010400u);
-    const uint32_t t3 = __builtin_amdgcn_perm(w3, w2, 0x07030602u);
-    out[0] = __builtin_amdgcn_perm(t2, t0, 0x05040100u);
-    out[1] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);
-    out[2] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
-    out[3] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
-}
 
 // NOCLAMP: score_s >= 13, so |dot m| < 2^53 keeps every score within +-2^40 (the clamp is a no-op).
 // LDS_TABLE: attn_exp (<= ATTN_LDS_TABLE entries) is read from a copy in LDS.
@@ -2774,7 +2736,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 }
 
 // =============================================================================================
-// Prefill attention, the common case: head_dim 64, at most 8 key blocks of 64 per group, attn_exp
+// Prefill attention of short windows: head_dim 64, at most 8 key blocks of 64 per group, attn_exp
 // in LDS, score shift 22 .. 63 and P <= 30. The algorithm and the layouts are k_attend_mfma's;
 // the per-score work is smaller:
 //  - |dot| <= 64 2^14 and |m| <= 2^31, so |score| <= 2^29 + 1 for s >= 22: the distance M - s is
@@ -2791,19 +2753,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 //    from an integer floor(y) is exact, else the element takes the i128 rule.
 //  - the Q fragment is read straight from global memory (each lane's 16 bytes of its row).
 // =============================================================================================
-// x, hidden from the optimizer (a value it cannot prove invariant in a loop)
-__device__ __forceinline__ int opaque_vgpr(int x) {
-    asm volatile("" : "+v"(x));
-    return x;
-}
-
-// v_med3_i32(x, 0, hi) for a wave-uniform hi (the compiler forms med3 only for constant bounds)
-__device__ __forceinline__ int32_t clamp0_uniform(int32_t x, int32_t hi) {
-    int32_t r;
-    asm("v_med3_i32 %0, %1, 0, %2" : "=v"(r) : "v"(x), "s"(hi));
-    return r;
-}
-
 // NB: key blocks of 64 (4: three workgroups per CU with a 32 KiB table; 8: two).
 // Persistent: the grid holds the resident workgroups (at most n_tasks), and workgroup i takes
 // the tasks (group, head), task = group n_head + head, of rounds r = 0, 1, .. in snake order:
@@ -3090,6 +3039,276 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB <= 4 ? 3
     }
 }
 
+// =============================================================================================
+// Prefill attention over any number of keys (head_dim 64, attn_exp in LDS, score shift 22 .. 63,
+// P <= 30, at most 2^15 keys): windows of a whole context. The exact integer softmax needs the row
+// max before the table entries and their sum before p, so the keys are walked three times, 128
+// at a time: the extreme dots; the sum of the entries; p, its digits and the PV products. Each
+// walk forms Q K^T again (4 MFMAs per 64 keys, less than keeping 1,024 scores a row would cost in
+// registers: a wave stays within 168, three workgroups per CU). What bounds it is the VALU work
+// of the scores, as in k_attend_short (per score: 2 instructions, then about 6 and a lookup,
+// then about 13 and a lookup), so the loads must not add waits: the K and V rows of 128 keys are
+// 8 KiB stages of one stream over a ring of three, two stages ahead of their use and across the
+// end of a task into the next one's.
+// Persistent, tasks in snake order, as k_attend_short.
+// =============================================================================================
+constexpr int AL_SB = 2;                  // key blocks of 64 per stage
+constexpr int AL_STAGE = AL_SB * 64 * 64;  // bytes
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_attend_long(AttnArgs a, const AttnGroup *groups, int n_tasks) {
+    __shared__ __attribute__((aligned(1024))) int8_t ring[3 * AL_STAGE];
+    extern __shared__ __attribute__((aligned(1024))) int32_t s_exp[];  // attn_exp
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int last = a.exp_last > 0 ? a.exp_last : a.exp_len - 1;
+    const int P = gridDim.x, wg = blockIdx.x;
+    auto task_at = [&](int r) { return r * P + ((r & 1) ? P - 1 - wg : wg); };
+    auto sw = [](int r) { return ((r >> 1) ^ (r >> 3)) & 3; };
+    auto keys_of = [&](const AttnGroup &g) { return g.pos0 + g.count < a.ctx_cap ? g.pos0 + g.count : a.ctx_cap; };
+    auto stages_of = [&](const AttnGroup &g) { return (keys_of(g) + 64 * AL_SB - 1) / (64 * AL_SB); };
+    // Stage sb of K or V of a (group, head) into ring slot `slot`: dense rows, 16-byte chunk c of row r at
+    // slot 4 r + (c ^ sw(r % 16)); rows past the cache read its last row (their keys are masked).
+    // Each wave issues AL_SB loads of 1 KiB.
+    auto stage = [&](const int8_t *cache, const AttnGroup &g, int hh, int sb, int slot) {
+        const int r = 16 * w + (lane >> 2), c = (lane & 3) ^ sw(r & 15);
+        const size_t base = ((size_t)g.slot * a.n_head + hh) * a.ctx_cap * 64;
+#pragma unroll
+        for (int b = 0; b < AL_SB; b++) {
+            int key = (sb * AL_SB + b) * 64 + r;
+            key = key < a.ctx_cap ? key : a.ctx_cap - 1;
+            __builtin_amdgcn_global_load_lds((const void *)(cache + base + (size_t)key * 64 + 16 * c),
+                                             (lds_void *)(ring + slot * AL_STAGE + (b * 64 + 16 * w) * 64), 16, 0, 0);
+        }
+    };
+    // Load j of a task of n stages: K 0 .. n - 1 (walk 1), K n - 2 .. 0 (walk 2 starts on the stage that
+    // walk 1 ends on), then V 0, K 1, V 1, K 2, .. V n - 1 (walk 3 starts on K 0): 4 n - 2 loads.
+    auto issue_load = [&](const AttnGroup &g, int hh, int n, int j, int slot) {
+        const int t = j - (2 * n - 1);
+        if (t < 0) stage(a.kc, g, hh, j < n ? j : 2 * n - 2 - j, slot);
+        else if (t & 1) stage(a.kc, g, hh, (t + 1) >> 1, slot);
+        else stage(a.vc, g, hh, t >> 1, slot);
+    };
+    auto q_frag = [&](const AttnGroup &g, int hh) -> v4i {  // this lane's row is 16 w + lane % 16
+        const int row = 16 * w + (lane & 15);
+        if (row < g.count) return *(const v4i *)(a.q + (size_t)(g.first + row) * a.ldq + hh * 64 + 16 * (lane >> 4));
+        return v4i{0, 0, 0, 0};
+    };
+    // score = (dot m + 2^(s-1)) >> s (exact in i64: |dot m| <= 2^51), an i32 for s >= 22
+    const int s_eff = a.score_s < 63 ? a.score_s : 63;
+    const int64_t s_half = (int64_t)1 << (s_eff - 1);
+    auto score = [&](int32_t dot) -> int32_t { return (int32_t)(((int64_t)dot * a.score_m + s_half) >> s_eff); };
+
+    int t = task_at(0);  // below n_tasks: the launcher takes P <= n_tasks
+    AttnGroup G = groups[t / a.n_head], Gn = G;
+    int h = t % a.n_head, hn = h, n = stages_of(G);
+    bool more = false;
+    int issued = 0, used = 0;  // loads of this task (issued: and of the next) issued and waited for
+    int slot_in = 0, slot = 0;
+    auto issue_next = [&]() {
+        const int T = 4 * n - 2;
+        if (issued < T) issue_load(G, h, n, issued, slot_in);
+        else if (more) issue_load(Gn, hn, stages_of(Gn), issued - T, slot_in);
+        else return;
+        issued++;
+        slot_in = slot_in == 2 ? 0 : slot_in + 1;
+    };
+    // The next load's stage: its loads landed (this wave's by the count, the others' by the barrier), and
+    // every wave is done with the stage before it, whose slot takes the load after next.
+    auto next_stage = [&]() -> const int8_t * {
+        if (issued > used + 1) wait_vmcnt<AL_SB>();
+        else wait_vmcnt<0>();
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        const int8_t *p = ring + slot * AL_STAGE;
+        slot = slot == 2 ? 0 : slot + 1;
+        used++;
+        issue_next();
+        return p;
+    };
+    for (int ch = w; ch < (last + 256) / 256; ch += 4)  // whole 1 KiB chunks of entries 0 .. last
+        __builtin_amdgcn_global_load_lds((const void *)(a.exp_table + ch * 256 + 4 * lane),
+                                         (lds_void *)(s_exp + ch * 256), 16, 0, 0);
+    issue_next();
+    issue_next();
+    for (int round = 0;; round++) {
+        const int ql = lane & 15, qg = lane >> 4;
+        const int tn = task_at(round + 1);
+        more = tn < n_tasks;  // uniform
+        if (more) {
+            Gn = groups[tn / a.n_head];
+            hn = tn % a.n_head;
+        }
+        const v4i qf = q_frag(G, h);
+        wait_vmcnt<0>();  // (stores of the task before may leave the count out of order: start from zero)
+        const int nk = keys_of(G), nkb = (nk + 63) / 64;
+        const int myrow = 16 * w + ql, mypos = G.pos0 + myrow;
+        // key 64 b + 16 t + 4 qg + e is visible to this lane's row iff 16 t + e <= lim - 64 b - 4 qg;
+        // block b is visible to every row of the wave iff 64 b + 63 <= wlim (uniform), and to none
+        // iff 64 b > wmax
+        const int lim = mypos < nk - 1 ? mypos : nk - 1;
+        const int wlim = G.pos0 + 16 * w < nk - 1 ? G.pos0 + 16 * w : nk - 1;
+        const int wmax = G.pos0 + 16 * w + 15 < nk - 1 ? G.pos0 + 16 * w + 15 : nk - 1;
+        // D[t][e]: the dot of this lane's row with key 64 kb + 16 t + 4 qg + e (block b of the stage at st)
+        auto dots = [&](const int8_t *st, int b, v4i (&D)[4]) {
+#pragma unroll
+            for (int tt = 0; tt < 4; tt++) {
+                const int r = tt * 16 + ql;
+                const v4i kf = *(const v4i *)&st[(4 * (b * 64 + r) + (qg ^ sw(r & 15))) * 16];
+                D[tt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf, qf, v4i{0, 0, 0, 0}, 0, 0, 0);
+            }
+        };
+        // walk 1: the extreme visible dots
+        int32_t dmax = INT32_MIN, dmin = INT32_MAX;
+        const int8_t *st = nullptr;
+        for (int sb = 0; sb < n; sb++) {
+            st = next_stage();
+#pragma unroll
+            for (int b = 0; b < AL_SB; b++) {
+                const int kb = sb * AL_SB + b;
+                if (kb >= nkb || 64 * kb > wmax) continue;
+                v4i D[4];
+                dots(st, b, D);
+                if (64 * kb + 63 <= wlim) {
+#pragma unroll
+                    for (int tt = 0; tt < 4; tt++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            dmax = D[tt][e] > dmax ? D[tt][e] : dmax;
+                            dmin = D[tt][e] < dmin ? D[tt][e] : dmin;
+                        }
+                } else {
+                    const int L = lim - 64 * kb - 4 * qg;
+#pragma unroll
+                    for (int tt = 0; tt < 4; tt++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            const bool ok = 16 * tt + e <= L;
+                            const int32_t hiv = ok ? D[tt][e] : INT32_MIN, lov = ok ? D[tt][e] : INT32_MAX;
+                            dmax = hiv > dmax ? hiv : dmax;
+                            dmin = lov < dmin ? lov : dmin;
+                        }
+                }
+            }
+        }
+#pragma unroll
+        for (int o = 16; o < 64; o <<= 1) {  // the 4 lanes of this row
+            const int32_t u = __shfl_xor(dmax, o, 64), v = __shfl_xor(dmin, o, 64);
+            dmax = u > dmax ? u : dmax;
+            dmin = v < dmin ? v : dmin;
+        }
+        const int32_t mx = score(dmax) > score(dmin) ? score(dmax) : score(dmin);
+        // the table entries attn_exp[min(M - s, last)] of a block's keys, 0 for a masked key
+        auto entries = [&](const int8_t *stg, int b, int kb, v4i (&E)[4]) {
+            dots(stg, b, E);
+#pragma unroll
+            for (int tt = 0; tt < 4; tt++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) E[tt][e] = clamp0_uniform(mx - score(E[tt][e]), last);
+#pragma unroll
+            for (int tt = 0; tt < 4; tt++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) E[tt][e] = s_exp[E[tt][e]];
+            if (64 * kb + 63 > wlim) {
+                const int L = lim - 64 * kb - 4 * qg;
+#pragma unroll
+                for (int tt = 0; tt < 4; tt++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) E[tt][e] = 16 * tt + e <= L ? E[tt][e] : 0;
+            }
+        };
+        // walk 2: their sum (entries are < 2^31: a pair sums in u32)
+        uint64_t sum = 0;
+        for (int sb = n - 1; sb >= 0; sb--) {
+            if (sb < n - 1) st = next_stage();
+#pragma unroll
+            for (int b = 0; b < AL_SB; b++) {
+                const int kb = sb * AL_SB + b;
+                if (kb >= nkb || 64 * kb > wmax) continue;
+                v4i E[4];
+                entries(st, b, kb, E);
+#pragma unroll
+                for (int tt = 0; tt < 4; tt++)
+#pragma unroll
+                    for (int e = 0; e < 4; e += 2) sum += (uint32_t)E[tt][e] + (uint32_t)E[tt][e + 1];
+            }
+        }
+#pragma unroll
+        for (int o = 16; o < 64; o <<= 1) sum += __shfl_xor(sum, o, 64);
+        const double R = ldexp(1.0 / (double)sum, a.softmax_p);
+        const double sp = softmax_sp(sum, a.softmax_p);
+        // walk 3: p + 0x80808080 (the packed digits), and the digit-plane PV products, the V^T operand
+        // by transposing LDS reads (the layouts of k_attend_short)
+        const int tr_k = ql >> 1, tr_h = ql & 1;
+        const int tr_key0 = 16 * (tr_k >> 2) + 4 * qg + (tr_k & 3);
+        v4i acc[4][4];  // [digit plane][channel tile]: channel 16 c + 4 (l / 16) + e of row l % 16
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) acc[k][c] = v4i{0, 0, 0, 0};
+        for (int sb = 0; sb < n; sb++) {
+            if (sb > 0) st = next_stage();
+            v4i pf[AL_SB][4];  // [block][digit plane]: word t holds the digits of keys 16 t + 4 (l / 16) + e
+#pragma unroll
+            for (int b = 0; b < AL_SB; b++) {
+                const int kb = sb * AL_SB + b;
+                if (kb >= nkb || 64 * kb > wmax) continue;
+                v4i E[4];
+                entries(st, b, kb, E);
+#pragma unroll
+                for (int tt = 0; tt < 4; tt++) {
+                    uint32_t dg[4], o[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) dg[e] = softmax_p_of((uint32_t)E[tt][e], R, sp) + 0x80808080u;
+                    byte_transpose(dg[0], dg[1], dg[2], dg[3], o);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) pf[b][k][tt] = (int32_t)(o[k] ^ 0x80808080u);
+                }
+            }
+            const int8_t *sv = next_stage();
+#pragma unroll
+            for (int b = 0; b < AL_SB; b++) {
+                const int kb = sb * AL_SB + b;
+                if (kb >= nkb || 64 * kb > wmax) continue;
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    const int8_t *p0 = sv + (4 * (b * 64 + tr_key0) + (c ^ sw(tr_key0 & 15))) * 16 + 8 * tr_h;
+                    const v2i r0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)p0);
+                    const v2i r1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(p0 + 32 * 64));
+                    const v4i vf = v4i{r0[0], r0[1], r1[0], r1[1]};
+#pragma unroll
+                    for (int k = 0; k < 4; k++)
+                        acc[k][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(vf, pf[b][k], acc[k][c], 0, 0, 0);
+                }
+            }
+        }
+        // The sum of the planes is |v| <= 2^P 128 <= 2^37 and each plane an i32 (|acc| <= keys 2^14): for
+        // shifts 48 .. 63 attn_out_planes on v = hi 2^16 + lo, 0 <= lo < 2^16, else the i128 rule.
+        if (myrow < G.count) {
+            int8_t *o = attn_out(a, G.first + myrow, h * 64);
+            const bool planes = a.out_s >= 48 && a.out_s <= 63;
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                uint32_t packed = 0;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int64_t v = (int64_t)acc[0][c][e] + (int64_t)acc[1][c][e] * 256 +
+                                      (int64_t)acc[2][c][e] * 65536 + (int64_t)acc[3][c][e] * 16777216;
+                    const int32_t r = planes ? attn_out_planes((int32_t)(v >> 16), (int32_t)(v & 0xffff), a.out_m,
+                                                               (uint32_t)a.out_s)
+                                             : (int32_t)clamp128(rescale_full(v, a.out_m, a.out_s), -127, 127);
+                    packed |= (uint32_t)(uint8_t)(int8_t)r << (8 * e);
+                }
+                *(uint32_t *)(o + 16 * c + 4 * qg) = packed;
+            }
+        }
+        if (!more) break;
+        issued -= 4 * n - 2;
+        used = 0;
+        G = Gn;
+        h = hn;
+        n = stages_of(G);
+    }
+}
+
 template <bool NOCLAMP, bool LDS_TABLE, bool MULTI>
 static hipError_t launch_attend_groups_t(const AttnArgs &a, const AttnGroup *groups, int n_groups,
                                          hipStream_t stream) {
@@ -3117,23 +3336,30 @@ hipError_t launch_attend_groups(const AttnArgs &a, const AttnGroup *groups, int 
     if (a.hd != 64 || (a.out_rows == 0 && a.ldo % 4 != 0) || ((uintptr_t)a.out & 3) != 0 || max_keys < 1)
         return hipErrorInvalidValue;
     const bool noclamp = a.score_s >= 13, lds_table = a.exp_len <= ATTN_LDS_TABLE;
-    if (lds_table && max_keys <= 8 * 64 && a.score_s >= 22 && a.softmax_p <= 30 && a.out_s >= 0) {
+    if (lds_table && max_keys <= 1 << 15 && a.score_s >= 22 && a.softmax_p <= 30 && a.out_s >= 0) {
         // whole 1 KiB chunks of the entries up to the zero tail (or the whole table)
         const int last = a.exp_last > 0 && a.exp_last < a.exp_len ? a.exp_last : a.exp_len - 1;
         const size_t lds = ((size_t)last + 256) / 256 * 1024;
-        const bool four = max_keys <= 4 * 64;
-        const void *fn = four ? (const void *)k_attend_short<4> : (const void *)k_attend_short<8>;
-        hipError_t e = allow_dynamic_lds(fn, lds);
-        if (e != hipSuccess) return e;
-        // the resident workgroups (CUs x workgroups per CU at this LDS size), at most one per task
-        int resident = 0;
-        e = resident_workgroups(fn, 256, lds, &resident);
-        if (e != hipSuccess) return e;
-        const int n_tasks = n_groups * a.n_head;
-        const int P = resident < n_tasks ? resident : n_tasks;
-        if (four) launch_k(k_attend_short<4>, dim3(P), dim3(256), lds, stream, a, groups, n_tasks);
-        else launch_k(k_attend_short<8>, dim3(P), dim3(256), lds, stream, a, groups, n_tasks);
-        return hipGetLastError();
+        // the scores of up to 256 or 512 keys stay in registers (48 windows of 512, 16 heads: 141 us
+        // against 172 walked); more keys are walked again (13 windows of 1,024, 12 heads: 235 ->
+        // 120 us against k_attend_mfma, which held four blocks' scores in i64 forms and loaded K
+        // and V between barriers)
+        auto run = [&](auto kernel) -> hipError_t {
+            const void *fn = (const void *)kernel;
+            hipError_t e = allow_dynamic_lds(fn, lds);
+            if (e != hipSuccess) return e;
+            // the resident workgroups (CUs x workgroups per CU at this LDS size), at most one per task
+            int resident = 0;
+            e = resident_workgroups(fn, 256, lds, &resident);
+            if (e != hipSuccess) return e;
+            const int n_tasks = n_groups * a.n_head;
+            const int P = resident < n_tasks ? resident : n_tasks;
+            launch_k(kernel, dim3(P), dim3(256), lds, stream, a, groups, n_tasks);
+            return hipGetLastError();
+        };
+        if (max_keys <= 256) return run(k_attend_short<4>);
+        if (max_keys <= 512) return run(k_attend_short<8>);
+        return run(k_attend_long);
     }
     if (noclamp && lds_table) return launch_attend_groups_m<true, true>(a, groups, n_groups, max_keys, stream);
     if (noclamp) return launch_attend_groups_m<true, false>(a, groups, n_groups, max_keys, stream);
@@ -4296,6 +4522,7 @@ int kernel_resources(KernelResource *out, int cap) {
         {"k_attend", (const void *)k_attend},
         {"k_attend_short<4>", (const void *)k_attend_short<4>},
         {"k_attend_short<8>", (const void *)k_attend_short<8>},
+        {"k_attend_long", (const void *)k_attend_long},
         {"k_attend_mfma<noclamp, lds table>", (const void *)k_attend_mfma<true, true, false>},
         {"k_attend_decode64<noclamp>", (const void *)k_attend_decode64<true>},
         {"k_attend_decode_wave<noclamp, 4>", (const void *)k_attend_decode_wave<true, 4>},

@@ -45,4 +45,56 @@ hipError_t launch_layernorm_f32(const LnArgs &a, int n_rows, hipStream_t stream)
 typedef int v4i __attribute__((ext_vector_type(4)));
 constexpr int32_t RES = (1 << 30) - 1;  // gpt2/mod.rs:116
 
+typedef __attribute__((address_space(3))) void lds_void;
+typedef int v2i __attribute__((ext_vector_type(2)));
+typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) v2i lds_v2i;
+
+// s_waitcnt vmcnt(N) with the other counters left at their maximum (gfx9 encoding).
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+    static_assert(N >= 0 && N < 64, "vmcnt range");
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+// A workgroup barrier for LDS data only: this wave's LDS operations complete (lgkmcnt 0), then
+// s_barrier, without the wait for every outstanding global load that the release fence of
+// __syncthreads brings. Global data read after it must not depend on other waves' stores.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0); vmcnt 63 and expcnt 7 leave those alone
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+__device__ __forceinline__ int8_t *attn_out(const AttnArgs &a, int r, int col) {
+    return a.out + (a.out_rows ? panel_off(r, col, a.out_rows) : (size_t)r * a.ldo + col);
+}
+
+// 4 x 4 byte transpose: out[k] holds byte k of w0, w1, w2, w3 (in that order).
+__device__ __forceinline__ void byte_transpose(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3,
+                                               uint32_t out[4]) {
+    const uint32_t t0 = __builtin_amdgcn_perm(w1, w0, 0x05010400u);
+    const uint32_t t1 = __builtin_amdgcn_perm(w1, w0, 0x07030602u);
+    const uint32_t t2 = __builtin_amdgcn_perm(w3, w2, 0x05010400u);
+    const uint32_t t3 = __builtin_amdgcn_perm(w3, w2, 0x07030602u);
+    out[0] = __builtin_amdgcn_perm(t2, t0, 0x05040100u);
+    out[1] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);
+    out[2] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
+    out[3] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
+}
+
+// x, hidden from the optimizer (a value it cannot prove invariant in a loop)
+__device__ __forceinline__ int opaque_vgpr(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
+// v_med3_i32(x, 0, hi) for a wave-uniform hi (the compiler forms med3 only for constant bounds)
+__device__ __forceinline__ int32_t clamp0_uniform(int32_t x, int32_t hi) {
+    int32_t r;
+    asm("v_med3_i32 %0, %1, 0, %2" : "=v"(r) : "v"(x), "s"(hi));
+    return r;
+}
+
 }  // namespace hs
