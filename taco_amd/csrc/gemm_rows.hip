@@ -20,7 +20,7 @@ namespace hs {
 // outputs) is stored with one access. `bias`, `mult`, `x` (the residual row's 4 values) and `ri`
 // (the row's slot and position) were loaded before the product.
 struct RowsEpi {
-    v4i bias, mult, x;
+    v4i bias, mult, x, wsum;
     RowInfo ri;
 };
 
@@ -39,8 +39,13 @@ __device__ __forceinline__ RowsEpi rows_epi_load(const GemmArgs &g, int m, int n
             p.mult[e] = g.mult[n];
         }
     }
-    const int mc = m < g.m ? m : g.m - 1;
-    if constexpr (EPI == (int)Epi::Residual) {
+    constexpr bool WIDE = EPI == (int)Epi::ResidualWide;
+    const int rows = WIDE ? g.rows : g.m, mc = m < rows ? m : rows - 1;
+    if constexpr (WIDE) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) p.wsum[e] = g.wsum[n4 + e < g.n ? n4 + e : g.n - 1];
+    }
+    if constexpr (EPI == (int)Epi::Residual || WIDE) {
         const int32_t *x = (const int32_t *)g.out + (size_t)mc * g.ldo + n4;
         if (n4 + 4 <= g.n && ((uintptr_t)x & 15) == 0) {
             p.x = *(const v4i *)x;
@@ -57,8 +62,10 @@ __device__ __forceinline__ RowsEpi rows_epi_load(const GemmArgs &g, int m, int n
 }
 
 template <int EPI>
-__device__ __forceinline__ void rows_epi(const GemmArgs &g, int m, int n4, const v4i &acc, const RowsEpi &p) {
-    if (m >= g.m || n4 >= g.n) return;
+__device__ __forceinline__ void rows_epi(const GemmArgs &g, int m, int n4, const v4i &acc, const v4i &lo,
+                                         const RowsEpi &p) {
+    constexpr bool WIDE = EPI == (int)Epi::ResidualWide;  // acc and lo: the planes' products
+    if (m >= (WIDE ? g.rows : g.m) || n4 >= g.n) return;
     const int cnt = g.n - n4 < 4 ? g.n - n4 : 4;
     if (EPI == (int)Epi::Raw) {
         int32_t *o = (int32_t *)g.out + (size_t)m * g.ldo + n4;
@@ -70,8 +77,17 @@ __device__ __forceinline__ void rows_epi(const GemmArgs &g, int m, int n4, const
     // rescale(a + bias, mult, shift) (int.rs:63-67): |a + bias| < 2^32, exact in i64
     int64_t r[4];
 #pragma unroll
-    for (int e = 0; e < 4; e++) r[e] = rescale_small((int64_t)acc[e] + p.bias[e], p.mult[e], (uint32_t)g.shift);
-    if (EPI == (int)Epi::Residual) {  // ops.rs:131-145: x = clamp(x + sat32(r), +-R)
+    for (int e = 0; e < 4; e++) {
+        if constexpr (WIDE) {  // dot = 256 hi + lo + 128 wsum (below 2^39)
+            const int64_t v = (int64_t)acc[e] * 256 + lo[e] + 128 * (int64_t)p.wsum[e] + p.bias[e];
+            r[e] = g.shift >= 16 && g.shift <= 62
+                       ? rescale_wide47(v, p.mult[e], (uint32_t)g.shift)
+                       : clamp128(rescale_full(v, p.mult[e], (uint32_t)g.shift), INT32_MIN, INT32_MAX);
+        } else {
+            r[e] = rescale_small((int64_t)acc[e] + p.bias[e], p.mult[e], (uint32_t)g.shift);
+        }
+    }
+    if (EPI == (int)Epi::Residual || WIDE) {  // ops.rs:131-145: x = clamp(x + sat32(r), +-R)
         int32_t *x = (int32_t *)g.out + (size_t)m * g.ldo + n4;
         v4i v;
 #pragma unroll
@@ -114,9 +130,9 @@ __device__ __forceinline__ void rows_epi(const GemmArgs &g, int m, int n4, const
     } else if (EPI == (int)Epi::Gelu) {  // the operand of the next product, in panels
         store4((int8_t *)g.out + panel_off(m, n4, g.out_rows), [&](int e) { return b[e]; });
     } else {  // GeluWide: the two planes of each i16 output, hi = v >> 8, lo = (v & 255) - 128
-        store4((int8_t *)g.out + panel_off(2 * (size_t)m, n4, g.out_rows),
+        store4((int8_t *)g.out + panel_off(plane_row(m, 0), n4, g.out_rows),
                [&](int e) { return (uint32_t)((int32_t)(int16_t)b[e] >> 8); });
-        store4((int8_t *)g.out + panel_off(2 * (size_t)m + 1, n4, g.out_rows),
+        store4((int8_t *)g.out + panel_off(plane_row(m, 1), n4, g.out_rows),
                [&](int e) { return (uint32_t)(((int32_t)(int16_t)b[e] & 255) - 128); });
     }
 }
@@ -125,7 +141,10 @@ __device__ __forceinline__ void rows_epi(const GemmArgs &g, int m, int n4, const
 // keeps U k-steps of fragments in flight: (MT + NT) U 16-byte registers per lane.
 template <int EPI, int MT, int NT, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void k_gemm_rows(GemmArgs g) {
-    constexpr int U = MT + NT <= 3 ? 6 : 4, TILES = MT * NT, TPW = (TILES + WAVES - 1) / WAVES;
+    constexpr int U = MT + NT <= 3 ? 6 : 4, TILES = MT * NT;
+    // the wide product: row tiles 2 i and 2 i + 1 hold the planes of the same 16 rows (plane_row)
+    constexpr int PL = EPI == (int)Epi::ResidualWide ? 2 : 1, OUTS = TILES / PL, TPW = (OUTS + WAVES - 1) / WAVES;
+    static_assert(MT % PL == 0, "whole plane pairs");
     __shared__ __attribute__((aligned(16))) v4i red[WAVES][TILES][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // Workgroup L runs on XCD L % 8: XCD x takes the x-th contiguous chunk of the tiles, row tiles
@@ -146,7 +165,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_rows(GemmArgs g) {
     // The epilogue's operands of the tiles this wave finishes (tile wave + t WAVES of the
     // workgroup): lane l holds row 16 i + l % 16, columns 16 j + 4 (l / 16) ..
     RowsEpi ep[TPW];
-    auto tile_m = [&](int t) { return m0 + 16 * (t / NT) + (lane & 15); };
+    auto tile_m = [&](int t) { return m0 / PL + 16 * (t / NT) + (lane & 15); };
     auto tile_n = [&](int t) { return n0 + 16 * (t % NT) + 4 * (lane >> 4); };
     // fragment loads: lane l reads row l % 16, bytes 16 (l / 16) .. of a 16 x 64 block
     const size_t pa = (size_t)g.a_rows * 64, pw = (size_t)g.w_rows * 64;  // bytes per panel
@@ -178,7 +197,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_rows(GemmArgs g) {
 #pragma unroll
         for (int t = 0; t < TPW; t++) {
             const int tile = wave + t * WAVES;
-            if (tile < TILES) ep[t] = rows_epi_load<EPI>(g, tile_m(tile), tile_n(tile));
+            if (tile < OUTS) ep[t] = rows_epi_load<EPI>(g, tile_m(tile), tile_n(tile));
         }
         int s = 0;
         for (; s + U < steps; s += U) {
@@ -195,7 +214,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_rows(GemmArgs g) {
 #pragma unroll
         for (int t = 0; t < TPW; t++) {
             const int tile = wave + t * WAVES;
-            if (tile < TILES) ep[t] = rows_epi_load<EPI>(g, tile_m(tile), tile_n(tile));
+            if (tile < OUTS) ep[t] = rows_epi_load<EPI>(g, tile_m(tile), tile_n(tile));
         }
     }
 #pragma unroll
@@ -206,11 +225,16 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_rows(GemmArgs g) {
 #pragma unroll
     for (int t = 0; t < TPW; t++) {
         const int tile = wave + t * WAVES;
-        if (tile >= TILES) break;
-        v4i sum = red[0][tile][lane];
+        if (tile >= OUTS) break;
+        const int src = PL == 2 ? (tile / NT) * 2 * NT + tile % NT : tile;
+        v4i sum = red[0][src][lane], lo = v4i{0, 0, 0, 0};
 #pragma unroll
-        for (int w = 1; w < WAVES; w++) sum += red[w][tile][lane];
-        rows_epi<EPI>(g, tile_m(tile), tile_n(tile), sum, ep[t]);
+        for (int w = 1; w < WAVES; w++) sum += red[w][src][lane];
+        if constexpr (PL == 2) {
+#pragma unroll
+            for (int w = 0; w < WAVES; w++) lo += red[w][src + NT][lane];
+        }
+        rows_epi<EPI>(g, tile_m(tile), tile_n(tile), sum, lo, ep[t]);
     }
 }
 
@@ -246,10 +270,12 @@ static RowsTile rows_tile(Epi epi, const GemmArgs &g) {
     auto tiles = [&](int mt, int nt) {
         return ((m + 16 * mt - 1) / (16 * mt)) * (long long)((n + 16 * nt - 1) / (16 * nt));
     };
-    if (tiles(1, 1) <= 256) return {1, 1};
-    if (m <= 16) return {1, 2};
+    if (epi != Epi::ResidualWide) {  // (its row tiles come in pairs)
+        if (tiles(1, 1) <= 256) return {1, 1};
+        if (m <= 16) return {1, 2};
+    }
     if (tiles(2, 1) <= 256) return {2, 1};
-    const bool narrow = epi != Epi::Residual && g.fast32 && g.shift >= 31;
+    const bool narrow = epi != Epi::Residual && epi != Epi::ResidualWide && g.fast32 && g.shift >= 31;
     const long long most = k_pad > 2048 ? 256 : narrow ? 512 : 768;
     if (tiles(2, 2) <= most) return {2, 2};
     if (k_pad > 2048 && tiles(4, 2) <= 256) return {4, 2};
@@ -260,14 +286,15 @@ static RowsTile rows_tile(Epi epi, const GemmArgs &g) {
 template <int EPI>
 static hipError_t launch_rows_e(const GemmArgs &g, const RowsTile &t, hipStream_t stream) {
     // four waves share a tile's k-steps; eight for the 64 x 64 tiles, whose waves hold the most
-    if (t.mt == 1) return t.nt == 1 ? launch_rows_t<EPI, 1, 1, 4>(g, stream) : launch_rows_t<EPI, 1, 2, 4>(g, stream);
+    if constexpr (EPI != (int)Epi::ResidualWide)
+        if (t.mt == 1) return t.nt == 1 ? launch_rows_t<EPI, 1, 1, 4>(g, stream) : launch_rows_t<EPI, 1, 2, 4>(g, stream);
     if (t.mt == 2) return t.nt == 1 ? launch_rows_t<EPI, 2, 1, 4>(g, stream) : launch_rows_t<EPI, 2, 2, 4>(g, stream);
     return t.nt == 2 ? launch_rows_t<EPI, 4, 2, 4>(g, stream) : launch_rows_t<EPI, 4, 4, 8>(g, stream);
 }
 
 bool gemm_rows_fits(Epi epi, const GemmArgs &g) {
     const bool ok = epi == Epi::Raw || epi == Epi::Act || epi == Epi::Residual || epi == Epi::Gelu ||
-                    epi == Epi::GeluWide;
+                    epi == Epi::GeluWide || epi == Epi::ResidualWide;
     return ok && rows_tile(epi, g).mt > 0;
 }
 
@@ -280,6 +307,7 @@ hipError_t launch_gemm_rows(Epi epi, const GemmArgs &g, hipStream_t stream) {
         case Epi::Residual: return launch_rows_e<2>(g, t, stream);
         case Epi::Gelu: return launch_rows_e<3>(g, t, stream);
         case Epi::GeluWide: return launch_rows_e<6>(g, t, stream);
+        case Epi::ResidualWide: return launch_rows_e<7>(g, t, stream);
         default: return hipErrorInvalidValue;
     }
 }

@@ -129,6 +129,7 @@ struct DevLinear {
     int32_t *b = nullptr, *m = nullptr;
     int s = 0, n = 0, k = 0, n_pad = 0, k_pad = 0;
     int fast32 = 0;  // k * 2^14 + max|b| < 2^31: every acc + b fits i32
+    int wide32 = 0;  // of an i16 input: every rescaled output fits i32 (fits_wide)
     int32_t *wsum = nullptr;  // sum_k w[n][k], for an i16 input as planes (|wsum| <= 2^23)
 };
 
@@ -158,6 +159,15 @@ int fits_i32(size_t k, const int32_t *b, size_t n) {
     int64_t mb = 0;
     for (size_t i = 0; b && i < n; i++) mb = std::max<int64_t>(mb, b[i] < 0 ? -(int64_t)b[i] : b[i]);
     return (int64_t)k * 16384 + mb < ((int64_t)1 << 31) ? 1 : 0;
+}
+
+// |w . a + b| <= k 2^22 + max|b| for i8 weights and i16 activations; when that is below 2^(s-1),
+// |(w . a + b) m| 2^-s < 2^30, so the rescaled value is an i32.
+int fits_wide(size_t k, const int32_t *b, size_t n, int s) {
+    if (s < 16 || s > 62 || k >= 32768) return 0;
+    int64_t mb = 0;
+    for (size_t i = 0; b && i < n; i++) mb = std::max<int64_t>(mb, b[i] < 0 ? -(int64_t)b[i] : b[i]);
+    return ((int64_t)k << 22) + mb < ((int64_t)1 << (s - 1)) ? 1 : 0;
 }
 
 struct DevLn {
@@ -222,6 +232,7 @@ hs_status upload_linear(DevMem &mem, const hs::HostLinear &l, DevLinear &o) {
     if (st == HS_OK) st = mem.upload(o.m, l.m.data(), l.m.size(), o.n_pad);
     o.s = l.s;
     o.fast32 = fits_i32(l.cols, l.b.data(), l.b.size());
+    o.wide32 = fits_wide(l.cols, l.b.data(), l.b.size(), l.s);
     return st;
 }
 
@@ -426,11 +437,11 @@ hs_status upload_model(hs_device *dev, std::unique_ptr<hs_model> &m, hs_model **
             return st;
         }
         b.gelu_off = (int)hb.gelu_len / 2;
-        if (!hb.gelu_wide && hb.gelu8.size() >= 16 && hb.gelu8.size() % 16 == 0) {
-            // the span [lo, hi] outside which every entry equals the end entry it lies beyond: the
-            // epilogue clamps its index to it and copies only entries lo16 .. (16-byte aligned)
-            const std::vector<int8_t> &t = hb.gelu8;
+        // the span [lo, hi] outside which every entry equals the end entry it lies beyond: the epilogue
+        // clamps its index to it and copies only entries lo16 .. (16-byte aligned)
+        auto span = [&](const auto &t) {
             const int len = (int)t.size();
+            if (len < 16 || len % 16 != 0) return;
             int lo = 0, hi = len - 1;
             while (lo + 1 < len && t[lo + 1] == t[0]) lo++;
             while (hi - 1 > lo && t[hi - 1] == t[len - 1]) hi--;
@@ -440,7 +451,9 @@ hs_status upload_model(hs_device *dev, std::unique_ptr<hs_model> &m, hs_model **
             b.gelu_chi = hi - b.gelu_off;
             b.gelu_shift = b.gelu_off - lo16;
             b.gelu_copy = end16 - lo16;
-        }
+        };
+        if (hb.gelu_wide) span(hb.gelu16);
+        else span(hb.gelu8);
     }
     if ((st = upload_ln(mem, h.ln_f, (int)h.ln_beta_frac, m->ln_f)) != HS_OK) return st;
     // padded to a multiple of 256 entries: the prefill attention loads it in 1 KiB chunks
@@ -1041,13 +1054,17 @@ hs_status run_pass(hs_batch &b, const std::vector<PassRow> &rows, Out out, const
         g.bias = lin.b; g.mult = lin.m; g.shift = lin.s; g.out = o; g.ldo = ldo;
         g.params_padded = 1;
         g.out_rows = (epi == Epi::GeluWide ? 2 : 1) * RP;
-        g.fast32 = epi == Epi::ResidualWide ? 0 : lin.fast32;
+        g.fast32 = epi == Epi::ResidualWide || epi == Epi::LogitsWide ? lin.wide32 : lin.fast32;
+        if (epi == Epi::ResidualWide || epi == Epi::LogitsWide) {  // rows_n rows of planes
+            g.rows = rows_n;
+            g.m = hs::plane_rows(rows_n);
+        }
         g.gelu = gelu; g.gelu16 = gelu16; g.gelu_off = gelu_off; g.wsum = lin.wsum;
         if (gspan && gspan->gelu_copy > 0) {
             g.gelu_lo = gspan->gelu_lo; g.gelu_clo = gspan->gelu_clo; g.gelu_chi = gspan->gelu_chi;
             g.gelu_shift = gspan->gelu_shift; g.gelu_copy = gspan->gelu_copy;
         }
-        const uint64_t ops = 2ull * (uint64_t)rows_n * (uint64_t)lin.n * (uint64_t)lin.k;
+        const uint64_t ops = 2ull * (uint64_t)(g.rows ? 2 * rows_n : rows_n) * (uint64_t)lin.n * (uint64_t)lin.k;
         return b.launch(label, ops, [&] { return hs::launch_gemm(epi, g, st); });
     };
     const bool kv_fused = m.hd % 16 == 0 && m.d % 16 == 0;
@@ -1112,8 +1129,8 @@ hs_status run_pass(hs_batch &b, const std::vector<PassRow> &rows, Out out, const
         HIP_TRY(ln(blk.ln2, nullptr, n, b.d_a));
         if (blk.gelu16) {  // i16 GELU outputs as planes, mlp_proj over 2n operand rows
             HIP_TRY(gemm("gemm_fc", Epi::GeluWide, blk.c_fc, b.d_a, RP, n, b.d_g, 0, nullptr, blk.gelu_off,
-                         blk.gelu16));
-            HIP_TRY(gemm("gemm_mlp", Epi::ResidualWide, blk.mlp_proj, b.d_g, 2 * RP, 2 * n, b.d_x, m.d));
+                         blk.gelu16, 0, &blk));
+            HIP_TRY(gemm("gemm_mlp", Epi::ResidualWide, blk.mlp_proj, b.d_g, 2 * RP, n, b.d_x, m.d));
         } else {
             HIP_TRY(gemm("gemm_fc", Epi::Gelu, blk.c_fc, b.d_a, RP, n, b.d_g, 0, blk.gelu, blk.gelu_off, nullptr, 0,
                          &blk));
@@ -1130,12 +1147,14 @@ hs_status run_pass(hs_batch &b, const std::vector<PassRow> &rows, Out out, const
         }
         return HS_OK;
     }
-    // a 16-bit ln_f (version 2) writes two operand rows (planes) per output row
+    // a 16-bit ln_f (version 2) writes two operand rows per output row (planes, in blocks of 16 rows:
+    // a chunk starts at a multiple of 256)
     const int pr = m.wide_ln_f ? 2 : 1;
     HIP_TRY(ln(m.ln_f, b.d_src, n_out, b.d_af, m.wide_ln_f ? 16 : 8));
     DevLinear head;
     head.w = m.wte; head.m = m.logit_m; head.s = m.host.logit_s; head.n = m.V; head.k = m.d;
     head.n_pad = m.V_pad; head.k_pad = m.d_pad; head.wsum = m.wte_sum;
+    head.wide32 = fits_wide((size_t)m.d, nullptr, 0, head.s);
     const size_t per_row = out == Out::Intervals ? 3 : (size_t)m.V;
     std::vector<uint64_t> host(out == Out::Weights ? (size_t)n_out * per_row : 0);
     for (int c0 = 0; c0 < n_out; c0 += (int)b.chunk_rows) {
@@ -1144,7 +1163,8 @@ hs_status run_pass(hs_batch &b, const std::vector<PassRow> &rows, Out out, const
             hs::GemmArgs g;
             // the chunk's operand rows start at row pr c0 of the panels of pr RP rows
             g.a = b.d_af + (size_t)pr * c0 * 64; g.a_rows = pr * RP; g.w = m.wte; g.w_rows = m.V_pad;
-            g.m = pr * cn; g.n = m.V; g.k_pad = m.d_pad;
+            g.m = m.wide_ln_f ? hs::plane_rows(cn) : cn; g.rows = cn; g.n = m.V; g.k_pad = m.d_pad;
+            g.fast32 = m.wide_ln_f && fits_wide((size_t)m.d, nullptr, 0, m.host.logit_s);
             g.mult = m.logit_m; g.shift = m.host.logit_s; g.out = b.d_d16; g.ldo = m.ld16;
             g.params_padded = 1;
             g.tmax = b.d_tmax; g.tmax_ld = m.ntiles; g.cap16 = (int)m.host.logits_exp.size() - 1;
@@ -1179,8 +1199,8 @@ hs_status run_pass(hs_batch &b, const std::vector<PassRow> &rows, Out out, const
             }
         } else {
             HIP_TRY(gemm("gemm_logits", m.wide_ln_f ? Epi::LogitsWide : Epi::Logits, head,
-                         b.d_af + (size_t)pr * c0 * 64, pr * RP, pr * cn, b.d_logits, m.V, nullptr, 0,
-                         nullptr, head_group(pr * cn)));
+                         b.d_af + (size_t)pr * c0 * 64, pr * RP, cn, b.d_logits, m.V, nullptr, 0, nullptr,
+                         head_group(m.wide_ln_f ? hs::plane_rows(cn) : cn)));
             hs::CoderArgs ca;
             ca.logits = b.d_logits; ca.ld = m.V; ca.vocab = m.V; ca.table = m.logits_exp;
             ca.table_len = (int)m.host.logits_exp.size();

@@ -368,6 +368,13 @@ HS_HD int32_t attn_out_planes(int32_t hi, int32_t lo, int32_t m, uint32_t s) {
     return r < -127 ? -127 : (r > 127 ? 127 : r);
 }
 
+// rescale_full(v, m, s) for |v| < 2^47 and 16 <= s <= 62 in i64, by the same split: v = hi 2^16 + lo
+// with 0 <= lo < 2^16, B = lo m + 2^(s-1) (below 2^62), A = hi m (|A| < 2^62).
+HS_HD int64_t rescale_wide47(int64_t v, int32_t m, uint32_t s) {
+    const int64_t b = (int64_t)(int32_t)((uint32_t)v & 0xffffu) * m + ((int64_t)1 << (s - 1));
+    return ((int64_t)(int32_t)(v >> 16) * m + (b >> 16)) >> (s - 16);
+}
+
 HS_HD double softmax_sp(uint64_t S, int P) { return -ldexp((double)S, -P); }
 HS_HD uint32_t softmax_p_of(uint32_t e, double R, double sp) {
     const double ed = (double)e;

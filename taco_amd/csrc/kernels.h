@@ -17,10 +17,11 @@ struct RowInfo {
 enum class Epi : int {
     Raw = 0, Act = 1, Residual = 2, Gelu = 3, Logits = 4, LogitsCompact = 5,
     // Model-file version 2 (i16 activations, crates/hardshell/src/gpt2/ops.rs:178-206,246-277).
-    // An i16 activation v is stored as two i8 planes in adjacent operand rows: row 2r holds
-    // hi = v >> 8, row 2r + 1 holds lo = (v & 255) - 128, so v = 256 hi + lo + 128.
+    // An i16 activation v is stored as two i8 planes, hi = v >> 8 and lo = (v & 255) - 128 (v = 256 hi +
+    // lo + 128), of 16 rows each in turn (plane_row): the lane of an MFMA tile pair that holds
+    // hi of a row and 4 columns then holds lo of the same outputs too.
     GeluWide = 6,          // c_fc + i16 GELU table (gelu16), out: the two planes of each row
-    ResidualWide = 7,      // m = 2 x rows of planes; x += rescale(256 hi + lo + 128 wsum + b)
+    ResidualWide = 7,      // m = plane_rows(rows); x += rescale(256 hi + lo + 128 wsum + b)
     LogitsWide = 8,        // as Logits over planes (i64 out)
     LogitsCompactWide = 9  // as LogitsCompact over planes
 };
@@ -33,11 +34,16 @@ __host__ __device__ inline size_t panel_off(size_t r, size_t k, size_t rows) {
     return ((k >> 6) * rows + r) * 64 + (k & 63);
 }
 
+// The operand row of plane pl (0: hi, 1: lo) of row r, and the operand rows of n rows of planes.
+__host__ __device__ inline size_t plane_row(size_t r, int pl) { return (r >> 4) * 32 + (r & 15) + 16 * (size_t)pl; }
+__host__ __device__ inline int plane_rows(int n) { return (n + 15) / 16 * 32; }
+
 struct GemmArgs {
     const int8_t *a = nullptr;  // panels [k_pad / 64][a_rows][64], rows m_pad and more
     const int8_t *w = nullptr;  // panels [k_pad / 64][w_rows][64], w_rows >= n_pad
     int a_rows = 0, w_rows = 0;  // the panel row counts (0: m_pad and n_pad)
     int m = 0, n = 0, k_pad = 0;
+    int rows = 0;  // the wide epilogues: the output rows (m = plane_rows(rows))
     const int32_t *bias = nullptr;  // [n] (Act, Residual, Gelu)
     const int32_t *mult = nullptr;  // [n]
     int params_padded = 0;          // 1: bias and mult hold round_up(n, 256) entries (zeros past n)
@@ -64,7 +70,9 @@ struct GemmArgs {
     int cap16 = 0;
     int group = 0;  // M-tiles per group of the tile order (0: gemm_group(m))
     // 1 if the caller has shown |acc + bias| < 2^31 for every output (K * 2^14 + max|bias|
-    // < 2^31: |a|, |w| <= 128); the epilogue then rescales with one i64 multiply-add.
+    // < 2^31: |a|, |w| <= 128); the epilogue then rescales with one i64 multiply-add. The wide
+    // epilogues: |dot + bias| < 2^(shift - 1), 16 <= shift <= 62 and K < 2^15, so that the rescaled
+    // value is an i32.
     int fast32 = 0;
     // Act only: when kv_rows is set, columns kv_d .. 3 kv_d (K and V of a c_attn output) go to
     // the caches kc, vc [slot][kv_h][kv_ctx][kv_hd] at the row's slot and position instead of
@@ -134,7 +142,7 @@ struct LnArgs {
     const int32_t *src = nullptr;  // optional: output row i reads x row src[i]
     const int64_t *gm = nullptr;   // gamma[j] * m, exact in i64 (|gamma m| < 2^46)
     int bits = 8;                  // 16: clamp to +-32767 and write the two i8 planes of each row
-                                   // (hi to out row 2i, lo to row 2i + 1), as the wide GEMMs read
+                                   // (plane_row), as the wide GEMMs read
     // The single-precision rule (ln_elem_z), set when it holds for this LayerNorm:
     // gamma and 128 + beta as floats, ln_margin of the largest |beta|, m 2^-s and 1 / d.
     const float *gf = nullptr, *bf = nullptr;

@@ -144,10 +144,14 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
     static_assert(NST <= 6 && (NST - 1) * LOADS < 64, "ring depth");
     static_assert(TI * TJ <= 32 && (BM == GEMM_BM || (BM == 128 && BN == 192) || (BM == 64 && BN == 64)),
                   "tile shapes");
-    // The i16-plane epilogues pair rows 2r and 2r + 1 in one lane and keep the W-as-columns
-    // layout; every other epilogue takes four consecutive columns of a row per lane.
-    constexpr bool SWAP = EPI != (int)Epi::ResidualWide && EPI != (int)Epi::LogitsWide &&
-                          EPI != (int)Epi::LogitsCompactWide;
+    // The wide epilogues: tiles 2 i and 2 i + 1 of a wave hold the hi and lo planes of the same 16
+    // rows (plane_row), so a wave's TI tiles are TR = TI / 2 tiles of outputs, staged and stored as
+    // those of the i8 products. (With planes in adjacent rows a lane held single columns, and
+    // stored 2 or 4 bytes at a time after i128 rescales: mlp.c_proj of 3,370 rows 49.7 us, 30.8
+    // now; the head's 2,048-row chunk 398 -> 209 us.)
+    constexpr bool WIDE = EPI == (int)Epi::ResidualWide || EPI == (int)Epi::LogitsWide ||
+                          EPI == (int)Epi::LogitsCompactWide;
+    constexpr int TR = WIDE ? TI / 2 : TI;
     extern __shared__ __attribute__((aligned(1024))) int8_t gemm_lds[];  // [stages][FRAGS][1024]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -171,10 +175,10 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
 
     // The first k-step's MFMAs take the accumulators' start values as their C operand (no
     // zeroing moves): 0, or, for the NARROW epilogues with a bias, the bias of the lane's columns
-    // (SWAP: columns cw + 16 j + 4 (lane / 16) + e). fast32 bounds every partial sum plus the
+    // (columns cw + 16 j + 4 (lane / 16) + e). fast32 bounds every partial sum plus the
     // bias by k 2^14 + max|b| < 2^31, so the i32 accumulation stays exact and the epilogue adds
     // no bias.
-    constexpr bool FOLD_BIAS = NARROW && SWAP && (EPI == (int)Epi::Act || EPI == (int)Epi::Residual ||
+    constexpr bool FOLD_BIAS = NARROW && (EPI == (int)Epi::Act || EPI == (int)Epi::Residual ||
                                                   EPI == (int)Epi::Gelu || EPI == (int)Epi::GeluWide);
     v4i acc[TI][TJ];
     v4i init[TJ];
@@ -192,8 +196,7 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
         }
     }
     auto mfma_ij = [&](const v4i &a, const v4i &b, const v4i &c) {
-        return SWAP ? __builtin_amdgcn_mfma_i32_16x16x64_i8(b, a, c, 0, 0, 0)
-                    : __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
+        return __builtin_amdgcn_mfma_i32_16x16x64_i8(b, a, c, 0, 0, 0);
     };
     auto mfma_step = [&](const v4i *af, const v4i *bf) {
 #pragma unroll
@@ -437,9 +440,8 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
     if (kt < nk) step(kt, fa1, fb1, fa0, fb0, Flag<false>{});
     }
 
-    // Epilogue. Lane layout of each 16 x 16 tile (i, j) of the wave: with SWAP (the W fragment is
-    // the MFMA's first operand) the lane holds C[16 i + lane % 16][16 j + 4 (lane / 16) + e], four
-    // consecutive columns of one row; otherwise C[16 i + 4 (lane / 16) + e][16 j + lane % 16].
+    // Epilogue. The W fragment is the MFMA's first operand, so of each 16 x 16 tile (i, j) of the wave
+    // the lane holds C[16 i + lane % 16][16 j + 4 (lane / 16) + e]: four consecutive columns of a row.
     // rescale(a + bias, mult, shift) (int.rs:63-67). With the host's bound |a + bias| < 2^31
     // (fast32; the logits have no bias and |a| <= 2^30), |(a + bias) mult| < 2^62: one i64
     // multiply-add and an arithmetic shift are exact, and a shift of 63 or more gives 0 as
@@ -451,10 +453,25 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
         if (NARROW || fast) return ((int64_t)(a + bias) * mult + half) >> s_eff;
         return rescale_small((int64_t)a + bias, mult, g.shift);
     };
-    const int rw = m0 + wm * 16 * TI, cw = n0 + wn * 16 * TJ;  // the wave's sub-tile origin
-    if constexpr (SWAP) {
+    // rescale of 256 hi + lo + add (add = 128 wsum + bias): |dot + bias| <= K 2^22 + 2^31 < 2^39
+    auto rqw = [&](int32_t hi, int32_t lo, int64_t add, int32_t mult) -> int64_t {
+        const int64_t v = (int64_t)hi * 256 + add + lo;
+        if (NARROW || (g.shift >= 16 && g.shift <= 62)) return rescale_wide47(v, mult, (uint32_t)g.shift);
+        return clamp128(rescale_full(v, mult, g.shift), -((int64_t)1 << 62), (int64_t)1 << 62);
+    };
+    // the same without a bias: 256 hi + 128 ws = 128 (2 hi + ws), an i32 for the NARROW forms (K < 2^15)
+    auto rqw2 = [&](int32_t hi, int32_t lo, int32_t ws, int32_t mult) -> int64_t {
+        if (NARROW) return rescale_wide47((int64_t)(2 * hi + ws) * 128 + lo, mult, (uint32_t)g.shift);
+        return rqw(hi, lo, 128 * (int64_t)ws, mult);
+    };
+    const int cw = n0 + wn * 16 * TJ;                     // the wave's first column
+    const int rw = (m0 + wm * 16 * TI) / (WIDE ? 2 : 1);  // and output row
+    const int M = WIDE ? g.rows : g.m;
+    {
         const int rl = lane & 15, cg = lane >> 4;
-        constexpr bool HAS_BIAS = EPI == (int)Epi::Act || EPI == (int)Epi::Residual || EPI == (int)Epi::Gelu ||
+        constexpr bool RESIDUAL = EPI == (int)Epi::Residual || EPI == (int)Epi::ResidualWide;
+        constexpr bool COMPACT = EPI == (int)Epi::LogitsCompact || EPI == (int)Epi::LogitsCompactWide;
+        constexpr bool HAS_BIAS = EPI == (int)Epi::Act || RESIDUAL || EPI == (int)Epi::Gelu ||
                                   EPI == (int)Epi::GeluWide;
         constexpr bool vec = VEC;
         // The rescale parameters of column group j of the lane (columns cw + 16 j + 4 cg + e).
@@ -478,6 +495,29 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
                 mj[e] = (EPI != (int)Epi::Raw && ok) ? g.mult[n] : 0;
             }
         };
+        // The wide epilogues: 128 wsum + bias of column group j.
+        auto addends = [&](int j, const int32_t *bj, int64_t *aj) {
+            const int n4 = cw + 16 * j + 4 * cg;
+#pragma unroll
+            for (int e = 0; e < 4; e++) aj[e] = n4 + e < g.n ? 128 * (int64_t)g.wsum[n4 + e] + bj[e] : 0;
+        };
+        if constexpr (EPI == (int)Epi::ResidualWide) {  // ops.rs:178-206: the i32 (saturated) updates, in place
+#pragma unroll
+            for (int j = 0; j < TJ; j++) {
+                int32_t bj[4], mj[4];
+                int64_t aj[4];
+                params(j, bj, mj);
+                addends(j, bj, aj);
+#pragma unroll
+                for (int i = 0; i < TR; i++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int64_t r = rqw(acc[2 * i][j][e], acc[2 * i + 1][j][e], aj[e], mj[e]);
+                        acc[i][j][e] = NARROW ? (int32_t)r : (int32_t)clamp64(r, INT32_MIN, INT32_MAX);
+                    }
+                asm volatile("" ::: "memory");  // the next group's parameter loads stay below
+            }
+        }
         // Act, Gelu, GeluWide, Residual: the op's rule in place, one column group at a time.
         if (EPI == (int)Epi::Act || EPI == (int)Epi::Gelu || EPI == (int)Epi::GeluWide || EPI == (int)Epi::Residual) {
 #pragma unroll
@@ -500,28 +540,29 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
                                         : (int32_t)clamp64(r, g.gelu_clo, g.gelu_chi)) +
                                 g.gelu_shift;
                         } else {
-                            v = (NARROW ? med3_i32((int32_t)r, -g.gelu_off, g.gelu_off - 1)
-                                        : (int32_t)clamp64(r, -g.gelu_off, g.gelu_off - 1)) +
-                                g.gelu_off;
-                            v = g.gelu16[v];  // the i16 table through the caches
+                            // GeluWide: the index from gelu_lo, as Gelu
+                            v = (NARROW ? med3_i32((int32_t)r, g.gelu_clo, g.gelu_chi)
+                                        : (int32_t)clamp64(r, g.gelu_clo, g.gelu_chi)) +
+                                g.gelu_shift;
+                            if (BN != 256) v = g.gelu16[g.gelu_lo + v];  // the i16 table through the caches
                         }
                         acc[i][j][e] = v;
                     }
                 asm volatile("" ::: "memory");  // the next group's parameter loads stay below
             }
         }
-        if (EPI == (int)Epi::Residual) {  // ops.rs:131-145
+        if (RESIDUAL) {  // ops.rs:131-145
             // clamp(x + clamp(r, +-2^40), +-R) == clamp(x + sat32(r), +-R) for |x| <= R, and
             // == med3(sat32(x + sat32(r)), -R, R): a sum beyond i32 saturates to a value beyond R
             // on the same side, so the i32 saturating add and one med3 give it exactly.
             auto res = [](int32_t x, int32_t r) { return med3_i32(__builtin_elementwise_add_sat(x, r), -RES, RES); };
             if (!vec) {
 #pragma unroll
-                for (int i = 0; i < TI; i++)
+                for (int i = 0; i < TR; i++)
 #pragma unroll
                     for (int j = 0; j < TJ; j++) {
                         const int m = rw + 16 * i + rl, n4 = cw + 16 * j + 4 * cg;
-                        if (m >= g.m) continue;
+                        if (m >= M) continue;
                         int32_t *x = (int32_t *)g.out + (size_t)m * g.ldo + n4;
 #pragma unroll
                         for (int e = 0; e < 4; e++)
@@ -533,9 +574,9 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
             // the lane's four outputs of a row are one 16-byte LDS write; the read-modify-write of
             // x then covers whole 16-byte pieces of rows (CPR per row), all Q loads of a part in
             // flight together (parts of 64 rows of 64 columns held 32 vectors per lane and spilled).
-            constexpr int HR = 32, NH = 16 * TI / HR, RS = 64 * TJ + 16;
+            constexpr int HR = TR >= 2 ? 32 : 16, NH = 16 * TR / HR, RS = 64 * TJ + 16;
             constexpr int CPR = 4 * TJ, Q = HR * CPR / 64;
-            static_assert(NH * HR == 16 * TI && HR * RS <= 18432 && Q * 64 == HR * CPR, "residual staging");
+            static_assert(NH * HR == 16 * TR && HR * RS <= 18432 && Q * 64 == HR * CPR, "residual staging");
             __syncthreads();  // every wave finished reading the stages
             int8_t *wr = gemm_lds + wave * 18432;
 #pragma unroll
@@ -551,14 +592,14 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
                     const int pc = q * 64 + lane, rl2 = pc / CPR, cl = (pc % CPR) * 4;
                     const int m = rw + HR * h + rl2, n = cw + cl;
                     rv[q] = *(const v4i *)(wr + rl2 * RS + cl * 4);
-                    xv[q] = (m < g.m && n + 4 <= g.n) ? *(const v4i *)((const int32_t *)g.out + (size_t)m * g.ldo + n)
+                    xv[q] = (m < M && n + 4 <= g.n) ? *(const v4i *)((const int32_t *)g.out + (size_t)m * g.ldo + n)
                                                        : v4i{0, 0, 0, 0};
                 }
 #pragma unroll
                 for (int q = 0; q < Q; q++) {
                     const int pc = q * 64 + lane, rl2 = pc / CPR, cl = (pc % CPR) * 4;
                     const int m = rw + HR * h + rl2, n = cw + cl;
-                    if (m >= g.m) continue;
+                    if (m >= M) continue;
                     int32_t *x = (int32_t *)g.out + (size_t)m * g.ldo + n;
                     if (n + 4 <= g.n) {
                         v4i o;
@@ -574,17 +615,19 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
             }
             return;
         }
-        if (EPI == (int)Epi::Raw || EPI == (int)Epi::Logits) {  // i32 products; ops.rs:229-234 (i64)
+        if (EPI == (int)Epi::Raw || EPI == (int)Epi::Logits || EPI == (int)Epi::LogitsWide) {  // i32 products; ops.rs:229-234 (i64)
 #pragma unroll
             for (int j = 0; j < TJ; j++) {
                 int32_t bj[4], mj[4];
+                int64_t aj[4] = {0, 0, 0, 0};
                 params(j, bj, mj);
+                if constexpr (WIDE) addends(j, bj, aj);
 #pragma unroll
-                for (int i = 0; i < TI; i++) {
+                for (int i = 0; i < TR; i++) {
                     const int m = rw + 16 * i + rl, n4 = cw + 16 * j + 4 * cg;
-                    if (m >= g.m || n4 >= g.n) continue;
+                    if (m >= M || n4 >= g.n) continue;
                     if (EPI == (int)Epi::Raw) {
-                        int32_t *o = (int32_t *)g.out + ((size_t)blockIdx.y * g.m + m) * g.ldo + n4;
+                        int32_t *o = (int32_t *)g.out + ((size_t)blockIdx.y * M + m) * g.ldo + n4;
                         if (vec && n4 + 4 <= g.n) *(v4i *)o = acc[i][j];
                         else
 #pragma unroll
@@ -594,7 +637,8 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
                         int64_t *o = (int64_t *)g.out + (size_t)m * g.ldo + n4;
 #pragma unroll
                         for (int e = 0; e < 4; e++) {
-                            const int64_t r = rq(acc[i][j][e], 0, mj[e]);
+                            const int64_t r = WIDE ? rqw(acc[WIDE ? 2 * i : 0][j][e], acc[WIDE ? 2 * i + 1 : 0][j][e], aj[e], mj[e])
+                                               : rq(acc[i][j][e], 0, mj[e]);
                             if (n4 + e < g.n) o[e] = NARROW ? r : clamp64(r, -SCORE_LIMIT, SCORE_LIMIT);
                         }
                     }
@@ -602,7 +646,7 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
             }
             return;
         }
-        if constexpr (EPI == (int)Epi::LogitsCompact) {
+        if constexpr (COMPACT) {
             static_assert(TI == 8 && TJ == 4, "the compact logits keep 64-column tiles");
             // logit = clamp(rescale(acc, m[n], s), +-2^40) (ops.rs:229-234), stored as the
             // largest logit of this wave's 64 columns (per row) and per logit the distance
@@ -611,10 +655,16 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
             // max - l = (max - tilemax) + (tilemax - l) and c >= cap16 >= len - 1. Each row's 64
             // columns are 16 in each of the 4 lanes lane % 16 + 16 c.
             int32_t mult[4][4];
+            int32_t ws[4][4];  // the wide form (no bias): wsum, 16 registers where the i64 addends take 32
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 int32_t bj[4];
                 params(j, bj, mult[j]);
+                if constexpr (WIDE) {
+                    const int n4 = cw + 16 * j + 4 * cg;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) ws[j][e] = n4 + e < g.n ? g.wsum[n4 + e] : 0;
+                }
             }
             int8_t *wr = gemm_lds + wave * 18432;  // this wave's staging region: 128 rows x 144 B
             if (vec) __syncthreads();              // every wave finished reading the stages
@@ -628,13 +678,14 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
             const bool full = cw + 64 <= g.n;
             auto rows = [&](auto FULL) {
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
+            for (int i = 0; i < TR; i++) {
                 L l[4][4], mx = LMIN;
 #pragma unroll
                 for (int j = 0; j < 4; j++)
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
-                        const int64_t r = rq(acc[i][j][e], 0, mult[j][e]);
+                        const int64_t r = WIDE ? rqw2(acc[WIDE ? 2 * i : 0][j][e], acc[WIDE ? 2 * i + 1 : 0][j][e], ws[j][e], mult[j][e])
+                                               : rq(acc[i][j][e], 0, mult[j][e]);
                         const bool ok = FULL || cw + 16 * j + 4 * cg + e < g.n;
                         l[j][e] = ok ? (NARROW ? (L)r : (L)clamp64(r, -SCORE_LIMIT, SCORE_LIMIT)) : LMIN;
                         mx = l[j][e] > mx ? l[j][e] : mx;
@@ -645,7 +696,7 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
                     mx = u > mx ? u : mx;
                 }
                 const int m = rw + 16 * i + rl;
-                if (m < g.m && cg == 0 && cw < g.n) g.tmax[(size_t)m * g.tmax_ld + cw / 64] = (int64_t)mx;
+                if (m < M && cg == 0 && cw < g.n) g.tmax[(size_t)m * g.tmax_ld + cw / 64] = (int64_t)mx;
                 const U cap = (U)g.cap16;
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
@@ -666,7 +717,7 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
                     }
                     if (vec) {
                         *(uint2 *)(wr + (16 * i + rl) * 144 + (16 * j + 4 * cg) * 2) = make_uint2(w2[0], w2[1]);
-                    } else if (m < g.m) {
+                    } else if (m < M) {
                         uint16_t *o = (uint16_t *)g.out + (size_t)m * g.ldo + cw + 16 * j + 4 * cg;
 #pragma unroll
                         for (int e = 0; e < 4; e++)
@@ -679,11 +730,11 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
             else rows(std::false_type{});
             if (!vec) return;
 #pragma unroll
-            for (int q = 0; q < 16; q++) {
+            for (int q = 0; q < 2 * TR; q++) {
                 const int rl2 = q * 8 + (lane >> 3), cl = (lane & 7) * 8;
                 const v4i v = *(const v4i *)(wr + rl2 * 144 + cl * 2);
                 const int m = rw + rl2, n = cw + cl;
-                if (m >= g.m) continue;
+                if (m >= M) continue;
                 uint16_t *o = (uint16_t *)g.out + (size_t)m * g.ldo + n;
                 if (n + 8 <= g.n) {
                     *(v4i *)o = v;
@@ -701,16 +752,27 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
         // follow it. The 64 x 64 tiles read the table through the caches instead
         // (a copy per workgroup would outweigh the 4,096 lookups of its tile).
         constexpr bool GELU_LDS = BM != 64;
-        const int8_t *gspan = g.gelu + g.gelu_lo;  // entry gelu_lo: index 0 of the lookups
+        const int8_t *gspan = EPI == (int)Epi::GeluWide ? (const int8_t *)(g.gelu16 + g.gelu_lo) : g.gelu + g.gelu_lo;
+        constexpr bool TABLE16 = EPI == (int)Epi::GeluWide && BN == 256;  // the i16 span, 2 bytes an entry
         int toff = 0;
         if (vec) {
             __syncthreads();  // every wave finished reading the stages
-            if (EPI == (int)Epi::Gelu && GELU_LDS) {
-                const int T = g.gelu_copy;
+            if ((EPI == (int)Epi::Gelu && GELU_LDS) || TABLE16) {
+                const int T = (TABLE16 ? 2 : 1) * g.gelu_copy;
                 for (int c = threadIdx.x; c < T / 16; c += 64 * WAVES)
                     *(v4i *)(gemm_lds + 16 * c) = *(const v4i *)(gspan + 16 * c);
                 __syncthreads();
                 toff = (T + 1023) & ~1023;
+            }
+        }
+        if constexpr (TABLE16) {
+#pragma unroll
+            for (int j = 0; j < TJ; j++) {
+#pragma unroll
+                for (int i = 0; i < TI; i++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[i][j][e] = ((const int16_t *)gemm_lds)[acc[i][j][e]];
+                asm volatile("" ::: "memory");  // 4 TI lookups in flight at most
             }
         }
         constexpr int RS8 = 16 * TJ + 16, Q8 = TI * TJ / 4;
@@ -733,7 +795,7 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
 #pragma unroll
             for (int q = 0; q < Q8; q++) {
                 const int m = rw + (q * 64 + lane) / TJ;
-                const RowInfo ri = g.kv_rows[m < g.m ? m : g.m - 1];
+                const RowInfo ri = g.kv_rows[m < M ? m : M - 1];
                 kv_slot[q] = ri.slot;
                 kv_pos[q] = ri.pos;
             }
@@ -756,7 +818,7 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
 #pragma unroll
                         for (int e = 0; e < 4; e++) {
                             const int m = rw + 16 * i + rl, n = cw + 16 * j + 4 * cg + e;
-                            if (m >= g.m || n >= g.n) continue;
+                            if (m >= M || n >= g.n) continue;
                             const int32_t a = EPI == (int)Epi::Gelu ? (int32_t)gspan[acc[i][j][e]] : acc[i][j][e];
                             const int8_t v = (int8_t)byte_of(a);
                             if (EPI == (int)Epi::Act && g.kv_rows && n >= g.kv_d) {
@@ -769,7 +831,7 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
                             if (EPI == (int)Epi::Act) {
                                 ((int8_t *)g.out)[(size_t)m * g.ldo + n] = v;
                             } else {  // the operand of the next product, in panels
-                                const size_t orow = EPI == (int)Epi::GeluWide ? 2 * (size_t)m + pl : (size_t)m;
+                                const size_t orow = EPI == (int)Epi::GeluWide ? plane_row(m, pl) : (size_t)m;
                                 ((int8_t *)g.out)[panel_off(orow, n, g.out_rows)] = v;
                             }
                         }
@@ -796,7 +858,7 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
                 const int pc = q * 64 + lane, rl2 = pc / TJ, cl = (pc % TJ) * 16;
                 const v4i v = *(const v4i *)(wr + rl2 * RS8 + cl);
                 const int m = rw + rl2, n = cw + cl;
-                if (m >= g.m) continue;
+                if (m >= M) continue;
                 if (to_kv) {
                     // K or V of the row straight into the cache (kv_d, kv_hd multiples of 16);
                     // the columns past N = 3 kv_d are padding and go nowhere
@@ -813,7 +875,7 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
                              (((size_t)ri.slot * g.kv_h + hh) * g.kv_ctx + ri.pos) * g.kv_hd + cc) = v;
                     continue;
                 }
-                const size_t orow = EPI == (int)Epi::GeluWide ? 2 * (size_t)m + pl : (size_t)m;
+                const size_t orow = EPI == (int)Epi::GeluWide ? plane_row(m, pl) : (size_t)m;
                 // Gelu and GeluWide write the operand of the next product, in panels (16 columns
                 // from a multiple of 16 lie in one panel)
                 int8_t *o = (int8_t *)g.out + (EPI == (int)Epi::Act ? orow * g.ldo + n : panel_off(orow, n, g.out_rows));
@@ -828,77 +890,17 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
         }
         return;
     }
-    // The wide epilogues (no SWAP)
-    if constexpr (EPI == (int)Epi::ResidualWide || EPI == (int)Epi::LogitsWide || EPI == (int)Epi::LogitsCompactWide) {
-        static_assert(TI == 8 && TJ == 4, "the plane epilogues keep 128 x 64 wave tiles");
-        // i16 operand rows as planes (ops.rs:178-206,246-277): the lane holds plane rows
-        // 4 (lane / 16) + e of each 16-row tile, so e = 0, 1 are the hi and lo planes of one row
-        // and e = 2, 3 those of the next. dot(w, v) = 256 dot(w, hi) + dot(w, lo) + 128 wsum:
-        // |dot| <= K 2^22 <= 2^38, so dot + b is an i64 and rescale takes the i128 product.
-        const int tile_n0 = n0 + wn * 64;
-        int32_t mlt[4];
-        int64_t add[4];
-        bool okn[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int n = tile_n0 + j * 16 + (lane & 15);
-            okn[j] = n < g.n;
-            mlt[j] = okn[j] ? g.mult[n] : 0;
-            add[j] = okn[j] ? 128 * (int64_t)g.wsum[n] + (EPI == (int)Epi::ResidualWide ? g.bias[n] : 0) : 0;
-        }
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-#pragma unroll
-            for (int p = 0; p < 2; p++) {
-                const int mp = m0 + wm * 128 + i * 16 + (lane >> 4) * 4 + 2 * p;  // the hi plane row
-                const int m = mp >> 1;
-                const bool okm = mp < g.m;
-                int64_t l[4], mx = INT64_MIN;
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int64_t dot = 256 * (int64_t)acc[i][j][2 * p] + acc[i][j][2 * p + 1] + add[j];
-                    const i128 r = rescale_full(dot, mlt[j], g.shift);
-                    const int n = tile_n0 + j * 16 + (lane & 15);
-                    if (EPI == (int)Epi::ResidualWide) {  // x = clamp(x + r, +-R), as Residual
-                        if (okm && okn[j]) {
-                            int32_t *x = (int32_t *)g.out + (size_t)m * g.ldo + n;
-                            *x = (int32_t)clamp64((int64_t)*x + clamp128(r, INT32_MIN, INT32_MAX), -RES, RES);
-                        }
-                    } else if (EPI == (int)Epi::LogitsWide) {
-                        if (okm && okn[j]) ((int64_t *)g.out)[(size_t)m * g.ldo + n] = clamp128(r, -SCORE_LIMIT, SCORE_LIMIT);
-                    } else {
-                        l[j] = okn[j] ? clamp128(r, -SCORE_LIMIT, SCORE_LIMIT) : INT64_MIN;
-                        mx = l[j] > mx ? l[j] : mx;
-                    }
-                }
-                if (EPI == (int)Epi::LogitsCompactWide) {
-#pragma unroll
-                    for (int o = 1; o < 16; o <<= 1) {  // the 16 lanes that hold this row
-                        const int64_t u = __shfl_xor(mx, o, 64);
-                        mx = u > mx ? u : mx;
-                    }
-                    if (okm) {
-                        if ((lane & 15) == 0 && tile_n0 < g.n) g.tmax[(size_t)m * g.tmax_ld + tile_n0 / 64] = mx;
-#pragma unroll
-                        for (int j = 0; j < 4; j++) {
-                            if (!okn[j]) continue;
-                            const int64_t dd = mx - l[j];
-                            ((uint16_t *)g.out)[(size_t)m * g.ldo + tile_n0 + j * 16 + (lane & 15)] =
-                                (uint16_t)(dd < g.cap16 ? dd : g.cap16);
-                        }
-                    }
-                }
-            }
-        }
-        return;
-    }
 }
+
+// The largest span of an i16 GELU table that 256 x 256 tiles copy into LDS, in entries (beside 80 KiB of
+// staging regions).
+constexpr int GELU16_LDS = 40960;
 
 template <int EPI, bool NARROW, int BN, bool VEC, int BM = GEMM_BM, bool DEEP = false>
 static hipError_t launch_gemm_t(const GemmArgs &ga, hipStream_t stream) {
     constexpr int WAVES = gemm_waves(BN), FRAGS = BM / 16 + BN / 16;
     GemmArgs g = ga;
-    if (EPI == (int)Epi::Gelu && g.gelu_copy <= 0) {  // the whole table
+    if ((EPI == (int)Epi::Gelu || EPI == (int)Epi::GeluWide) && g.gelu_copy <= 0) {  // the whole table
         g.gelu_lo = 0;
         g.gelu_clo = -g.gelu_off;
         g.gelu_chi = g.gelu_off - 1;
@@ -913,9 +915,11 @@ static hipError_t launch_gemm_t(const GemmArgs &ga, hipStream_t stream) {
     constexpr size_t stages = BN == 256 ? (size_t)2 * (BM + BN) * 128 : (size_t)gemm_stages(BM, DEEP) * FRAGS * 1024;
     constexpr bool I8OUT = EPI == (int)Epi::Act || EPI == (int)Epi::Gelu || EPI == (int)Epi::GeluWide;
     constexpr size_t regions = (size_t)WAVES * (I8OUT ? 10240 : 18432);
-    // the largest request: the stages, or the 64 KiB GELU table and the staging regions after it
-    constexpr bool GELU_LDS = EPI == (int)Epi::Gelu && BM != 64;  // the 64 x 64 tiles read it from memory
-    constexpr size_t after_table = (GELU_LDS ? 65536 : 0) + regions;
+    // the largest request: the stages, or the GELU table (64 KiB of i8 entries, or the i16 span of
+    // 256 x 256 tiles) and the staging regions after it
+    constexpr bool TABLE16 = EPI == (int)Epi::GeluWide && BN == 256;
+    constexpr bool GELU_LDS = (EPI == (int)Epi::Gelu && BM != 64) || TABLE16;  // the 64 x 64 tiles read it from memory
+    constexpr size_t after_table = (TABLE16 ? (size_t)2 * GELU16_LDS : GELU_LDS ? 65536 : 0) + regions;
     constexpr size_t lds_max = stages > after_table ? stages : after_table;
     static_assert(lds_max <= 160 * 1024, "LDS of one workgroup");
     {
@@ -924,7 +928,7 @@ static hipError_t launch_gemm_t(const GemmArgs &ga, hipStream_t stream) {
     }
     size_t lds = stages > regions ? stages : regions;
     if (GELU_LDS && VEC) {
-        const size_t t = ((size_t)g.gelu_copy + 1023) & ~(size_t)1023;
+        const size_t t = ((size_t)(TABLE16 ? 2 : 1) * g.gelu_copy + 1023) & ~(size_t)1023;
         lds = stages > t + regions ? stages : t + regions;
     }
     launch_k((k_gemm<EPI, NARROW, BN, VEC, BM, DEEP>), dim3(gm * gn), dim3(64 * WAVES), lds, stream, g);
@@ -948,20 +952,17 @@ static bool gemm_small_tiles(int m, int n, int k_pad) {
 // path.
 template <int EPI, bool NARROW>
 static hipError_t launch_gemm_w(const GemmArgs &g, hipStream_t stream) {
-    constexpr bool WIDE = EPI == (int)Epi::ResidualWide || EPI == (int)Epi::LogitsWide ||
-                          EPI == (int)Epi::LogitsCompactWide;
-    if constexpr (WIDE) {
-        return launch_gemm_t<EPI, NARROW, 128, true>(g, stream);
-    } else {
-        constexpr size_t ES = EPI == (int)Epi::Residual || EPI == (int)Epi::Raw ? 4
-                              : EPI == (int)Epi::LogitsCompact ? 2
-                              : EPI == (int)Epi::Logits ? 8 : 1;
+    {
+        constexpr bool RESIDUAL = EPI == (int)Epi::Residual || EPI == (int)Epi::ResidualWide;
+        constexpr size_t ES = RESIDUAL || EPI == (int)Epi::Raw ? 4
+                              : EPI == (int)Epi::LogitsCompact || EPI == (int)Epi::LogitsCompactWide ? 2
+                              : EPI == (int)Epi::Logits || EPI == (int)Epi::LogitsWide ? 8 : 1;
         // (the GELU outputs are panels of 64-byte rows: aligned when the base is)
         constexpr bool PANEL_OUT = EPI == (int)Epi::Gelu || EPI == (int)Epi::GeluWide;
         const bool vec = ((uintptr_t)g.out & 15) == 0 && (PANEL_OUT || ((size_t)g.ldo * ES) % 16 == 0);
         if (!vec) return launch_gemm_t<EPI, NARROW, 128, false>(g, stream);
-        if constexpr (EPI == (int)Epi::Act || EPI == (int)Epi::Residual || EPI == (int)Epi::Gelu ||
-                      EPI == (int)Epi::GeluWide || EPI == (int)Epi::Raw) {
+        if constexpr (EPI == (int)Epi::Act || RESIDUAL || EPI == (int)Epi::Gelu || EPI == (int)Epi::GeluWide ||
+                      EPI == (int)Epi::Raw) {
             if (gemm_small_tiles(g.m, g.n, g.k_pad)) {
                 if (g.k_pad >= 1024) return launch_gemm_t<EPI, NARROW, 64, true, 64, true>(g, stream);
                 return launch_gemm_t<EPI, NARROW, 64, true, 64>(g, stream);
@@ -981,7 +982,14 @@ static hipError_t launch_gemm_w(const GemmArgs &g, hipStream_t stream) {
         const int gcopy = g.gelu_copy > 0 ? g.gelu_copy : 2 * g.gelu_off;
         const bool wide = g.n > 512 && (g.k_pad >= 2048 ||
                                         (EPI == (int)Epi::Gelu && g.n > 1024 && (gcopy > 32768 || g.k_pad >= 1536)));
-        if constexpr (EPI == (int)Epi::Act || EPI == (int)Epi::Residual) {
+        // The i16 GELU table, 2 bytes an entry, is gathered from LDS only in 256 x 256 tiles (its span takes
+        // most of what the staging leaves); through the caches the gathers took longer than the product
+        // (3,370 x 3,072 x 768: 37 us, 25 from LDS).
+        if constexpr (EPI == (int)Epi::GeluWide) {
+            if (gcopy <= GELU16_LDS) return launch_gemm_t<EPI, NARROW, 256, true>(g, stream);
+            return launch_gemm_t<EPI, NARROW, 128, true>(g, stream);
+        }
+        if constexpr (EPI == (int)Epi::Act || RESIDUAL) {
             // 128 x 192 tiles for a product that is one partial round of resident workgroups
             // (at most 512 of 256 x 128, or 256 of 256 x 256) and one round of 128 x 192: the
             // round then holds three quarters of the work per CU, spread over every CU
@@ -1001,8 +1009,10 @@ static hipError_t launch_gemm_w(const GemmArgs &g, hipStream_t stream) {
 
 template <int EPI>
 static hipError_t launch_gemm_e(const GemmArgs &g, hipStream_t stream) {
+    constexpr bool WIDE = EPI == (int)Epi::ResidualWide || EPI == (int)Epi::LogitsWide ||
+                          EPI == (int)Epi::LogitsCompactWide;
     const bool fast = EPI == (int)Epi::Logits || EPI == (int)Epi::LogitsCompact || g.fast32;
-    if (fast && g.shift >= 31) return launch_gemm_w<EPI, true>(g, stream);
+    if (fast && (WIDE || g.shift >= 31)) return launch_gemm_w<EPI, true>(g, stream);
     return launch_gemm_w<EPI, false>(g, stream);
 }
 
@@ -1099,8 +1109,13 @@ hipError_t launch_gemm(Epi epi, const GemmArgs &ga, hipStream_t stream) {
     if (g.a_rows == 0) g.a_rows = gm * GEMM_BM;
     if (g.w_rows == 0) g.w_rows = n_pad;
     if (g.a_rows < gm * GEMM_BM || g.w_rows < n_pad) return hipErrorInvalidValue;
-    if ((epi == Epi::Gelu && g.out_rows < g.m) || (epi == Epi::GeluWide && g.out_rows < 2 * g.m))
+    if ((epi == Epi::Gelu && g.out_rows < g.m) || (epi == Epi::GeluWide && g.out_rows < plane_rows(g.m)))
         return hipErrorInvalidValue;
+    // the wide epilogues: whole blocks of planes, their row sums, and a shift inside the bound of fast32
+    if (epi == Epi::ResidualWide || epi == Epi::LogitsWide || epi == Epi::LogitsCompactWide) {
+        if (!g.wsum || g.rows <= 0 || g.m != plane_rows(g.rows)) return hipErrorInvalidValue;
+        if (g.fast32 && (g.shift < 16 || g.shift > 62)) return hipErrorInvalidValue;
+    }
     g.kslice = 0;
     if (g.splits > 1) {
         const int sp = gemm_split_plan(g.k_pad, g.splits);
@@ -1122,10 +1137,9 @@ hipError_t launch_gemm(Epi epi, const GemmArgs &ga, hipStream_t stream) {
         case Epi::ResidualWide:
         case Epi::LogitsWide:
         case Epi::LogitsCompactWide:
-            if (!g.wsum || (g.m & 1)) return hipErrorInvalidValue;  // rows of plane pairs
-            if (epi == Epi::ResidualWide) return launch_gemm_w<7, false>(g, stream);
-            if (epi == Epi::LogitsWide) return launch_gemm_w<8, false>(g, stream);
-            return launch_gemm_w<9, false>(g, stream);
+            if (epi == Epi::ResidualWide) return launch_gemm_e<7>(g, stream);
+            if (epi == Epi::LogitsWide) return launch_gemm_e<8>(g, stream);
+            return launch_gemm_e<9>(g, stream);
     }
     return hipErrorInvalidValue;
 }
@@ -1360,8 +1374,7 @@ __global__ __launch_bounds__(256) void k_layernorm(LnArgs a, int n_rows) {
     const bool small = (u128)cmax * inv < ((u128)1 << 63);
     const bool wide = a.bits == 16;
     // the operand rows of this row (two planes when wide), in panels (panel_off)
-    const size_t orow = (size_t)row * (wide ? 2 : 1);
-    auto at = [&](int pl, int j) { return a.out + panel_off(orow + pl, j, a.out_rows); };
+    auto at = [&](int pl, int j) { return a.out + panel_off(wide ? plane_row(row, pl) : (size_t)row, j, a.out_rows); };
     // clamp_act_i8, or clamp_act_i16 stored as the planes hi = v >> 8, lo = (v & 255) - 128
     auto put = [&](int j, int64_t y) {
         if (!wide) {
@@ -1446,8 +1459,7 @@ __global__ __launch_bounds__(256) void k_layernorm_rows(LnArgs a, int n_rows) {
     const bool fast = small && a.beta_frac == 0 && a.s >= 64 && a.s <= 126;
     const bool wide = a.bits == 16;
     // the operand rows of this row (two planes when wide), in panels (panel_off)
-    const size_t orow = (size_t)row * (wide ? 2 : 1);
-    auto at = [&](int pl, int j) { return a.out + panel_off(orow + pl, j, a.out_rows); };
+    auto at = [&](int pl, int j) { return a.out + panel_off(wide ? plane_row(row, pl) : (size_t)row, j, a.out_rows); };
     // Each element first takes the double-precision form of the rule (ln_elem_f64), which gives
     // the exact integer or declines; a declined element takes the integer rule below.
     const bool fpath = a.beta_frac == 0 && a.s <= 126;
@@ -1614,8 +1626,9 @@ __global__ __launch_bounds__(64 * LN_WAVES) void k_layernorm_rows4(LnArgs a, int
     const bool small = flags & 1, fast = (flags >> 1) & 1;
     // the operand rows of this row (two planes when wide), in panels (panel_off); a wave's four
     // rows are adjacent in every panel, so each store instruction writes 256 contiguous bytes
-    const size_t orow = (size_t)row * (wide ? 2 : 1);
-    auto at = [&](int pl, int j) { return (uint32_t *)(a.out + panel_off(orow + pl, j, a.out_rows)); };
+    auto at = [&](int pl, int j) {
+        return (uint32_t *)(a.out + panel_off(wide ? plane_row(row, pl) : (size_t)row, j, a.out_rows));
+    };
     // Each element first takes the double-precision form of the rule (ln_elem_f64), which gives
     // the exact integer or declines. Every group is stored from it; the groups with a declined
     // element are then recomputed by the integer rule and stored again (the same lane rewrites
@@ -4502,8 +4515,9 @@ int kernel_resources(KernelResource *out, int cap) {
         {"k_gemm<Act, 256x128>", (const void *)k_gemm<1, false, 128, true>},
         {"k_gemm<Residual, 256x128>", (const void *)k_gemm<2, false, 128, true>},
         {"k_gemm<GeluWide, 256x128>", (const void *)k_gemm<6, false, 128, true>},
-        {"k_gemm<ResidualWide, 256x128>", (const void *)k_gemm<7, false, 128, true>},
-        {"k_gemm<LogitsCompactWide, 256x128>", (const void *)k_gemm<9, false, 128, true>},
+        {"k_gemm<GeluWide, narrow, 256x256>", (const void *)k_gemm<6, true, 256, true>},
+        {"k_gemm<ResidualWide, narrow, 256x256>", (const void *)k_gemm<7, true, 256, true>},
+        {"k_gemm<LogitsCompactWide, narrow, 256x128>", (const void *)k_gemm<9, true, 128, true>},
         {"k_gemm<Raw, split-K partials, 64x64>", (const void *)k_gemm<0, false, 64, true, 64>},
         {"k_gemm<Act, narrow, 128x192>", (const void *)k_gemm<1, true, 192, true, 128>},
         {"k_gemm<Residual, narrow, 128x192>", (const void *)k_gemm<2, true, 192, true, 128>},

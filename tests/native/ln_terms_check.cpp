@@ -101,6 +101,21 @@ int main() {
         std::printf("ln_elem_z declined too often\n");
         return 1;
     }
+    // rescale_wide47 against the i128 rule: |v| < 2^47, shifts 16 .. 62, on and beside rounding steps
+    for (int i = 0; i < 1000000; i++) {
+        const uint32_t s = 16 + (uint32_t)(next() % 47);
+        int64_t v = (int64_t)(next() >> (17 + next() % 46));
+        int32_t m = (int32_t)(uint32_t)next();
+        if (i % 16 == 0) v = (1ll << 47) - 1;
+        if (i % 16 == 1) m = INT32_MIN;
+        if (i % 16 == 2) m = 1, v = ((1ll << (s < 47 ? s : 46)) >> 1) + (int64_t)(next() % 3) - 1;
+        if (next() & 1) v = -v;
+        if ((i128)hs::rescale_wide47(v, m, s) != hs::rescale_full(v, m, s)) {
+            std::printf("rescale_wide47 v %lld m %d s %u\n", (long long)v, m, s);
+            return 1;
+        }
+        count++;
+    }
     std::printf("ok %ld (terms %ld, elements %ld of %ld)\n", count, taken, kept, elems);
     return 0;
 }
