@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <cstring>
 #include <memory>
 #include <mutex>
@@ -1241,8 +1242,12 @@ hs_status run_pass(hs_batch &b, const std::vector<PassRow> &rows, Out out, const
     const uint64_t *res = out == Out::Intervals ? b.h_intervals : host.data();
     // The event times are read back in bulk (hs_batch_profile), not inside every call.
     if (b.profiling && b.pending.size() > 8192) HIP_TRY(b.collect());
-    for (int i = 0; i < n_out; i++)
-        std::memcpy(sink + (size_t)owner[i] * per_row, res + (size_t)i * per_row, per_row * 8);
+    for (int i = 0; i < n_out;) {  // runs of consecutive inputs go in one copy
+        int e = i + 1;
+        while (e < n_out && owner[e] == owner[e - 1] + 1) e++;
+        std::memcpy(sink + (size_t)owner[i] * per_row, res + (size_t)i * per_row, (size_t)(e - i) * per_row * 8);
+        i = e;
+    }
     if (mx && mx->plain_sink)
         for (int i = 0; i < n_out; i++)
             std::memcpy(mx->plain_sink + (size_t)owner[i] * 3, b.h_intervals2 + (size_t)i * 3, 24);
@@ -1296,19 +1301,17 @@ extern "C" hs_status hs_batch_run_weights(hs_batch *b, const hs_input *in, size_
 
 namespace {
 
-// coder_words (batch.rs:647-666): the query words, each checked against the vocabulary and
-// the total 2^freq_bits.
-hs_status coder_words(const hs_query *queries, size_t n, uint32_t V, uint32_t freq_bits,
-                      std::vector<uint32_t> &words) {
+// coder_words (batch.rs:647-666): each query checked against the vocabulary and the total
+// 2^freq_bits. An hs_query is the kernels' pair of words as it is.
+static_assert(sizeof(hs_query) == 8 && offsetof(hs_query, value) == 4, "queries are read as (kind, value) words");
+const uint32_t *query_words(const hs_query *queries) { return queries ? &queries->kind : nullptr; }
+hs_status check_queries(const hs_query *queries, size_t n, uint32_t V, uint32_t freq_bits) {
     if (freq_bits == 0 || freq_bits > 32 || (uint64_t)V > (1ull << freq_bits))
         return hs::fail(HS_UNSUPPORTED, 0, "freq_bits must be in 1..=32 and 2^freq_bits >= vocab");
-    words.resize(2 * n);
     for (size_t i = 0; i < n; i++) {
         const bool ok = (queries[i].kind == 0 && queries[i].value < V) ||
                         (queries[i].kind == 1 && (uint64_t)queries[i].value < (1ull << freq_bits));
         if (!ok) return hs::fail(HS_UNSUPPORTED, 0, "a coder token or target is out of range");
-        words[2 * i] = queries[i].kind;
-        words[2 * i + 1] = queries[i].value;
     }
     return HS_OK;
 }
@@ -1337,9 +1340,8 @@ extern "C" hs_status hs_batch_run_coded(hs_batch *b, const hs_input *in, const h
     hs_status s = check_inputs(b, in, n);
     if (s != HS_OK) return s;
     if (n && (!queries || !out)) return hs::fail(HS_INVALID_ARGUMENT, 0, "NULL argument");
-    static thread_local std::vector<uint32_t> words;
-    HS_TRY(coder_words(queries, n, b->model->host.vocab, freq_bits, words));
-    return run(b, in, n, Out::Intervals, words.data(), freq_bits, (uint64_t *)out);
+    HS_TRY(check_queries(queries, n, b->model->host.vocab, freq_bits));
+    return run(b, in, n, Out::Intervals, query_words(queries), freq_bits, (uint64_t *)out);
 }
 
 extern "C" hs_status hs_batch_run_coded_mixed(hs_batch *b, const hs_input *in, const hs_query *queries,
@@ -1349,13 +1351,12 @@ extern "C" hs_status hs_batch_run_coded_mixed(hs_batch *b, const hs_input *in, c
     HS_TRY(check_inputs(b, in, n));
     if (n && (!queries || !tables || !out)) return hs::fail(HS_INVALID_ARGUMENT, 0, "NULL argument");
     const uint32_t V = b->model->host.vocab;
-    std::vector<uint32_t> words;
-    HS_TRY(coder_words(queries, n, V, freq_bits, words));
+    HS_TRY(check_queries(queries, n, V, freq_bits));
     HS_TRY(check_tables(tables, n, V, true));
     if (!mixer && needs_mixer(tables, n)) return hs::fail(HS_INVALID_ARGUMENT, 0, "mixer is NULL");
     Mixing mx;
     mx.tables = tables; mx.fn = mixer; mx.user = user;
-    return run(b, in, n, Out::Intervals, words.data(), freq_bits, (uint64_t *)out, &mx);
+    return run(b, in, n, Out::Intervals, query_words(queries), freq_bits, (uint64_t *)out, &mx);
 }
 
 extern "C" hs_status hs_batch_run_coded_dual(hs_batch *b, const hs_input *in, const uint32_t *tokens,
@@ -1368,13 +1369,12 @@ extern "C" hs_status hs_batch_run_coded_dual(hs_batch *b, const hs_input *in, co
     const uint32_t V = b->model->host.vocab;
     std::vector<hs_query> queries(n);
     for (size_t i = 0; i < n; i++) queries[i] = hs_query{0, tokens[i]};
-    std::vector<uint32_t> words;
-    HS_TRY(coder_words(queries.data(), n, V, freq_bits, words));
+    HS_TRY(check_queries(queries.data(), n, V, freq_bits));
     HS_TRY(check_tables(predictions, n, V, false));
     if (!mixer && needs_mixer(predictions, n)) return hs::fail(HS_INVALID_ARGUMENT, 0, "mixer is NULL");
     Mixing mx;
     mx.tables = predictions; mx.fn = mixer; mx.user = user; mx.plain_sink = (uint64_t *)plain;
-    return run(b, in, n, Out::Intervals, words.data(), freq_bits, (uint64_t *)mixed, &mx);
+    return run(b, in, n, Out::Intervals, query_words(queries.data()), freq_bits, (uint64_t *)mixed, &mx);
 }
 
 extern "C" hs_status hs_batch_step(hs_batch *b, const hs_input *in, size_t n) {
@@ -1920,8 +1920,7 @@ extern "C" hs_status hs_op_mixed_coder(hs_device *dev, const uint64_t *weights, 
         return hs::fail(HS_INVALID_ARGUMENT, 0, "NULL argument");
     if (rows == 0) return HS_OK;
     if (vocab == 0 || vocab > (1u << 30)) return hs::fail(HS_UNSUPPORTED, 0, "the vocabulary is too large");
-    std::vector<uint32_t> q;
-    HS_TRY(coder_words(queries, rows, (uint32_t)vocab, freq_bits, q));
+    HS_TRY(check_queries(queries, rows, (uint32_t)vocab, freq_bits));
     HS_TRY(check_tables(predictions, rows, (uint32_t)vocab, false));
     if (!mixer && needs_mixer(predictions, rows)) return hs::fail(HS_INVALID_ARGUMENT, 0, "mixer is NULL");
     for (size_t r = 0; r < rows; r++) {  // each row's sum below 2^64
@@ -1938,7 +1937,7 @@ extern "C" hs_status hs_op_mixed_coder(hs_device *dev, const uint64_t *weights, 
     std::vector<hs::MixRec> rec(rows);
     for (size_t r = 0; r < rows; r++) rec[r] = hs::MixRec{predictions[r], 0, 0, 0, 0, 0};
     HS_TRY(mem.upload(dw, weights, rows * vocab));
-    HS_TRY(mem.upload(dq, q.data(), q.size()));
+    HS_TRY(mem.upload(dq, query_words(queries), 2 * rows));
     HS_TRY(mem.upload(dm, rec.data(), rows));
     HS_TRY(mem.alloc(dst, 3 * rows));
     HS_TRY(mem.alloc(di, 3 * rows));
@@ -1982,8 +1981,7 @@ hs_status coder_on_logits(hs_device *dev, const int64_t *logits, size_t rows, si
         return hs::fail(HS_UNSUPPORTED, 0, "the table must start in 1..=2^40");
     for (size_t i = 1; i < len; i++)
         if (table[i] > table[i - 1]) return hs::fail(HS_UNSUPPORTED, 0, "the table must be non-increasing");
-    std::vector<uint32_t> q;
-    HS_TRY(coder_words(queries, rows, (uint32_t)vocab, freq_bits, q));
+    HS_TRY(check_queries(queries, rows, (uint32_t)vocab, freq_bits));
     if (predictions) {
         HS_TRY(check_tables(predictions, rows, (uint32_t)vocab, true));
         if (!mixer && needs_mixer(predictions, rows)) return hs::fail(HS_INVALID_ARGUMENT, 0, "mixer is NULL");
@@ -1996,7 +1994,7 @@ hs_status coder_on_logits(hs_device *dev, const int64_t *logits, size_t rows, si
     std::vector<hs::MixRec> rec(predictions ? rows : 0);
     for (size_t r = 0; r < rec.size(); r++) rec[r] = hs::MixRec{predictions[r], 0, 0, 0, 0, 0};
     HS_TRY(mem.upload(dt, table, len, std::max<size_t>(len, hs::CODER_TABLE_READ)));  // as the model's
-    HS_TRY(mem.upload(dq, q.data(), q.size()));
+    HS_TRY(mem.upload(dq, query_words(queries), 2 * rows));
     HS_TRY(mem.alloc(di, 3 * rows));
     if (predictions) {
         HS_TRY(mem.upload(dm, rec.data(), rows));

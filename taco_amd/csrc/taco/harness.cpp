@@ -276,20 +276,26 @@ extern "C" hs_status tc_fold_blocks(hs_batch *batch, uint32_t overlap, const uin
         }
     }
     // Host scratch kept from call to call on this thread (fresh vectors of a fold step's 16k
-    // rows would touch new pages of memory on every call). The names below are references to
-    // the calling thread's instances, so the range-coder tasks on the pool's threads (which
-    // capture them) see this call's rows.
+    // rows would touch new pages of memory on every call), filled through plain pointers: three
+    // push_backs a row took 300 us of a 16,384-row fold, this takes 20. The names below are
+    // references to the calling thread's instances, so the range-coder tasks on the pool's
+    // threads (which capture them) see this call's rows.
+    struct Run {  // the coded rows [begin, end) of a window of a block
+        size_t block, begin, end;
+    };
     struct Scratch {
         std::vector<hs_input> inputs;
         std::vector<hs_query> queries;
-        std::vector<int64_t> owner;
         std::vector<hs_interval> answers;
+        std::vector<Run> runs;
+        std::vector<size_t> tasks;  // the first run of each block of the wave
     };
     static thread_local Scratch scratch;
     std::vector<hs_input> &inputs = scratch.inputs;
     std::vector<hs_query> &queries = scratch.queries;
-    std::vector<int64_t> &owner = scratch.owner;  // the block of each coded row, -1 for a row that codes nothing
     std::vector<hs_interval> &answers = scratch.answers;
+    std::vector<Run> &runs = scratch.runs;
+    std::vector<size_t> &tasks = scratch.tasks;
     {
         size_t most = 0;  // rows of the largest wave of windows
         for (size_t w0 = 0; w0 < windows.size(); w0 += slots) {
@@ -297,64 +303,60 @@ extern "C" hs_status tc_fold_blocks(hs_batch *batch, uint32_t overlap, const uin
             for (size_t wi = w0; wi < std::min(windows.size(), w0 + slots); wi++) r += windows[wi].len + k + 1;
             most = std::max(most, r);
         }
-        inputs.reserve(most);
-        queries.reserve(most);
-        owner.reserve(most);
-        answers.reserve(most);
+        if (inputs.size() < most) {  // the vectors only grow: rows past a wave's count are not read
+            inputs.resize(most);
+            queries.resize(most);
+            answers.resize(most);
+        }
     }
     for (size_t w0 = 0; w0 < windows.size(); w0 += slots) {
         const size_t w1 = std::min(windows.size(), w0 + slots);
-        inputs.clear();
-        queries.clear();
-        owner.clear();
+        runs.clear();
+        tasks.clear();
+        size_t n = 0;  // rows of this wave
+        hs_input *in = inputs.data();
+        hs_query *qs = queries.data();
         for (size_t wi = w0; wi < w1; wi++) {
             const Window &w = windows[wi];
             if (enc[w.block].stopped()) continue;
             const uint32_t slot = (uint32_t)(wi - w0);
             hs_batch_reset(batch, slot);
             const uint32_t *t = tokens + offsets[w.block];
-            // Window::rows (gpu_fold.rs:145-160)
-            auto row = [&](uint32_t in, int64_t code) {
-                inputs.push_back(hs_input{slot, in});
-                queries.push_back(hs_query{0, code >= 0 ? (uint32_t)code : eot});
-                owner.push_back(code >= 0 ? (int64_t)w.block : -1);
+            // Window::rows (gpu_fold.rs:145-160); a row that codes nothing queries EOT
+            auto row = [&](uint32_t token, uint32_t code) {
+                in[n] = hs_input{slot, token};
+                qs[n++] = hs_query{0, code};
             };
-            if (w.first == 0) {
-                row(eot, t[0]);
-            } else {
-                row(eot, -1);
+            if (w.first > 0) {
+                row(eot, eot);
                 const size_t kept0 = w.first >= 1 + k ? w.first - 1 - k : 0;
-                for (size_t i = kept0; i < w.first - 1; i++) row(t[i], -1);
-                row(t[w.first - 1], t[w.first]);
+                for (size_t i = kept0; i < w.first - 1; i++) row(t[i], eot);
             }
+            const size_t begin = n;
+            row(w.first > 0 ? t[w.first - 1] : eot, t[w.first]);
             for (size_t i = w.first + 1; i < w.first + w.len; i++) row(t[i - 1], t[i]);
+            if (runs.empty() || runs.back().block != w.block) tasks.push_back(runs.size());
+            runs.push_back(Run{w.block, begin, n});
         }
-        if (inputs.empty()) continue;
-        answers.resize(inputs.size());
-        hs_status s = hs_batch_run_coded(batch, inputs.data(), queries.data(), inputs.size(),
-                                         TC_FREQ_BITS, answers.data());
+        if (n == 0) continue;
+        hs_status s = hs_batch_run_coded(batch, inputs.data(), queries.data(), n, TC_FREQ_BITS, answers.data());
         if (s != HS_OK) return s;
-        // The rows are in window order: the rows of a block in this wave are one run, so each
+        // The rows are in window order: the windows of a block in this wave are adjacent runs, so each
         // block's tokens reach its encoder in order, and the blocks' coders run in parallel.
-        std::vector<std::pair<size_t, size_t>> runs;  // [begin, end) of each block's coded rows
-        for (size_t i = 0; i < inputs.size(); i++) {
-            if (owner[i] < 0) continue;
-            if (runs.empty() || (size_t)owner[runs.back().first] != (size_t)owner[i]) runs.push_back({i, i});
-            runs.back().second = i + 1;
-        }
         std::atomic<bool> bad(false);
-        Pool::get().run(runs.size(), [&](size_t r) {
-            BlockEnc &be = enc[(size_t)owner[runs[r].first]];
-            for (size_t i = runs[r].first; i < runs[r].second; i++) {
-                if (owner[i] < 0) continue;
-                const hs_interval &a = answers[i];
-                // lanes.rs:121-128: a bad interval or last-symbol flag is a fault of the device
-                if (a.freq == 0 || a.start > TOTAL || a.freq > TOTAL - a.start || a.symbol != queries[i].value) {
-                    bad = true;
-                    return;
+        Pool::get().run(tasks.size(), [&](size_t task) {
+            const size_t r0 = tasks[task], r1 = task + 1 < tasks.size() ? tasks[task + 1] : runs.size();
+            BlockEnc &be = enc[runs[r0].block];
+            for (size_t r = r0; r < r1; r++)
+                for (size_t i = runs[r].begin; i < runs[r].end; i++) {
+                    const hs_interval &a = answers[i];
+                    // lanes.rs:121-128: a bad interval or last-symbol flag is a fault of the device
+                    if (a.freq == 0 || a.start > TOTAL || a.freq > TOTAL - a.start || a.symbol != queries[i].value) {
+                        bad = true;
+                        return;
+                    }
+                    be.push(a.start, a.freq);
                 }
-                be.push(a.start, a.freq);
-            }
         });
         if (bad) return hs::fail(HS_DEVICE_ERROR, 0, "the coder op gave a bad interval");
     }
