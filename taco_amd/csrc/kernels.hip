@@ -2060,6 +2060,63 @@ __global__ void k_split_out(AttnArgs a, int n_rows, SplitPlan pl, void *scratch)
     *attn_out(a, r, h * hd + t) = (int8_t)clamp128(rescale_full(o, a.out_m, a.out_s), -127, 127);
 }
 
+// ---- The pieces of the one-launch decode kernels (head_dim 64) ------------------------------------
+// Sum p v of one query row is a product of a 64-channel x 64-key matrix with p, and p is four
+// balanced i8 digits (the bytes of p + 0x80808080, xor 0x80): one v_mfma_i32_16x16x64_i8 takes 16
+// channels x 64 keys against the four digit planes as four of its columns (the other twelve
+// repeat them), so a block of 64 keys is 4 MFMAs where 24-bit multiplies took 192 VALU
+// instructions a wave, and the sums need no butterfly over the lanes.
+// A block's V rows lie in LDS as dense 64-byte rows, 16-byte chunk c of row r at slot
+// 4 r + (c ^ vsw(r)); the V^T operand comes by transposing reads (as in k_attend_short), whose
+// operand byte 4 t + e of lane group g holds key 16 t + 4 g + e. `mem` is 1 KiB of the wave.
+__device__ __forceinline__ int vsw(int r) { return ((r >> 1) ^ (r >> 3)) & 3; }
+
+__device__ __forceinline__ void decode_pv_block(const int8_t *sv, int8_t *mem, uint32_t p, int lane, v4i (&acc)[4]) {
+    // the digits of this lane's key to [plane][key in operand order]
+    const uint32_t q = (p + 0x80808080u) ^ 0x80808080u;
+    int8_t *w = mem + 16 * ((lane >> 2) & 3) + 4 * (lane >> 4) + (lane & 3);
+#pragma unroll
+    for (int k = 0; k < 4; k++) w[64 * k] = (int8_t)(q >> (8 * k));
+    const v4i pf = *(const v4i *)(mem + 64 * (lane & 3) + 16 * (lane >> 4));
+    const int ql = lane & 15, qg = lane >> 4;
+    const int tr_k = ql >> 1, tr_h = ql & 1;
+    const int key0 = 16 * (tr_k >> 2) + 4 * qg + (tr_k & 3);
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        const int8_t *p0 = sv + (4 * key0 + (c ^ vsw(key0 & 15))) * 16 + 8 * tr_h;
+        const v2i r0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)p0);
+        const v2i r1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(p0 + 32 * 64));
+        acc[c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(v4i{r0[0], r0[1], r1[0], r1[1]}, pf, acc[c], 0, 0, 0);
+    }
+}
+
+// acc[c][e] of lane l holds channel 16 c + 4 (l / 16) + e of plane l % 16 (< 4): to [plane][64] in mem.
+__device__ __forceinline__ void decode_pv_store(int8_t *mem, int lane, const v4i (&acc)[4]) {
+    if ((lane & 15) < 4) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) *(v4i *)(mem + 256 * (lane & 15) + 64 * c + 16 * (lane >> 4)) = acc[c];
+    }
+}
+// The planes' sum of channel ch: below 2^24 per plane, |sum| <= 1,024 2^30 2^7 < 2^53.
+__device__ __forceinline__ int64_t decode_pv_sum(const int8_t *mem, int ch) {
+    const int32_t *m = (const int32_t *)mem + ch;
+    return (int64_t)m[0] + (int64_t)m[64] * 256 + (int64_t)m[128] * 65536 + (int64_t)m[192] * 16777216;
+}
+
+// The extreme values over the wave.
+__device__ __forceinline__ void wave_min_max(int32_t &mn, int32_t &mx) {
+    butterfly<64>([&](auto st) {
+        constexpr int S = decltype(st)::value;
+        const int32_t u = lane_move<S>(mn), v = lane_move<S>(mx);
+        mn = u < mn ? u : mn;
+        mx = v > mx ? v : mx;
+    });
+}
+__device__ __forceinline__ uint64_t wave_sum_dpp(uint64_t v) {
+    butterfly<64>([&](auto st) { v += (uint64_t)lane_move64<decltype(st)::value>((int64_t)v); });
+    return v;
+}
+
 // Decode attention for head_dim 64 and at most 1,024 keys in one launch: one workgroup (4 waves)
 // per (row, head). The row's K rows (thread t: keys t + 256 j) and V rows (in the layout the p v
 // sums read them: thread t, keys t / 4 + 64 i, chunk t % 4) go to registers in one round of
@@ -2073,16 +2130,14 @@ __global__ void k_split_out(AttnArgs a, int n_rows, SplitPlan pl, void *scratch)
 template <bool NOCLAMP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_attend_decode64(AttnArgs a,
                                                                                                   int kmax) {
-    extern __shared__ __attribute__((aligned(16))) int8_t s_dyn[];
+    __shared__ __attribute__((aligned(16))) int8_t s_v[4][4096];    // a wave's block of V rows
+    __shared__ __attribute__((aligned(16))) int8_t s_mem[4][1024];  // a wave's digits, then its plane sums
     __shared__ int32_t s_mm[2][4];
     __shared__ uint64_t s_sum[4];
-    __shared__ int64_t s_acc[4][64];
     const int rh = blockIdx.x, tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
     const int r = rh / a.n_head, h = rh - r * a.n_head;
-    const int kmax64 = (kmax + 63) & ~63;
     int keys = split_keys(a, r);
     keys = keys < kmax ? keys : kmax;  // the launch's bound holds every row's count
-    uint32_t *s_p = (uint32_t *)s_dyn;
     const size_t base = ((size_t)split_slot(a, r) * a.n_head + h) * a.ctx_cap * 64;
     // q straight into every thread's registers (one 64-byte row, the same for all)
     int qv[16];
@@ -2102,13 +2157,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
         for (int t = 0; t < 4; t++) kk[j][t] = k16[t];
     }
-    // V after K (keys past the row reload the row's last key; their weight is 0)
-    constexpr int VR = 1024 / 64;
-    v4i vr[VR];
+    // V after K: the rows of this wave's four blocks of 64 keys, 64 (4 j + w) .. (the keys whose p its
+    // lanes form), lane l the chunk (l % 4) ^ vsw of row 16 u + l / 4 (keys past the row reload the
+    // row's last key; their weight is 0)
+    v4i vr[16];
 #pragma unroll
-    for (int i = 0; i < VR; i++) {
-        const int k = (tid >> 2) + 64 * i;
-        vr[i] = *(const v4i *)(a.vc + base + (size_t)(k < keys ? k : keys - 1) * 64 + 16 * (tid & 3));
+    for (int i = 0; i < 16; i++) {
+        const int row = 16 * (i & 3) + (lane >> 2), k = 64 * (4 * (i >> 2) + w) + row;
+        vr[i] = *(const v4i *)(a.vc + base + (size_t)(k < keys ? k : keys - 1) * 64 + 16 * ((lane & 3) ^ vsw(row & 15)));
     }
     __builtin_amdgcn_sched_barrier(0);  // every load issued before the first wait
     // the dots wait for K alone (the compiler's waits on the K registers)
@@ -2130,12 +2186,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             dmax = x > dmax ? x : dmax;
         }
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const int32_t u = __shfl_xor(dmin, o, 64), v = __shfl_xor(dmax, o, 64);
-        dmin = u < dmin ? u : dmin;
-        dmax = v > dmax ? v : dmax;
-    }
+    wave_min_max(dmin, dmax);
     if (lane == 0) {
         s_mm[0][w] = dmin;
         s_mm[1][w] = dmax;
@@ -2164,63 +2215,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             sum += e[j];
         }
     }
-    sum = (uint64_t)wave_sum64((int64_t)sum);
+    sum = wave_sum_dpp(sum);
     if (lane == 0) s_sum[w] = sum;
     __syncthreads();
     sum = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
     const double R = ldexp(1.0 / (double)sum, a.softmax_p);
     const double sp = softmax_sp(sum, a.softmax_p);
+    v4i acc[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) acc[c] = v4i{0, 0, 0, 0};
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        const int k = tid + 256 * j;
-        if (k < keys) s_p[k] = softmax_p_of(e[j], R, sp);
+        if (64 * (4 * j + w) >= keys) break;  // uniform
+#pragma unroll
+        for (int u = 0; u < 4; u++) *(v4i *)(s_v[w] + 1024 * u + 16 * lane) = vr[4 * j + u];
+        // p <= 2^P <= 2^30; 0 for keys past the row (e = 0)
+        decode_pv_block(s_v[w], s_mem[w], softmax_p_of(e[j], R, sp), lane, acc);
     }
+    decode_pv_store(s_mem[w], lane, acc);
     __syncthreads();
-    // sum p v: thread t takes channels 16 (t % 4) .. +16 of keys t / 4 + 64 i. p = 2^16 ph + pl
-    // with pl, ph < 2^16 and |v| <= 128: at most 16 keys per thread keep the i32 sums of both
-    // halves below 2^27, exact (24-bit multiplies)
-    const int g = tid & 3;
-    int32_t lo[16], hi[16];
-#pragma unroll
-    for (int i = 0; i < 16; i++) lo[i] = hi[i] = 0;
-    auto pv = [&](int k, const v4i raw) {
-        const uint32_t p = s_p[k];
-        const int32_t pl = (int32_t)(p & 0xffffu), ph = (int32_t)(p >> 16);
-        const int8_t *v = (const int8_t *)&raw;
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            lo[i] += pl * (int32_t)v[i];
-            hi[i] += ph * (int32_t)v[i];
-        }
-    };
-#pragma unroll
-    for (int i = 0; i < VR; i++) {
-        const int k = (tid >> 2) + 64 * i;
-        if (k < keys) pv(k, vr[i]);
-    }
-    // Per wave, a butterfly over the 16 lanes of a channel group (lane bits 2..5) halves the
-    // channels a lane keeps in each round, so lane l ends with the wave's sum of one channel,
-    // 16 (l % 4) + 8 b2 + 4 b3 + 2 b4 + b5. lo and hi stay i32: a wave's 256 keys keep
-    // |sum pl v| <= 256 (2^16 - 1) 128 < 2^31 and |sum ph v| <= 256 2^14 128.
-    auto halve = [&](auto n, int o) {  // n channels -> n / 2
-        const bool up = (lane & o) != 0;
-#pragma unroll
-        for (int c = 0; c < n / 2; c++) {
-            const int32_t lk = up ? lo[n / 2 + c] : lo[c], ls = up ? lo[c] : lo[n / 2 + c];
-            const int32_t hk = up ? hi[n / 2 + c] : hi[c], hs = up ? hi[c] : hi[n / 2 + c];
-            lo[c] = lk + __shfl_xor(ls, o, 64);
-            hi[c] = hk + __shfl_xor(hs, o, 64);
-        }
-    };
-    halve(std::integral_constant<int, 16>{}, 4);
-    halve(std::integral_constant<int, 8>{}, 8);
-    halve(std::integral_constant<int, 4>{}, 16);
-    halve(std::integral_constant<int, 2>{}, 32);
-    s_acc[w][16 * (lane & 3) + ((lane >> 2) & 1) * 8 + ((lane >> 3) & 1) * 4 + ((lane >> 4) & 1) * 2 + ((lane >> 5) & 1)] =
-        (int64_t)hi[0] * 65536 + lo[0];
-    __syncthreads();
-    if (tid < 64) {  // |o| <= 1,024 2^30 2^7 < 2^53
-        const int64_t o = s_acc[0][tid] + s_acc[1][tid] + s_acc[2][tid] + s_acc[3][tid];
+    if (tid < 64) {
+        const int64_t o = decode_pv_sum(s_mem[0], tid) + decode_pv_sum(s_mem[1], tid) +
+                          decode_pv_sum(s_mem[2], tid) + decode_pv_sum(s_mem[3], tid);
         const double mo = a.out_s > 95 ? 0.0 : ldexp((double)a.out_m, -a.out_s);
         *attn_out(a, r, h * 64 + tid) = (int8_t)attn_out_byte(o, mo, a.out_m, a.out_s);
     }
@@ -2250,8 +2266,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     int qv[16];
 #pragma unroll
     for (int t = 0; t < 16; t++) qv[t] = ((const int *)(a.q + (size_t)r * a.ldq + h * 64))[t];
-    extern __shared__ __attribute__((aligned(16))) int8_t s_v[];  // 4 waves x KB x 4 KiB
-    int8_t *sv = s_v + (threadIdx.x >> 6) * (KB * 4096);
+    extern __shared__ __attribute__((aligned(16))) int8_t s_v[];  // 4 waves x (KB x 4 KiB of V rows, 1 KiB)
+    int8_t *sv = s_v + (threadIdx.x >> 6) * (KB * 4096 + 1024), *mem = sv + KB * 4096;
     v4i kk[KB][4];
 #pragma unroll
     for (int j = 0; j < KB; j++) {
@@ -2264,8 +2280,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
     for (int i = 0; i < 4 * KB; i++) {
         if (16 * i >= keys) break;
-        const int k = (lane >> 2) + 16 * i;
-        __builtin_amdgcn_global_load_lds((const void *)(a.vc + base + (size_t)(k < keys ? k : keys - 1) * 64 + 16 * (lane & 3)),
+        const int k = (lane >> 2) + 16 * i, c = (lane & 3) ^ vsw(lane >> 2);
+        __builtin_amdgcn_global_load_lds((const void *)(a.vc + base + (size_t)(k < keys ? k : keys - 1) * 64 + 16 * c),
                                          (lds_void *)(sv + i * 1024), 16, 0, 0);
     }
     int32_t d[KB];
@@ -2288,12 +2304,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             dmax = x > dmax ? x : dmax;
         }
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const int32_t u = __shfl_xor(dmin, o, 64), v = __shfl_xor(dmax, o, 64);
-        dmin = u < dmin ? u : dmin;
-        dmax = v > dmax ? v : dmax;
-    }
+    wave_min_max(dmin, dmax);
     // the row max of the scores: the score is monotone in the dot (keys >= 1)
     const int64_t s0 = attn_score<NOCLAMP>(a, dmin), s1 = attn_score<NOCLAMP>(a, dmax);
     const int64_t M = s0 > s1 ? s0 : s1;
@@ -2309,57 +2320,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             sum += e[j];
         }
     }
-    sum = (uint64_t)wave_sum64((int64_t)sum);
+    sum = wave_sum_dpp(sum);
     const double R = ldexp(1.0 / (double)sum, a.softmax_p);
     const double sp = softmax_sp(sum, a.softmax_p);
-    uint32_t p[KB];
-#pragma unroll
-    for (int j = 0; j < KB; j++)  // <= 2^P <= 2^30; 0 for keys past the row (e = 0)
-        p[j] = softmax_p_of(e[j], R, sp);
     wait_vmcnt<0>();  // this wave's V rows landed in its LDS region
-    int32_t lo[16], hi[16];
+    v4i acc[4];
 #pragma unroll
-    for (int c = 0; c < 16; c++) lo[c] = hi[c] = 0;
+    for (int c = 0; c < 4; c++) acc[c] = v4i{0, 0, 0, 0};
 #pragma unroll
-    for (int i = 0; i < 4 * KB; i++) {
-        if (16 * i >= keys) break;
-        const uint32_t pk = (uint32_t)__shfl((int)p[i >> 2], 16 * (i & 3) + (lane >> 2), 64);
-        const int k = (lane >> 2) + 16 * i;
-        const uint32_t pv = k < keys ? pk : 0u;
-        const int32_t pl = (int32_t)(pv & 0xffffu), ph = (int32_t)(pv >> 16);
-        const v4i raw = *(const v4i *)(sv + i * 1024 + 16 * lane);
-        const int8_t *v = (const int8_t *)&raw;
-#pragma unroll
-        for (int c = 0; c < 16; c++) {
-            lo[c] += pl * (int32_t)v[c];
-            hi[c] += ph * (int32_t)v[c];
-        }
+    for (int j = 0; j < KB; j++) {
+        if (64 * j >= keys) break;
+        // p <= 2^P <= 2^30; 0 for keys past the row (e = 0)
+        decode_pv_block(sv + 4096 * j, mem, softmax_p_of(e[j], R, sp), lane, acc);
     }
-    // The 16 lanes of channel group g = lane % 4 (lane bits 2..5) hold partial sums of channels
-    // 16 g .. +16 over disjoint keys. A butterfly halves the channels a lane keeps in each round
-    // (bit 2: channels 8..15 or 0..7 of the 16, then bits 3, 4, 5), so lane l ends with the whole
-    // sum of one channel, 16 g + 8 b2 + 4 b3 + 2 b4 + b5. lo and hi stay i32: over at most 256
-    // keys |sum pl v| <= 256 (2^16 - 1) 128 < 2^31 and |sum ph v| <= 256 2^14 128.
-    auto halve = [&](auto n, int o) {  // n channels -> n / 2
-        const bool up = (lane & o) != 0;
-#pragma unroll
-        for (int c = 0; c < n / 2; c++) {
-            const int32_t lk = up ? lo[n / 2 + c] : lo[c], ls = up ? lo[c] : lo[n / 2 + c];
-            const int32_t hk = up ? hi[n / 2 + c] : hi[c], hs = up ? hi[c] : hi[n / 2 + c];
-            lo[c] = lk + __shfl_xor(ls, o, 64);
-            hi[c] = hk + __shfl_xor(hs, o, 64);
-        }
-    };
-    halve(std::integral_constant<int, 16>{}, 4);
-    halve(std::integral_constant<int, 8>{}, 8);
-    halve(std::integral_constant<int, 4>{}, 16);
-    halve(std::integral_constant<int, 2>{}, 32);
-    const int ch = 16 * (lane & 3) + ((lane >> 2) & 1) * 8 + ((lane >> 3) & 1) * 4 + ((lane >> 4) & 1) * 2 +
-                   ((lane >> 5) & 1);
-    // |acc| <= 256 2^30 2^7 < 2^53
+    decode_pv_store(mem, lane, acc);
+    asm volatile("" ::: "memory");  // (the wave's LDS operations stay in order)
     const double mo = a.out_s > 95 ? 0.0 : ldexp((double)a.out_m, -a.out_s);
-    const int64_t acc = (int64_t)hi[0] * 65536 + lo[0];
-    *attn_out(a, r, h * 64 + ch) = (int8_t)attn_out_byte(acc, mo, a.out_m, a.out_s);
+    *attn_out(a, r, h * 64 + lane) = (int8_t)attn_out_byte(decode_pv_sum(mem, lane), mo, a.out_m, a.out_s);
 }
 
 template <bool NOCLAMP>
@@ -2367,7 +2344,7 @@ static hipError_t launch_decode_wave(const AttnArgs &a, int n_rows, int kmax, hi
     const int n_rh = n_rows * a.n_head;
     const dim3 grid((n_rh + 3) / 4);
     const int kb = (kmax + 63) / 64;
-    const size_t lds = (size_t)4 * kb * 4096;  // 16 to 64 KiB
+    const size_t lds = (size_t)4 * (kb * 4096 + 1024);  // 20 to 68 KiB
     if (kb <= 1) launch_k((k_attend_decode_wave<NOCLAMP, 1>), grid, dim3(256), lds, stream, a, n_rh, kmax);
     else if (kb == 2) launch_k((k_attend_decode_wave<NOCLAMP, 2>), grid, dim3(256), lds, stream, a, n_rh, kmax);
     else if (kb == 3) launch_k((k_attend_decode_wave<NOCLAMP, 3>), grid, dim3(256), lds, stream, a, n_rh, kmax);
@@ -2414,17 +2391,8 @@ hipError_t launch_attend_split(const AttnArgs &a, int n_rows, const SplitPlan &p
         return attn_noclamp(a) ? launch_decode_wave<true>(a, n_rows, kmax, stream)
                                : launch_decode_wave<false>(a, n_rows, kmax, stream);
     if (attend_split_one_launch(a.hd, a.ctx_cap, p)) {  // one launch, no scratch
-        const int kmax64 = (kmax + 63) & ~63;
-        if (kmax64 > 1024) return hipErrorInvalidValue;  // the kernel's register rows end at 1,024 keys
-        const size_t dyn = (size_t)kmax64 * 4;  // the weights p
-        const bool nc = attn_noclamp(a);
-        const void *fn = nc ? (const void *)k_attend_decode64<true> : (const void *)k_attend_decode64<false>;
-        {
-            const hipError_t e = allow_dynamic_lds(fn, 4096);
-            if (e != hipSuccess) return e;
-        }
-        if (nc) launch_k(k_attend_decode64<true>, dim3(n_rows * a.n_head), dim3(256), dyn, stream, a, kmax);
-        else launch_k(k_attend_decode64<false>, dim3(n_rows * a.n_head), dim3(256), dyn, stream, a, kmax);
+        if (attn_noclamp(a)) launch_k(k_attend_decode64<true>, dim3(n_rows * a.n_head), dim3(256), 0, stream, a, kmax);
+        else launch_k(k_attend_decode64<false>, dim3(n_rows * a.n_head), dim3(256), 0, stream, a, kmax);
         return hipGetLastError();
     }
     const dim3 grid(n_rows * a.n_head, p.chunks);

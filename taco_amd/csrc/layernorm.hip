@@ -12,44 +12,7 @@
 #include "intmath.h"
 #include "launch.h"
 
-#include <type_traits>
-
 namespace hs {
-
-namespace {
-
-// Butterfly moves inside a row of 16 lanes: xor 1, xor 2, then mirrors (equal inside the quads and
-// octets by then), 64-bit values as two words; xor 16 and 32 across.
-template <int CTRL>
-__device__ __forceinline__ int32_t dpp_mov(int32_t v) {
-    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
-}
-template <int STEP>
-__device__ __forceinline__ int32_t lane_move(int32_t v) {
-    if constexpr (STEP == 0) return dpp_mov<0xB1>(v);        // quad_perm [1,0,3,2]
-    else if constexpr (STEP == 1) return dpp_mov<0x4E>(v);   // quad_perm [2,3,0,1]
-    else if constexpr (STEP == 2) return dpp_mov<0x141>(v);  // row_half_mirror
-    else if constexpr (STEP == 3) return dpp_mov<0x140>(v);  // row_mirror
-    else return __shfl_xor(v, STEP == 4 ? 16 : 32, 64);  // across the rows
-}
-template <int STEP>
-__device__ __forceinline__ int64_t lane_move64(int64_t v) {
-    const uint32_t lo = (uint32_t)lane_move<STEP>((int32_t)v), hi = (uint32_t)lane_move<STEP>((int32_t)(v >> 32));
-    return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-
-// Runs f(step) for the butterfly steps over LPR lanes.
-template <int LPR, typename F>
-__device__ __forceinline__ void butterfly(F f) {
-    f(std::integral_constant<int, 0>{});
-    f(std::integral_constant<int, 1>{});
-    f(std::integral_constant<int, 2>{});
-    f(std::integral_constant<int, 3>{});
-    if constexpr (LPR >= 32) f(std::integral_constant<int, 4>{});
-    if constexpr (LPR >= 64) f(std::integral_constant<int, 5>{});
-}
-
-}  // namespace
 
 // NG groups of 4 columns per lane (d % 4 == 0, d <= 4 NG LPR). Every load of x is unconditional,
 // from a clamped address (a row past n_rows reads the last row, a column past d the last group;
