@@ -312,4 +312,150 @@ hipError_t launch_gemm_rows(Epi epi, const GemmArgs &g, hipStream_t stream) {
     }
 }
 
+// ---- The LM head of few rows, compact logits (LogitsCompact) -------------------------------------
+// What bounds it is wte (39 MB at width 768: 8 us at 5 TB/s), once every column block is read once
+// and ahead of its use: the 256 x 128 tiles of k_gemm compute 256 rows for one and wait at every
+// k-step. Here the rows' A goes to LDS once, in fragment order (lane l's 16 bytes at 16 l: no bank
+// conflicts), and each wave takes 16 columns over all of K with U k-steps of W in flight in
+// registers. Every wave holding A from the caches instead read 4 bytes of it for each byte of W:
+// 18.6 us at 64 rows. A row's tile max meets over the 4 waves of a 64-column tile in LDS.
+// Measured against the tiles of k_gemm, us a launch: width 768 1 row 15.8 -> 8.2, 16 rows 15.9 -> 8.5,
+// 32 rows 16.5 -> 9.6, 64 rows 17.6 -> 12.2; width 1024 1 row 19.0 -> 11.2, 64 rows 20.5 -> 15.6;
+// width 1600 1 row 29.3 -> 17.3, 64 rows 31.3 -> 22.2. 128 rows (128 accumulated rows a wave): 20.3 ->
+// 19.5 at width 768 but 32.9 -> 41 at 1600, so more than 64 rows stay with the tiles.
+template <int MT, bool NARROW, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void k_head_rows(GemmArgs g) {
+    constexpr int U = 12;
+    extern __shared__ __align__(16) char s_a[];  // the rows' A: [k-step][16-row tile][lane][16 B]
+    using L = typename std::conditional<NARROW, int32_t, int64_t>::type;
+    constexpr L LMIN = NARROW ? (L)INT32_MIN : (L)INT64_MIN;
+    __shared__ L s_max[WAVES][16 * MT];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n0 = blockIdx.x * 16 * WAVES;
+    const int steps = g.k_pad / GEMM_BK;
+    const size_t pa = (size_t)g.a_rows * 64, pw = (size_t)g.w_rows * 64;  // bytes per panel
+    const uint32_t lane_off = (uint32_t)((lane & 15) * 64 + (lane >> 4) * 16);
+    const int8_t *ab = g.a + lane_off, *wb = g.w + (size_t)(n0 + 16 * wave) * 64 + lane_off;
+    v4i fw[U], acc[MT];
+    auto load = [&](int u, int s) { fw[u] = *(const v4i *)(wb + (size_t)s * pw); };
+    auto mul = [&](int u, int s) {
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            const v4i f = *(const v4i *)(s_a + ((s * MT + i) * 64 + lane) * 16);
+            acc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[u], f, acc[i], 0, 0, 0);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < MT; i++) acc[i] = v4i{0, 0, 0, 0};
+#pragma unroll
+    for (int u = 0; u < U; u++) load(u, u < steps ? u : steps - 1);
+    for (int c = wave; c < steps * MT; c += WAVES)
+        __builtin_amdgcn_global_load_lds((const void *)(ab + (size_t)(c / MT) * pa + (c % MT) * 1024),
+                                         (lds_void *)(s_a + c * 1024), 16, 0, 0);
+    wait_vmcnt<0>();  // this wave's part landed (the barrier shows it to all)
+    lds_barrier();
+    // the lane's 4 columns (n4 is below n_pad: the multipliers are padded)
+    const int n4 = n0 + 16 * wave + 4 * (lane >> 4);
+    const v4i mult = *(const v4i *)(g.mult + n4);
+    int s = 0;
+    for (; s + U < steps; s += U) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            mul(u, s + u);
+            load(u, s + u + U < steps ? s + u + U : steps - 1);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+        if (s + u < steps) mul(u, s + u);
+    // logit = clamp(rescale(acc, m, s), +-2^40) (ops.rs:229-234): |acc m| < 2^62; NARROW (shift 31
+    // or more): an i32
+    const int s_eff = g.shift < 63 ? g.shift : 63;
+    const int64_t half = s_eff ? (int64_t)1 << (s_eff - 1) : 0;
+    L l[MT][4];
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+        L mx = LMIN;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int64_t r = ((int64_t)acc[i][e] * mult[e] + half) >> s_eff;
+            l[i][e] = n4 + e < g.n ? (NARROW ? (L)r : (L)clamp64(r, -((int64_t)1 << 40), (int64_t)1 << 40)) : LMIN;
+            mx = l[i][e] > mx ? l[i][e] : mx;
+        }
+#pragma unroll
+        for (int o = 16; o < 64; o <<= 1) {  // the 4 lanes of a row
+            const L u = __shfl_xor(mx, o, 64);
+            mx = u > mx ? u : mx;
+        }
+        if (lane < 16) s_max[wave][16 * i + lane] = mx;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+        const int m = 16 * i + (lane & 15);
+        const int w0 = wave & ~3;  // the 4 waves of a 64-column tile
+        L mx = s_max[w0][m];
+#pragma unroll
+        for (int w = 1; w < 4; w++) mx = s_max[w0 + w][m] > mx ? s_max[w0 + w][m] : mx;
+        if (m >= g.m || n0 + 16 * w0 >= g.n) continue;
+        if (wave == w0 && lane < 16) g.tmax[(size_t)m * g.tmax_ld + n0 / 64 + w0 / 4] = (int64_t)mx;
+        // distances capped as the fused epilogue caps them: 65535 (NARROW), else cap16
+        uint16_t d[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            if (NARROW) {
+                const uint32_t u = (uint32_t)mx - (uint32_t)l[i][e];
+                d[e] = (uint16_t)(u < 65535u ? u : 65535u);
+            } else {
+                const int64_t u = (int64_t)mx - (int64_t)l[i][e];
+                d[e] = (uint16_t)(u < g.cap16 ? u : g.cap16);
+            }
+        }
+        uint16_t *o = (uint16_t *)g.out + (size_t)m * g.ldo + n4;
+        if (n4 + 4 <= g.n) {
+            *(uint2 *)o = make_uint2(d[0] | ((uint32_t)d[1] << 16), d[2] | ((uint32_t)d[3] << 16));
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (n4 + e < g.n) o[e] = d[e];
+        }
+    }
+}
+
+// Up to 64 rows whose A fits in LDS beside the row maxima, 8-byte output groups, padded multipliers.
+// (launch_gemm has checked that the panels hold 256 rows and round_up(n, 256) columns: a workgroup
+// reads 16 MT of the rows and at most 256 columns.)
+static int head_tiles(const GemmArgs &g) { return g.m <= 16 ? 1 : g.m <= 32 ? 2 : 4; }
+static size_t head_lds(const GemmArgs &g) { return (size_t)g.k_pad * 16 * head_tiles(g); }
+
+bool head_rows_fits(const GemmArgs &g) {
+    return g.m <= 64 && head_lds(g) <= (size_t)144 * 1024 && g.params_padded && g.ldo % 4 == 0 &&
+           ((uintptr_t)g.out & 7) == 0;
+}
+
+template <int MT, int WAVES>
+static hipError_t head_rows_run(const GemmArgs &g, hipStream_t stream) {
+    auto run = [&](auto kernel) {
+        const size_t lds = head_lds(g);
+        const hipError_t e = allow_dynamic_lds((const void *)kernel, lds);
+        if (e != hipSuccess) return e;
+        launch_k(kernel, dim3((g.n + 16 * WAVES - 1) / (16 * WAVES)), dim3(64 * WAVES), lds, stream, g);
+        return hipGetLastError();
+    };
+    return g.shift >= 31 ? run(k_head_rows<MT, true, WAVES>) : run(k_head_rows<MT, false, WAVES>);
+}
+
+// 8 waves a workgroup while two or more fit a CU's LDS, else 16: 16 waves of one workgroup read W
+// as two of 8 would (64 rows at width 1600: 27.0 us with 8 waves, 22.2 with 16; at width 768 12.2 and
+// 13.3).
+hipError_t launch_head_rows(const GemmArgs &g, hipStream_t stream) {
+    const int mt = head_tiles(g);
+    if (head_lds(g) <= (size_t)64 * 1024) {
+        return mt == 1 ? head_rows_run<1, 8>(g, stream) : mt == 2 ? head_rows_run<2, 8>(g, stream)
+                                                                  : head_rows_run<4, 8>(g, stream);
+    }
+    return mt == 1 ? head_rows_run<1, 16>(g, stream) : mt == 2 ? head_rows_run<2, 16>(g, stream)
+                                                               : head_rows_run<4, 16>(g, stream);
+}
+
 }  // namespace hs

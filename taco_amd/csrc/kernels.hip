@@ -1132,7 +1132,9 @@ hipError_t launch_gemm(Epi epi, const GemmArgs &ga, hipStream_t stream) {
         case Epi::Residual: return launch_gemm_e<2>(g, stream);
         case Epi::Gelu: return launch_gemm_e<3>(g, stream);
         case Epi::Logits: return launch_gemm_e<4>(g, stream);
-        case Epi::LogitsCompact: return launch_gemm_e<5>(g, stream);
+        case Epi::LogitsCompact:
+            if (head_rows_fits(g)) return launch_head_rows(g, stream);
+            return launch_gemm_e<5>(g, stream);
         case Epi::GeluWide: return launch_gemm_e<6>(g, stream);
         case Epi::ResidualWide:
         case Epi::LogitsWide:

@@ -40,6 +40,10 @@ hipError_t allow_dynamic_lds(const void *fn, size_t bytes);
 bool gemm_rows_fits(Epi epi, const GemmArgs &g);
 hipError_t launch_gemm_rows(Epi epi, const GemmArgs &g, hipStream_t stream);
 
+// The LM head of few rows with compact logits (gemm_rows.hip).
+bool head_rows_fits(const GemmArgs &g);
+hipError_t launch_head_rows(const GemmArgs &g, hipStream_t stream);
+
 // LayerNorm with 8-bit outputs in single precision (layernorm.hip).
 bool layernorm_f32_fits(const LnArgs &a);
 hipError_t launch_layernorm_f32(const LnArgs &a, int n_rows, hipStream_t stream);
