@@ -187,8 +187,8 @@ struct AttnArgs {
 };
 hipError_t launch_attend(const AttnArgs &a, int n_rows, hipStream_t stream);
 
-// Decode attention (head_dim 16, 32, 64, 128 or 256). head_dim 64 with at most 1,024 keys: one
-// launch, a workgroup per (row, head), `scratch` unused. Otherwise split over key chunks: four
+// Decode attention (head_dim 16, 32, 64, 128 or 256). Head dims up to 128 with at most 1,024 keys: one
+// launch, a wave or a workgroup per (row, head), `scratch` unused. Otherwise split over key chunks: four
 // launches over (row, head, chunk) with exact integer partials in `scratch` (attend_split_bytes
 // bytes, 256-byte aligned). The plan's `max_keys` bounds every row's key count.
 struct SplitPlan {
@@ -197,7 +197,7 @@ struct SplitPlan {
 };
 inline bool attend_split_ok(int hd) { return hd >= 16 && hd <= 256 && (hd & (hd - 1)) == 0; }
 SplitPlan attend_split_plan(int n_rows, int n_head, int max_keys);
-// True when the plan takes the one-launch kernel (head_dim 64, at most 1,024 keys): no scratch.
+// True when the plan takes a one-launch kernel (head dims up to 128, at most 1,024 keys): no scratch.
 bool attend_split_one_launch(int hd, int ctx_cap, const SplitPlan &p);
 // The scratch bytes of the split launches (0 when the plan takes the one-launch kernel).
 size_t attend_split_bytes(const AttnArgs &a, int n_rows, const SplitPlan &p);

@@ -1998,59 +1998,6 @@ __global__ __launch_bounds__(64) void k_split_sum(AttnArgs a, int n_rows, SplitP
     if (lane == 0) S.ps[(size_t)rh * pl.chunks + c] = sum;
 }
 
-template <bool NOCLAMP>
-__global__ __launch_bounds__(64) void k_split_pv(AttnArgs a, int n_rows, SplitPlan pl, void *scratch) {
-    extern __shared__ uint32_t s_p[];  // chunk_keys entries
-    const int rh = blockIdx.x, c = blockIdx.y, lane = threadIdx.x;
-    const int r = rh / a.n_head, h = rh - r * a.n_head, hd = a.hd;
-    const SplitScratch S = split_scratch(scratch, n_rows, a.n_head, a.ctx_cap, pl.chunks, hd);
-    const int keys = split_keys(a, r), k0 = c * pl.chunk_keys;
-    const int k1 = k0 + pl.chunk_keys < keys ? k0 + pl.chunk_keys : keys;
-    if (k0 >= k1) {  // an empty chunk contributes nothing
-        for (int i = lane; i < hd; i += 64) S.part[((size_t)rh * pl.chunks + c) * hd + i] = 0;
-        return;
-    }
-    const int nch = (keys + pl.chunk_keys - 1) / pl.chunk_keys;
-    const int64_t M = split_max<NOCLAMP>(a, S, pl, rh, nch);
-    uint64_t sum = 0;
-    for (int cc = 0; cc < nch; cc++) sum += S.ps[(size_t)rh * pl.chunks + cc];
-    const uint64_t frac = sum >= 2 ? div_2p64(sum) : 0;
-    const int64_t last = a.exp_len - 1;
-    for (int k = k0 + lane; k < k1; k += 64) {
-        const int64_t dd = M - attn_score<NOCLAMP>(a, S.dots[(size_t)rh * a.ctx_cap + k]);
-        const uint64_t num = (uint64_t)a.exp_table[dd < last ? dd : last] << a.softmax_p;
-        uint64_t q = num;
-        if (sum >= 2) {
-            q = __umul64hi(num, frac);  // q <= floor(num / S) <= q + 1
-            if (num - q * sum >= sum) q++;
-        }
-        s_p[k - k0] = (uint32_t)q;  // <= 2^P <= 2^30
-    }
-    __syncthreads();
-    // lane l: channels 16 (l % G) .. +16 of rows k0 + l / G, k0 + l / G + 64 / G, ... (G = hd / 16,
-    // a power of two, so the lanes of one channel group differ exactly in the bits >= G)
-    const int G = hd / 16, R = 64 / G;
-    int64_t acc[16];
-#pragma unroll
-    for (int i = 0; i < 16; i++) acc[i] = 0;
-    const int8_t *V = a.vc + ((size_t)split_slot(a, r) * a.n_head + h) * a.ctx_cap * hd;
-    for (int k = k0 + lane / G; k < k1; k += R) {
-        const int64_t p = s_p[k - k0];
-        const v4i raw = *(const v4i *)(V + (size_t)k * hd + (lane % G) * 16);
-        const int8_t *v = (const int8_t *)&raw;
-#pragma unroll
-        for (int i = 0; i < 16; i++) acc[i] += p * v[i];
-    }
-#pragma unroll
-    for (int i = 0; i < 16; i++)
-        for (int o = G; o < 64; o <<= 1) acc[i] += __shfl_xor(acc[i], o, 64);
-    if (lane < G) {
-        int64_t *dst = S.part + ((size_t)rh * pl.chunks + c) * hd + lane * 16;
-#pragma unroll
-        for (int i = 0; i < 16; i++) dst[i] = acc[i];
-    }
-}
-
 __global__ void k_split_out(AttnArgs a, int n_rows, SplitPlan pl, void *scratch) {
     const int rh = blockIdx.x, t = threadIdx.x;
     const int r = rh / a.n_head, h = rh - r * a.n_head, hd = a.hd;
@@ -2062,47 +2009,127 @@ __global__ void k_split_out(AttnArgs a, int n_rows, SplitPlan pl, void *scratch)
     *attn_out(a, r, h * hd + t) = (int8_t)clamp128(rescale_full(o, a.out_m, a.out_s), -127, 127);
 }
 
-// ---- The pieces of the one-launch decode kernels (head_dim 64) ------------------------------------
+// ---- The pieces of the one-launch decode kernels ---------------------------------------------------
 // Sum p v of one query row is a product of a 64-channel x 64-key matrix with p, and p is four
 // balanced i8 digits (the bytes of p + 0x80808080, xor 0x80): one v_mfma_i32_16x16x64_i8 takes 16
 // channels x 64 keys against the four digit planes as four of its columns (the other twelve
 // repeat them), so a block of 64 keys is 4 MFMAs where 24-bit multiplies took 192 VALU
 // instructions a wave, and the sums need no butterfly over the lanes.
-// A block's V rows lie in LDS as dense 64-byte rows, 16-byte chunk c of row r at slot
-// 4 r + (c ^ vsw(r)); the V^T operand comes by transposing reads (as in k_attend_short), whose
-// operand byte 4 t + e of lane group g holds key 16 t + 4 g + e. `mem` is 1 KiB of the wave.
-__device__ __forceinline__ int vsw(int r) { return ((r >> 1) ^ (r >> 3)) & 3; }
+// A block's V rows lie in LDS as dense rows of 16 NC bytes (NC = 4: head dims from 64 on, in groups
+// of 64 channels; below that one group of hd), 16-byte chunk c of row r at slot NC r + (c ^ vsw(r));
+// the V^T operand comes by transposing reads (as in k_attend_short), whose operand byte 4 t + e of
+// lane group g holds key 16 t + 4 g + e. `mem` is 1 KiB of the wave.
+template <int NC>
+__device__ __forceinline__ int vsw(int r) {
+    return NC == 4 ? ((r >> 1) ^ (r >> 3)) & 3 : NC == 2 ? (r >> 2) & 1 : 0;
+}
 
-__device__ __forceinline__ void decode_pv_block(const int8_t *sv, int8_t *mem, uint32_t p, int lane, v4i (&acc)[4]) {
-    // the digits of this lane's key to [plane][key in operand order]
+// Lane l's p of key l to the digit operand of the block.
+__device__ __forceinline__ v4i decode_pv_digits(int8_t *mem, uint32_t p, int lane) {
     const uint32_t q = (p + 0x80808080u) ^ 0x80808080u;
     int8_t *w = mem + 16 * ((lane >> 2) & 3) + 4 * (lane >> 4) + (lane & 3);
 #pragma unroll
     for (int k = 0; k < 4; k++) w[64 * k] = (int8_t)(q >> (8 * k));
-    const v4i pf = *(const v4i *)(mem + 64 * (lane & 3) + 16 * (lane >> 4));
+    return *(const v4i *)(mem + 64 * (lane & 3) + 16 * (lane >> 4));
+}
+template <int NC>
+__device__ __forceinline__ void decode_pv_block(const int8_t *sv, const v4i &pf, int lane, v4i *acc) {
     const int ql = lane & 15, qg = lane >> 4;
     const int tr_k = ql >> 1, tr_h = ql & 1;
     const int key0 = 16 * (tr_k >> 2) + 4 * qg + (tr_k & 3);
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
-        const int8_t *p0 = sv + (4 * key0 + (c ^ vsw(key0 & 15))) * 16 + 8 * tr_h;
+    for (int c = 0; c < NC; c++) {
+        const int8_t *p0 = sv + (NC * key0 + (c ^ vsw<NC>(key0 & 15))) * 16 + 8 * tr_h;
         const v2i r0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)p0);
-        const v2i r1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(p0 + 32 * 64));
+        const v2i r1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(p0 + 32 * 16 * NC));
         acc[c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(v4i{r0[0], r0[1], r1[0], r1[1]}, pf, acc[c], 0, 0, 0);
     }
 }
 
 // acc[c][e] of lane l holds channel 16 c + 4 (l / 16) + e of plane l % 16 (< 4): to [plane][64] in mem.
-__device__ __forceinline__ void decode_pv_store(int8_t *mem, int lane, const v4i (&acc)[4]) {
+template <int NC>
+__device__ __forceinline__ void decode_pv_store(int8_t *mem, int lane, const v4i *acc) {
     if ((lane & 15) < 4) {
 #pragma unroll
-        for (int c = 0; c < 4; c++) *(v4i *)(mem + 256 * (lane & 15) + 64 * c + 16 * (lane >> 4)) = acc[c];
+        for (int c = 0; c < NC; c++) *(v4i *)(mem + 256 * (lane & 15) + 64 * c + 16 * (lane >> 4)) = acc[c];
     }
 }
 // The planes' sum of channel ch: below 2^24 per plane, |sum| <= 1,024 2^30 2^7 < 2^53.
 __device__ __forceinline__ int64_t decode_pv_sum(const int8_t *mem, int ch) {
     const int32_t *m = (const int32_t *)mem + ch;
     return (int64_t)m[0] + (int64_t)m[64] * 256 + (int64_t)m[128] * 65536 + (int64_t)m[192] * 16777216;
+}
+
+// The split form's sums p v of a chunk: one wave, 64 keys at a time on the digit planes (above), the
+// next block's V rows in flight. (One i64 multiply-add a channel and key and a butterfly at the end
+// took 29.1 us at head_dim 64, 2,000 keys, 512 row-heads; this 13.0.) At most 4,096 keys: below 2^26
+// a plane.
+template <bool NOCLAMP, int HD>
+__global__ __launch_bounds__(64) void k_split_pv(AttnArgs a, int n_rows, SplitPlan pl, void *scratch) {
+    constexpr int QT = HD / 16, NC = HD < 64 ? QT : 4, NG = QT / NC, RB = 16 * NC, RL = 64 / NC, SH = NC / 2;
+    __shared__ __attribute__((aligned(16))) int8_t s_v[64 * HD], s_mem[1024];
+    const int rh = blockIdx.x, c = blockIdx.y, lane = threadIdx.x;
+    const int r = rh / a.n_head, h = rh - r * a.n_head;
+    const SplitScratch S = split_scratch(scratch, n_rows, a.n_head, a.ctx_cap, pl.chunks, HD);
+    int64_t *part = S.part + ((size_t)rh * pl.chunks + c) * HD;
+    const int keys = split_keys(a, r), k0 = c * pl.chunk_keys;
+    const int k1 = k0 + pl.chunk_keys < keys ? k0 + pl.chunk_keys : keys;
+    if (k0 >= k1) {  // an empty chunk contributes nothing
+        for (int i = lane; i < HD; i += 64) part[i] = 0;
+        return;
+    }
+    // lane l: chunk (l % NC) ^ vsw of rows l / NC + RL u (keys past the chunk reload its last key;
+    // their weight is 0)
+    const int8_t *V = a.vc + ((size_t)split_slot(a, r) * a.n_head + h) * a.ctx_cap * HD;
+    v4i vr[NG][NC];
+    auto load = [&](int kb) {
+#pragma unroll
+        for (int u = 0; u < NC; u++) {
+            const int row = RL * u + (lane >> SH), k = kb + row;
+            const int8_t *v = V + (size_t)(k < k1 ? k : k1 - 1) * HD + 16 * ((lane & (NC - 1)) ^ vsw<NC>(row & 15));
+#pragma unroll
+            for (int g = 0; g < NG; g++) vr[g][u] = *(const v4i *)(v + 64 * g);
+        }
+    };
+    load(k0);
+    const int nch = (keys + pl.chunk_keys - 1) / pl.chunk_keys;
+    const int64_t M = split_max<NOCLAMP>(a, S, pl, rh, nch);
+    uint64_t sum = 0;
+    for (int cc = 0; cc < nch; cc++) sum += S.ps[(size_t)rh * pl.chunks + cc];
+    const uint64_t frac = sum >= 2 ? div_2p64(sum) : 0;
+    const int64_t last = a.exp_len - 1;
+    v4i acc[NG][NC];
+#pragma unroll
+    for (int g = 0; g < NG; g++)
+#pragma unroll
+        for (int i = 0; i < NC; i++) acc[g][i] = v4i{0, 0, 0, 0};
+    for (int kb = k0; kb < k1; kb += 64) {
+        uint64_t q = 0;
+        if (kb + lane < k1) {
+            const int64_t dd = M - attn_score<NOCLAMP>(a, S.dots[(size_t)rh * a.ctx_cap + kb + lane]);
+            const uint64_t num = (uint64_t)a.exp_table[dd < last ? dd : last] << a.softmax_p;
+            q = num;
+            if (sum >= 2) {
+                q = __umul64hi(num, frac);  // q <= floor(num / S) <= q + 1
+                if (num - q * sum >= sum) q++;
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < NG; g++)
+#pragma unroll
+            for (int u = 0; u < NC; u++) *(v4i *)(s_v + 64 * RB * g + 1024 * u + 16 * lane) = vr[g][u];
+        load(kb + 64);
+        const v4i pf = decode_pv_digits(s_mem, (uint32_t)q, lane);  // q <= 2^P <= 2^30
+#pragma unroll
+        for (int g = 0; g < NG; g++) decode_pv_block<NC>(s_v + 64 * RB * g, pf, lane, acc[g]);
+    }
+#pragma unroll
+    for (int g = 0; g < NG; g++) {
+        decode_pv_store<NC>(s_mem, lane, acc[g]);
+        asm volatile("" ::: "memory");  // (the wave's LDS operations stay in order)
+        if (lane < RB) part[64 * g + lane] = decode_pv_sum(s_mem, lane);
+        asm volatile("" ::: "memory");
+    }
 }
 
 // The extreme values over the wave.
@@ -2120,13 +2147,12 @@ __device__ __forceinline__ uint64_t wave_sum_dpp(uint64_t v) {
 }
 
 // Decode attention for head_dim 64 and at most 1,024 keys in one launch: one workgroup (4 waves)
-// per (row, head). The row's K rows (thread t: keys t + 256 j) and V rows (in the layout the p v
-// sums read them: thread t, keys t / 4 + 64 i, chunk t % 4) go to registers in one round of
+// per (row, head). The row's K rows (thread t: keys t + 256 j) and the V rows of the
+// wave's key blocks go to registers in one round of
 // loads with no branch around them, K first, so the dots wait for K alone (the compiler counts the
 // in-order loads exactly; with part of V going to LDS by global_load_lds it waited for every
 // load); the dots, the row max, the table sum, the weights p and the sums p v then follow the rules
-// of the split kernels above. Dynamic LDS: the kmax64 = 64 ceil(kmax / 64) weights. 155 VGPRs:
-// three workgroups per CU (768 row-heads in one round). Measured at 1,024 keys and 768 row-heads:
+// of the split kernels above. 140 VGPRs: three workgroups per CU (768 row-heads in one round). Measured at 1,024 keys and 768 row-heads:
 // 34.2 us with all of V in LDS (two workgroups per CU), 31.0 with half, then 29.8 -> 27.9 with
 // the butterfly reduction.
 template <bool NOCLAMP>
@@ -2166,7 +2192,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
     for (int i = 0; i < 16; i++) {
         const int row = 16 * (i & 3) + (lane >> 2), k = 64 * (4 * (i >> 2) + w) + row;
-        vr[i] = *(const v4i *)(a.vc + base + (size_t)(k < keys ? k : keys - 1) * 64 + 16 * ((lane & 3) ^ vsw(row & 15)));
+        vr[i] = *(const v4i *)(a.vc + base + (size_t)(k < keys ? k : keys - 1) * 64 + 16 * ((lane & 3) ^ vsw<4>(row & 15)));
     }
     __builtin_amdgcn_sched_barrier(0);  // every load issued before the first wait
     // the dots wait for K alone (the compiler's waits on the K registers)
@@ -2232,9 +2258,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
         for (int u = 0; u < 4; u++) *(v4i *)(s_v[w] + 1024 * u + 16 * lane) = vr[4 * j + u];
         // p <= 2^P <= 2^30; 0 for keys past the row (e = 0)
-        decode_pv_block(s_v[w], s_mem[w], softmax_p_of(e[j], R, sp), lane, acc);
+        decode_pv_block<4>(s_v[w], decode_pv_digits(s_mem[w], softmax_p_of(e[j], R, sp), lane), lane, acc);
     }
-    decode_pv_store(s_mem[w], lane, acc);
+    decode_pv_store<4>(s_mem[w], lane, acc);
     __syncthreads();
     if (tid < 64) {
         const int64_t o = decode_pv_sum(s_mem[0], tid) + decode_pv_sum(s_mem[1], tid) +
@@ -2244,47 +2270,187 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     }
 }
 
-// Decode attention for head_dim 64 and at most 64 KB keys (KB <= 4): one wave per (row, head),
-// four independent waves per workgroup, no barrier. Lane l holds the K rows of keys l + 64 j, and
-// the wave's V rows go to its own LDS region ([key][64 B], 16 keys per global_load_lds), all
-// loads issued at once; the lane later reads the 16-byte V chunk l % 4 of keys l / 4 + 16 i
-// back. The dots, the row
-// max (from the extreme dots), the table sum and p = floor(e 2^P / S) (the 2^64 / S reciprocal
-// with one correction) follow the rules of the kernels above. For sum p v the lane fetches the p
-// of its V keys from the lanes that formed them (the key of V slot i is l / 4 + 16 i, formed by
-// lane (l / 4 + 16 i) % 64 in its K round i / 4), splits p = 2^16 ph + pl so both halves sum in
-// i32 (at most 16 keys per lane, |v| <= 128: below 2^27), and the lanes of one chunk are summed
-// with xor shuffles.
-template <bool NOCLAMP, int KB>
+// The same for head dims 16, 32 and 128: 4 waves of 4 keys a lane, at head_dim 128 8 of 2. (At head_dim
+// 64 this form, with the same loads in the same order, took 14.3 us where k_attend_decode64 takes
+// 14.0, 768 row-heads at 640 keys.) Kernel time against
+// the four split launches: head_dim 128, 600 row-heads at 388 keys 35.3 -> 16.9 us; head_dim 32, 1,200
+// row-heads at 1,000 keys 41.7 -> 12.1 us.
+template <bool NOCLAMP, int HD>
+__global__ __launch_bounds__(HD > 64 ? 512 : 256) __attribute__((amdgpu_waves_per_eu(2))) void k_attend_decode_wg(
+    AttnArgs a, int kmax) {
+    constexpr int NW = HD > 64 ? 8 : 4, NTH = 64 * NW, KT = 1024 / NTH, QT = HD / 16;
+    constexpr int NC = HD < 64 ? QT : 4, NG = QT / NC, RB = 16 * NC;  // 64-channel groups of NC chunks
+    __shared__ __attribute__((aligned(16))) int8_t s_v[NW][64 * RB];  // a wave's block of V rows, one group
+    __shared__ __attribute__((aligned(16))) int8_t s_mem[NW][NG * 1024];  // a wave's digits, then its plane sums
+    __shared__ int32_t s_mm[2][NW];
+    __shared__ uint64_t s_sum[NW];
+    const int rh = blockIdx.x, tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+    const int r = rh / a.n_head, h = rh - r * a.n_head;
+    int keys = split_keys(a, r);
+    keys = keys < kmax ? keys : kmax;  // the launch's bound holds every row's count
+    const size_t base = ((size_t)split_slot(a, r) * a.n_head + h) * a.ctx_cap * HD;
+    // q straight into every thread's registers (one row, the same for all)
+    int qv[4 * QT];
+#pragma unroll
+    for (int t = 0; t < QT; t++) {
+        const v4i q4 = ((const v4i *)(a.q + (size_t)r * a.ldq + h * HD))[t];
+#pragma unroll
+        for (int e = 0; e < 4; e++) qv[4 * t + e] = q4[e];
+    }
+    // K: KT keys per thread, with no branch around the loads (keys past the row reload the
+    // row's last key and are left out of every sum)
+    v4i kk[KT][QT];
+#pragma unroll
+    for (int j = 0; j < KT; j++) {
+        const int k = tid + NTH * j;
+        const v4i *k16 = (const v4i *)(a.kc + base + (size_t)(k < keys ? k : keys - 1) * HD);
+#pragma unroll
+        for (int t = 0; t < QT; t++) kk[j][t] = k16[t];
+    }
+    // V after K: the rows of this wave's KT blocks of 64 keys, 64 (NW j + w) .. (the keys whose p its
+    // lanes form), by group of channels; a load takes 64 / NC rows, lane l the chunk (l % NC) ^ vsw of
+    // row l / NC of them (keys past the row reload the row's last key; their weight is 0)
+    constexpr int RL = 64 / NC, SH = NC / 2;  // (log2 of NC)
+    v4i vr[KT][NG][NC];
+#pragma unroll
+    for (int j = 0; j < KT; j++) {
+#pragma unroll
+        for (int u = 0; u < NC; u++) {
+            const int row = RL * u + (lane >> SH), k = 64 * (NW * j + w) + row;
+            const int8_t *v = a.vc + base + (size_t)(k < keys ? k : keys - 1) * HD + 16 * ((lane & (NC - 1)) ^ vsw<NC>(row & 15));
+#pragma unroll
+            for (int g = 0; g < NG; g++) vr[j][g][u] = *(const v4i *)(v + 64 * g);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // every load issued before the first wait
+    // the dots wait for K alone (the compiler's waits on the K registers)
+    int32_t d[KT];
+    int32_t dmin = INT32_MAX, dmax = INT32_MIN;
+#pragma unroll
+    for (int j = 0; j < KT; j++) {
+        int32_t x = 0;
+#pragma unroll
+        for (int t = 0; t < QT; t++) {
+            x = __builtin_amdgcn_sdot4(qv[4 * t], kk[j][t][0], x, false);
+            x = __builtin_amdgcn_sdot4(qv[4 * t + 1], kk[j][t][1], x, false);
+            x = __builtin_amdgcn_sdot4(qv[4 * t + 2], kk[j][t][2], x, false);
+            x = __builtin_amdgcn_sdot4(qv[4 * t + 3], kk[j][t][3], x, false);
+        }
+        d[j] = x;
+        if (tid + NTH * j < keys) {
+            dmin = x < dmin ? x : dmin;
+            dmax = x > dmax ? x : dmax;
+        }
+    }
+    wave_min_max(dmin, dmax);
+    if (lane == 0) {
+        s_mm[0][w] = dmin;
+        s_mm[1][w] = dmax;
+    }
+    lds_barrier();  // not the fence of __syncthreads, which would wait for the V loads too
+    // the row max of the scores: the score is monotone in the dot, so it is the score of the
+    // smallest or of the largest dot
+    int64_t M = INT64_MIN;
+#pragma unroll
+    for (int i = 0; i < NW; i++) {
+        const int32_t mn = s_mm[0][i], mx = s_mm[1][i];
+        if (mn > mx) continue;  // a wave with no key
+        const int64_t s0 = attn_score<NOCLAMP>(a, mn), s1 = attn_score<NOCLAMP>(a, mx);
+        M = s0 > M ? s0 : M;
+        M = s1 > M ? s1 : M;
+    }
+    const int64_t last = a.exp_len - 1;
+    uint32_t e[KT];
+    uint64_t sum = 0;
+#pragma unroll
+    for (int j = 0; j < KT; j++) {
+        e[j] = 0;
+        if (tid + NTH * j < keys) {
+            const int64_t dd = M - attn_score<NOCLAMP>(a, d[j]);
+            e[j] = (uint32_t)a.exp_table[dd < last ? dd : last];
+            sum += e[j];
+        }
+    }
+    sum = wave_sum_dpp(sum);
+    if (lane == 0) s_sum[w] = sum;
+    __syncthreads();
+    sum = 0;
+#pragma unroll
+    for (int i = 0; i < NW; i++) sum += s_sum[i];
+    const double R = ldexp(1.0 / (double)sum, a.softmax_p);
+    const double sp = softmax_sp(sum, a.softmax_p);
+    v4i acc[NG][NC];
+#pragma unroll
+    for (int g = 0; g < NG; g++)
+#pragma unroll
+        for (int c = 0; c < NC; c++) acc[g][c] = v4i{0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < KT; j++) {
+        if (64 * (NW * j + w) >= keys) break;  // uniform
+        v4i pf;
+#pragma unroll
+        for (int g = 0; g < NG; g++) {
+#pragma unroll
+            for (int u = 0; u < NC; u++) *(v4i *)(s_v[w] + 1024 * u + 16 * lane) = vr[j][g][u];
+            if (g == 0) {  // p <= 2^P <= 2^30; 0 for keys past the row (e = 0)
+                __builtin_amdgcn_sched_barrier(0);  // the weights' arithmetic covers the stores of V
+                pf = decode_pv_digits(s_mem[w], softmax_p_of(e[j], R, sp), lane);
+            }
+            decode_pv_block<NC>(s_v[w], pf, lane, acc[g]);
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < NG; g++) decode_pv_store<NC>(s_mem[w] + 1024 * g, lane, acc[g]);
+    __syncthreads();
+    if (tid < HD) {
+        int64_t o = 0;
+#pragma unroll
+        for (int i = 0; i < NW; i++) o += decode_pv_sum(s_mem[i] + 1024 * (tid >> 6), tid & 63);
+        const double mo = a.out_s > 95 ? 0.0 : ldexp((double)a.out_m, -a.out_s);
+        *attn_out(a, r, h * HD + tid) = (int8_t)attn_out_byte(o, mo, a.out_m, a.out_s);
+    }
+}
+
+// Decode attention for at most 64 KB keys (head_dim 64: KB <= 4): one wave per (row, head), four
+// independent waves per workgroup, no barrier. Lane l holds the K rows of keys l + 64 j, and the
+// wave's V rows go to its own LDS region ([channel group][key][16 NC B], 64 / NC keys per
+// global_load_lds), all loads issued at once. The dots, the row max (from the extreme dots), the table
+// sum and p = floor(e 2^P / S) follow the rules of the kernels above, the sums p v come from the digit
+// planes block by block. Against the four split launches, a prefill pass of 120,792 row-heads at
+// head_dim 32 and up to 400 keys: 665 -> 196 us a layer.
+template <bool NOCLAMP, int KB, int HD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_attend_decode_wave(AttnArgs a, int n_rh,
                                                                                                      int kmax) {
+    constexpr int QT = HD / 16, NC = HD < 64 ? QT : 4, NG = QT / NC, RB = 16 * NC, RL = 64 / NC, SH = NC / 2;
     const int lane = threadIdx.x & 63;
     const int rh = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (rh >= n_rh) return;
     const int r = rh / a.n_head, h = rh - r * a.n_head;
     int keys = split_keys(a, r);
     keys = keys < kmax ? keys : kmax;
-    const size_t base = ((size_t)split_slot(a, r) * a.n_head + h) * a.ctx_cap * 64;
-    int qv[16];
+    const size_t base = ((size_t)split_slot(a, r) * a.n_head + h) * a.ctx_cap * HD;
+    int qv[4 * QT];
 #pragma unroll
-    for (int t = 0; t < 16; t++) qv[t] = ((const int *)(a.q + (size_t)r * a.ldq + h * 64))[t];
-    extern __shared__ __attribute__((aligned(16))) int8_t s_v[];  // 4 waves x (KB x 4 KiB of V rows, 1 KiB)
-    int8_t *sv = s_v + (threadIdx.x >> 6) * (KB * 4096 + 1024), *mem = sv + KB * 4096;
-    v4i kk[KB][4];
+    for (int t = 0; t < 4 * QT; t++) qv[t] = ((const int *)(a.q + (size_t)r * a.ldq + h * HD))[t];
+    extern __shared__ __attribute__((aligned(16))) int8_t s_v[];  // 4 waves x (KB blocks of V rows, 1 KiB)
+    int8_t *sv = s_v + (threadIdx.x >> 6) * (KB * 64 * HD + 1024), *mem = sv + KB * 64 * HD;
+    v4i kk[KB][QT];
 #pragma unroll
     for (int j = 0; j < KB; j++) {
         if (64 * j >= keys) break;  // uniform: the rounds past the row issue nothing
         const int k = lane + 64 * j;
-        const v4i *k16 = (const v4i *)(a.kc + base + (size_t)(k < keys ? k : keys - 1) * 64);
+        const v4i *k16 = (const v4i *)(a.kc + base + (size_t)(k < keys ? k : keys - 1) * HD);
 #pragma unroll
-        for (int t = 0; t < 4; t++) kk[j][t] = k16[t];
+        for (int t = 0; t < QT; t++) kk[j][t] = k16[t];
     }
 #pragma unroll
-    for (int i = 0; i < 4 * KB; i++) {
-        if (16 * i >= keys) break;
-        const int k = (lane >> 2) + 16 * i, c = (lane & 3) ^ vsw(lane >> 2);
-        __builtin_amdgcn_global_load_lds((const void *)(a.vc + base + (size_t)(k < keys ? k : keys - 1) * 64 + 16 * c),
-                                         (lds_void *)(sv + i * 1024), 16, 0, 0);
+    for (int i = 0; i < NC * KB; i++) {
+        if (RL * i >= keys) break;
+        const int k = (lane >> SH) + RL * i, c = (lane & (NC - 1)) ^ vsw<NC>((lane >> SH) & 15);
+        const int8_t *v = a.vc + base + (size_t)(k < keys ? k : keys - 1) * HD + 16 * c;
+#pragma unroll
+        for (int g = 0; g < NG; g++)
+            __builtin_amdgcn_global_load_lds((const void *)(v + 64 * g), (lds_void *)(sv + (g * NC * KB + i) * 1024), 16, 0, 0);
     }
     int32_t d[KB];
     int32_t dmin = INT32_MAX, dmax = INT32_MIN;
@@ -2293,7 +2459,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         int32_t x = 0;
         if (64 * j < keys) {
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
+            for (int t = 0; t < QT; t++) {
                 x = __builtin_amdgcn_sdot4(qv[4 * t], kk[j][t][0], x, false);
                 x = __builtin_amdgcn_sdot4(qv[4 * t + 1], kk[j][t][1], x, false);
                 x = __builtin_amdgcn_sdot4(qv[4 * t + 2], kk[j][t][2], x, false);
@@ -2326,32 +2492,70 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const double R = ldexp(1.0 / (double)sum, a.softmax_p);
     const double sp = softmax_sp(sum, a.softmax_p);
     wait_vmcnt<0>();  // this wave's V rows landed in its LDS region
-    v4i acc[4];
+    v4i acc[NG][NC];
 #pragma unroll
-    for (int c = 0; c < 4; c++) acc[c] = v4i{0, 0, 0, 0};
+    for (int g = 0; g < NG; g++)
+#pragma unroll
+        for (int c = 0; c < NC; c++) acc[g][c] = v4i{0, 0, 0, 0};
 #pragma unroll
     for (int j = 0; j < KB; j++) {
         if (64 * j >= keys) break;
         // p <= 2^P <= 2^30; 0 for keys past the row (e = 0)
-        decode_pv_block(sv + 4096 * j, mem, softmax_p_of(e[j], R, sp), lane, acc);
+        const v4i pf = decode_pv_digits(mem, softmax_p_of(e[j], R, sp), lane);
+#pragma unroll
+        for (int g = 0; g < NG; g++) decode_pv_block<NC>(sv + (g * KB + j) * 64 * RB, pf, lane, acc[g]);
     }
-    decode_pv_store(mem, lane, acc);
-    asm volatile("" ::: "memory");  // (the wave's LDS operations stay in order)
     const double mo = a.out_s > 95 ? 0.0 : ldexp((double)a.out_m, -a.out_s);
-    *attn_out(a, r, h * 64 + lane) = (int8_t)attn_out_byte(decode_pv_sum(mem, lane), mo, a.out_m, a.out_s);
+#pragma unroll
+    for (int g = 0; g < NG; g++) {
+        decode_pv_store<NC>(mem, lane, acc[g]);
+        asm volatile("" ::: "memory");  // (the wave's LDS operations stay in order)
+        if (lane < RB)
+            *attn_out(a, r, h * HD + 64 * g + lane) =
+                (int8_t)attn_out_byte(decode_pv_sum(mem, lane), mo, a.out_m, a.out_s);
+        asm volatile("" ::: "memory");
+    }
+}
+
+// The most keys k_attend_decode_wave takes: eight blocks of 64 or 64 VGPRs of K, whichever is less. Past
+// it a workgroup per row-head, up to 1,024 keys.
+static int decode_wave_keys(int hd) { return hd == 128 ? 128 : hd == 64 ? 256 : 512; }
+
+template <bool NOCLAMP, int HD>
+static hipError_t launch_decode(const AttnArgs &a, int n_rows, int kmax, hipStream_t stream) {
+    const int n_rh = n_rows * a.n_head;
+    if (kmax > decode_wave_keys(HD)) {
+        if constexpr (HD == 64) launch_k(k_attend_decode64<NOCLAMP>, dim3(n_rh), dim3(256), 0, stream, a, kmax);
+        else launch_k((k_attend_decode_wg<NOCLAMP, HD>), dim3(n_rh), dim3(HD > 64 ? 512 : 256), 0, stream, a, kmax);
+        return hipGetLastError();
+    }
+    auto run = [&](auto kernel, int kb) {
+        const size_t lds = (size_t)4 * (kb * 64 * HD + 1024);
+        const hipError_t e = lds > 65536 ? allow_dynamic_lds((const void *)kernel, lds) : hipSuccess;
+        if (e != hipSuccess) return e;
+        launch_k(kernel, dim3((n_rh + 3) / 4), dim3(256), lds, stream, a, n_rh, kmax);
+        return hipGetLastError();
+    };
+    const int kb = (kmax + 63) / 64;
+    if (kb <= 1) return run(k_attend_decode_wave<NOCLAMP, 1, HD>, 1);
+    if (kb == 2) return run(k_attend_decode_wave<NOCLAMP, 2, HD>, 2);
+    if constexpr (HD <= 64) {
+        if (kb == 3) return run(k_attend_decode_wave<NOCLAMP, 3, HD>, 3);
+        if (kb == 4) return run(k_attend_decode_wave<NOCLAMP, 4, HD>, 4);
+        if constexpr (HD < 64) return run(k_attend_decode_wave<NOCLAMP, 8, HD>, 8);
+    }
+    return hipErrorInvalidValue;
 }
 
 template <bool NOCLAMP>
-static hipError_t launch_decode_wave(const AttnArgs &a, int n_rows, int kmax, hipStream_t stream) {
-    const int n_rh = n_rows * a.n_head;
-    const dim3 grid((n_rh + 3) / 4);
-    const int kb = (kmax + 63) / 64;
-    const size_t lds = (size_t)4 * (kb * 4096 + 1024);  // 20 to 68 KiB
-    if (kb <= 1) launch_k((k_attend_decode_wave<NOCLAMP, 1>), grid, dim3(256), lds, stream, a, n_rh, kmax);
-    else if (kb == 2) launch_k((k_attend_decode_wave<NOCLAMP, 2>), grid, dim3(256), lds, stream, a, n_rh, kmax);
-    else if (kb == 3) launch_k((k_attend_decode_wave<NOCLAMP, 3>), grid, dim3(256), lds, stream, a, n_rh, kmax);
-    else launch_k((k_attend_decode_wave<NOCLAMP, 4>), grid, dim3(256), lds, stream, a, n_rh, kmax);
-    return hipGetLastError();
+static hipError_t launch_decode_hd(const AttnArgs &a, int n_rows, int kmax, hipStream_t stream) {
+    switch (a.hd) {
+    case 16: return launch_decode<NOCLAMP, 16>(a, n_rows, kmax, stream);
+    case 32: return launch_decode<NOCLAMP, 32>(a, n_rows, kmax, stream);
+    case 64: return launch_decode<NOCLAMP, 64>(a, n_rows, kmax, stream);
+    case 128: return launch_decode<NOCLAMP, 128>(a, n_rows, kmax, stream);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 SplitPlan attend_split_plan(int n_rows, int n_head, int max_keys) {
@@ -2370,7 +2574,7 @@ SplitPlan attend_split_plan(int n_rows, int n_head, int max_keys) {
 
 bool attend_split_one_launch(int hd, int ctx_cap, const SplitPlan &p) {
     const int kmax = p.max_keys < ctx_cap ? p.max_keys : ctx_cap;
-    return hd == 64 && kmax >= 1 && kmax <= 1024;
+    return (hd == 16 || hd == 32 || hd == 64 || hd == 128) && kmax >= 1 && kmax <= 1024;
 }
 
 size_t attend_split_bytes(const AttnArgs &a, int n_rows, const SplitPlan &p) {
@@ -2380,38 +2584,37 @@ size_t attend_split_bytes(const AttnArgs &a, int n_rows, const SplitPlan &p) {
     return al(rh * a.ctx_cap * 4) + 2 * al(rh * p.chunks * 8) + al(rh * p.chunks * a.hd * 8);
 }
 
+template <int HD>
+static void launch_split(const AttnArgs &a, int n_rows, const SplitPlan &p, void *scratch, hipStream_t stream) {
+    const dim3 grid(n_rows * a.n_head, p.chunks);
+    launch_k(k_split_dots<HD>, grid, dim3(64), 0, stream, a, n_rows, p, scratch);
+    if (attn_noclamp(a)) {
+        launch_k(k_split_sum<true>, grid, dim3(64), 0, stream, a, n_rows, p, scratch);
+        launch_k((k_split_pv<true, HD>), grid, dim3(64), 0, stream, a, n_rows, p, scratch);
+    } else {
+        launch_k(k_split_sum<false>, grid, dim3(64), 0, stream, a, n_rows, p, scratch);
+        launch_k((k_split_pv<false, HD>), grid, dim3(64), 0, stream, a, n_rows, p, scratch);
+    }
+}
+
 hipError_t launch_attend_split(const AttnArgs &a, int n_rows, const SplitPlan &p, void *scratch,
                                hipStream_t stream) {
     if (n_rows <= 0) return hipSuccess;
     if (!attend_split_ok(a.hd) || p.chunk_keys % 64 != 0 || p.chunk_keys > 4096) return hipErrorInvalidValue;
     const int kmax = p.max_keys < a.ctx_cap ? p.max_keys : a.ctx_cap;
-    // a wave per (row, head) up to 256 keys (measured, with the butterfly reduction and the
-    // branch-free weights in both kernels: 768 row-heads at 128 keys 10.7 -> 9.6 us per launch
-    // against a workgroup per row-head; 4,096 row-heads of a GPT-2-medium decode pass 42 -> 37 us
-    // before those changes)
-    if (a.hd == 64 && kmax >= 1 && kmax <= 256)
-        return attn_noclamp(a) ? launch_decode_wave<true>(a, n_rows, kmax, stream)
-                               : launch_decode_wave<false>(a, n_rows, kmax, stream);
-    if (attend_split_one_launch(a.hd, a.ctx_cap, p)) {  // one launch, no scratch
-        if (attn_noclamp(a)) launch_k(k_attend_decode64<true>, dim3(n_rows * a.n_head), dim3(256), 0, stream, a, kmax);
-        else launch_k(k_attend_decode64<false>, dim3(n_rows * a.n_head), dim3(256), 0, stream, a, kmax);
-        return hipGetLastError();
-    }
-    const dim3 grid(n_rows * a.n_head, p.chunks);
-    const size_t lds = p.chunk_keys * sizeof(uint32_t);
+    // one launch and no scratch up to 1,024 keys; of it a wave per (row, head) up to 256 keys at
+    // head_dim 64 (measured, with the butterfly reduction and the branch-free weights in both kernels:
+    // 768 row-heads at 128 keys 10.7 -> 9.6 us per launch against a workgroup per row-head; 4,096
+    // row-heads of a GPT-2-medium decode pass 42 -> 37 us before those changes)
+    if (attend_split_one_launch(a.hd, a.ctx_cap, p))
+        return attn_noclamp(a) ? launch_decode_hd<true>(a, n_rows, kmax, stream)
+                               : launch_decode_hd<false>(a, n_rows, kmax, stream);
     switch (a.hd) {
-    case 16: launch_k(k_split_dots<16>, grid, dim3(64), 0, stream, a, n_rows, p, scratch); break;
-    case 32: launch_k(k_split_dots<32>, grid, dim3(64), 0, stream, a, n_rows, p, scratch); break;
-    case 64: launch_k(k_split_dots<64>, grid, dim3(64), 0, stream, a, n_rows, p, scratch); break;
-    case 128: launch_k(k_split_dots<128>, grid, dim3(64), 0, stream, a, n_rows, p, scratch); break;
-    default: launch_k(k_split_dots<256>, grid, dim3(64), 0, stream, a, n_rows, p, scratch); break;
-    }
-    if (attn_noclamp(a)) {
-        launch_k(k_split_sum<true>, grid, dim3(64), 0, stream, a, n_rows, p, scratch);
-        launch_k(k_split_pv<true>, grid, dim3(64), lds, stream, a, n_rows, p, scratch);
-    } else {
-        launch_k(k_split_sum<false>, grid, dim3(64), 0, stream, a, n_rows, p, scratch);
-        launch_k(k_split_pv<false>, grid, dim3(64), lds, stream, a, n_rows, p, scratch);
+    case 16: launch_split<16>(a, n_rows, p, scratch, stream); break;
+    case 32: launch_split<32>(a, n_rows, p, scratch, stream); break;
+    case 64: launch_split<64>(a, n_rows, p, scratch, stream); break;
+    case 128: launch_split<128>(a, n_rows, p, scratch, stream); break;
+    default: launch_split<256>(a, n_rows, p, scratch, stream); break;
     }
     launch_k(k_split_out, dim3(n_rows * a.n_head), dim3(a.hd), 0, stream, a, n_rows, p, scratch);
     return hipGetLastError();
@@ -4509,9 +4712,10 @@ int kernel_resources(KernelResource *out, int cap) {
         {"k_attend_long", (const void *)k_attend_long},
         {"k_attend_mfma<noclamp, lds table>", (const void *)k_attend_mfma<true, true, false>},
         {"k_attend_decode64<noclamp>", (const void *)k_attend_decode64<true>},
-        {"k_attend_decode_wave<noclamp, 4>", (const void *)k_attend_decode_wave<true, 4>},
+        {"k_attend_decode_wg<noclamp, 128>", (const void *)k_attend_decode_wg<true, 128>},
+        {"k_attend_decode_wave<noclamp, 4, 64>", (const void *)k_attend_decode_wave<true, 4, 64>},
         {"k_split_dots<64>", (const void *)k_split_dots<64>},
-        {"k_split_pv<noclamp>", (const void *)k_split_pv<true>},
+        {"k_split_pv<noclamp, 64>", (const void *)k_split_pv<true, 64>},
         {"k_coder_compact", (const void *)k_coder_compact<false, true, false, 256>},
         {"k_coder_compact, few rows with Decode", (const void *)k_coder_compact<false, true, true, 1024>},
         {"k_weights_compact", (const void *)k_weights_compact},
