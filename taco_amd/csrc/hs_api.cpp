@@ -1654,7 +1654,10 @@ extern "C" hs_status hs_op_attend_decode_dev_noalloc(hs_device *dev, const int8_
         return HS_OK;
     }
     const hs::SplitPlan plan = hs::attend_split_plan((int)b, (int)h, (int)ctx_cap);
-    const size_t bytes = hs::attend_split_bytes(at, (int)b, plan);
+    // one limit for every key count at head dims other than 64, the split form's, also where the
+    // plan takes one launch: which calls are refused does not depend on the kernel chosen
+    const size_t bytes = hd == 64 ? hs::attend_split_bytes(at, (int)b, plan)
+                                  : hs::attend_split_partials(at, (int)b, plan);
     if (bytes > HS_FIXED_SCRATCH_BYTES)
         return hs::fail(HS_UNSUPPORTED, 0, "the split attention needs " + std::to_string(bytes) +
                                                " bytes of scratch; the fixed scratch holds " +

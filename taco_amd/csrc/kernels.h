@@ -199,7 +199,9 @@ inline bool attend_split_ok(int hd) { return hd >= 16 && hd <= 256 && (hd & (hd 
 SplitPlan attend_split_plan(int n_rows, int n_head, int max_keys);
 // True when the plan takes a one-launch kernel (head dims up to 128, at most 1,024 keys): no scratch.
 bool attend_split_one_launch(int hd, int ctx_cap, const SplitPlan &p);
-// The scratch bytes of the split launches (0 when the plan takes the one-launch kernel).
+// The bytes of the split launches' partials, whichever form the plan takes.
+size_t attend_split_partials(const AttnArgs &a, int n_rows, const SplitPlan &p);
+// The scratch bytes the plan needs (0 when it takes a one-launch kernel).
 size_t attend_split_bytes(const AttnArgs &a, int n_rows, const SplitPlan &p);
 hipError_t launch_attend_split(const AttnArgs &a, int n_rows, const SplitPlan &p, void *scratch,
                                hipStream_t stream);

@@ -2577,11 +2577,14 @@ bool attend_split_one_launch(int hd, int ctx_cap, const SplitPlan &p) {
     return (hd == 16 || hd == 32 || hd == 64 || hd == 128) && kmax >= 1 && kmax <= 1024;
 }
 
-size_t attend_split_bytes(const AttnArgs &a, int n_rows, const SplitPlan &p) {
-    if (attend_split_one_launch(a.hd, a.ctx_cap, p)) return 0;
+size_t attend_split_partials(const AttnArgs &a, int n_rows, const SplitPlan &p) {
     auto al = [](size_t x) { return (x + 255) / 256 * 256; };
     const size_t rh = (size_t)n_rows * a.n_head;
     return al(rh * a.ctx_cap * 4) + 2 * al(rh * p.chunks * 8) + al(rh * p.chunks * a.hd * 8);
+}
+
+size_t attend_split_bytes(const AttnArgs &a, int n_rows, const SplitPlan &p) {
+    return attend_split_one_launch(a.hd, a.ctx_cap, p) ? 0 : attend_split_partials(a, n_rows, p);
 }
 
 template <int HD>
