@@ -303,11 +303,14 @@ extern "C" hs_status tc_fold_blocks(hs_batch *batch, uint32_t overlap, const uin
             for (size_t wi = w0; wi < std::min(windows.size(), w0 + slots); wi++) r += windows[wi].len + k + 1;
             most = std::max(most, r);
         }
-        if (inputs.size() < most) {  // the vectors only grow: rows past a wave's count are not read
-            inputs.resize(most);
-            queries.resize(most);
-            answers.resize(most);
-        }
+        // The vectors only grow (rows past a wave's count are not read), each by its own size: a call
+        // whose allocation failed leaves some of them shorter than the others.
+        auto hold = [&](auto &v) {
+            if (v.size() < most) v.resize(most);
+        };
+        hold(inputs);
+        hold(queries);
+        hold(answers);
     }
     for (size_t w0 = 0; w0 < windows.size(); w0 += slots) {
         const size_t w1 = std::min(windows.size(), w0 + slots);
