@@ -1069,29 +1069,41 @@ hs_status run_pass(hs_batch &b, const std::vector<PassRow> &rows, Out out, const
         return b.launch(label, ops, [&] { return hs::launch_gemm(epi, g, st); });
     };
     const bool kv_fused = m.hd % 16 == 0 && m.d % 16 == 0;
-    // Decode-shaped passes (short runs): attention split over key chunks when the scratch fits
-    // (at most 1 GiB), else the row kernel.
-    bool split_attn = false;
+    // Decode-shaped passes (short runs) and head dims that the group kernels do not take: attention in
+    // one launch, or split over key chunks, as many rows at a time as 1 GiB of scratch holds; where
+    // the device has no memory for that, the row kernel, which needs none.
+    bool split_attn = !mfma_attn && hs::attend_split_ok(m.hd);
     hs::SplitPlan split_plan;
-    if (!mfma_attn && hs::attend_split_ok(m.hd)) {
+    int split_rows = n;
+    if (split_attn) {
         int max_keys = 1;
-        for (int r = 0; r < n; r++) max_keys = std::max<int>(max_keys, (int)rows[r].pos + 1);
-        split_plan = hs::attend_split_plan(n, m.H, max_keys);
+        int64_t keys = 0;
+        for (int r = 0; r < n; r++) {
+            max_keys = std::max<int>(max_keys, (int)rows[r].pos + 1);
+            keys += (int)rows[r].pos + 1;
+        }
+        split_plan = hs::attend_split_plan(n, m.H, max_keys, (int)(keys / std::max(n, 1)));
         hs::AttnArgs probe;
         probe.n_head = m.H; probe.hd = m.hd; probe.ctx_cap = m.C;
-        const size_t need = hs::attend_split_bytes(probe, n, split_plan);  // 0: one launch
-        if (need <= (1ull << 30)) {
-            if (need > b.split_bytes) {
-                if (b.split) {
-                    HIP_TRY(hipStreamSynchronize(st));
-                    HIP_TRY(hipFree(b.split));
-                    b.split = nullptr;
-                    b.split_bytes = 0;
-                }
-                HIP_TRY(hipMalloc(&b.split, need));
-                b.split_bytes = need;
+        size_t need = hs::attend_split_bytes(probe, n, split_plan);  // 0: one launch
+        if (need > (1ull << 30)) {
+            split_rows = std::max<int>(1, (int)((double)n * (1ull << 30) / (double)need));
+            need = hs::attend_split_bytes(probe, split_rows, split_plan);
+        }
+        if (need > b.split_bytes) {
+            if (b.split) {
+                HIP_TRY(hipStreamSynchronize(st));
+                HIP_TRY(hipFree(b.split));
+                b.split = nullptr;
+                b.split_bytes = 0;
             }
-            split_attn = true;
+            if (hipMalloc(&b.split, need) == hipSuccess) {
+                b.split_bytes = need;
+            } else {
+                (void)hipGetLastError();
+                b.split = nullptr;
+                split_attn = false;
+            }
         }
     }
     for (int l = 0; l < m.L; l++) {
@@ -1123,8 +1135,16 @@ hs_status run_pass(hs_batch &b, const std::vector<PassRow> &rows, Out out, const
         at.out = b.d_att; at.out_rows = RP;
         HIP_TRY(b.launch("attention", 4ull * attn_keys * (uint64_t)m.d, [&] {
             if (mfma_attn) return hs::launch_attend_groups(at, b.d_groups, n_groups, group_keys, st);
-            if (split_attn) return hs::launch_attend_split(at, n, split_plan, b.split, st);
-            return hs::launch_attend(at, n, st);
+            if (!split_attn) return hs::launch_attend(at, n, st);
+            for (int r0 = 0; r0 < n; r0 += split_rows) {
+                hs::AttnArgs c = at;
+                c.rows += r0;
+                c.q += (size_t)r0 * at.ldq;
+                c.out += (size_t)r0 * 64;  // rows of the panels
+                const hipError_t e = hs::launch_attend_split(c, std::min(split_rows, n - r0), split_plan, b.split, st);
+                if (e != hipSuccess) return e;
+            }
+            return hipSuccess;
         }));
         HIP_TRY(gemm("gemm_proj", Epi::Residual, blk.c_proj, b.d_att, RP, n, b.d_x, m.d));
         HIP_TRY(ln(blk.ln2, nullptr, n, b.d_a));

@@ -188,16 +188,19 @@ struct AttnArgs {
 hipError_t launch_attend(const AttnArgs &a, int n_rows, hipStream_t stream);
 
 // Decode attention (head_dim 16, 32, 64, 128 or 256). Head dims up to 128 with at most 1,024 keys: one
-// launch, a wave or a workgroup per (row, head), `scratch` unused. Otherwise split over key chunks: four
+// launch, a wave or a workgroup per (row, head), `scratch` unused (head dim 128 past 128 keys: only where
+// attend_split_one_launch says so). Otherwise split over key chunks: four
 // launches over (row, head, chunk) with exact integer partials in `scratch` (attend_split_bytes
 // bytes, 256-byte aligned). The plan's `max_keys` bounds every row's key count.
 struct SplitPlan {
     int chunks = 1, chunk_keys = 64;
     int max_keys = 0;  // the bound on every row's key count the plan was made for
+    long long row_heads = 0;
+    int mean_keys = 0;  // the rows' mean key count, 0 where the caller does not know it
 };
 inline bool attend_split_ok(int hd) { return hd >= 16 && hd <= 256 && (hd & (hd - 1)) == 0; }
-SplitPlan attend_split_plan(int n_rows, int n_head, int max_keys);
-// True when the plan takes a one-launch kernel (head dims up to 128, at most 1,024 keys): no scratch.
+SplitPlan attend_split_plan(int n_rows, int n_head, int max_keys, int mean_keys = 0);
+// True when the plan takes a one-launch kernel: no scratch.
 bool attend_split_one_launch(int hd, int ctx_cap, const SplitPlan &p);
 // The bytes of the split launches' partials, whichever form the plan takes.
 size_t attend_split_partials(const AttnArgs &a, int n_rows, const SplitPlan &p);

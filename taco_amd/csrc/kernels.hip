@@ -2558,7 +2558,7 @@ static hipError_t launch_decode_hd(const AttnArgs &a, int n_rows, int kmax, hipS
     }
 }
 
-SplitPlan attend_split_plan(int n_rows, int n_head, int max_keys) {
+SplitPlan attend_split_plan(int n_rows, int n_head, int max_keys, int mean_keys) {
     // about 4096 waves over (row, head, chunk), chunks of a multiple of 64 keys
     SplitPlan p;
     const long long rh = (long long)n_rows * n_head;
@@ -2569,12 +2569,27 @@ SplitPlan attend_split_plan(int n_rows, int n_head, int max_keys) {
     p.chunk_keys = p.chunk_keys > 4096 ? 4096 : p.chunk_keys;  // the p values of a chunk in LDS
     p.chunks = (max_keys + p.chunk_keys - 1) / p.chunk_keys;
     p.max_keys = max_keys;
+    p.row_heads = rh;
+    p.mean_keys = mean_keys;
     return p;
 }
 
+// The one-launch kernels. Past 128 keys a row-head of head_dim 128 takes a workgroup of 512 threads that
+// fills a CU for 4 us and more, however few of those keys it has: 3,072 row-heads of 16 to 32 keys in
+// caches of 256 took 48.7 us, 16,384 of them 259 (the four split launches 19.8 and 55.6), and the passes
+// of a prefill, whose rows hold half of the longest one's keys in the mean, 577 us for 32,768
+// row-heads of up to 256 (176 split). So it is for few row-heads (768 at 300 keys 20.2 us, split 29.3;
+// 800 at 500 keys 29.5 and 32.2), and for more of them where the caller knows that most hold many
+// keys (4,096 at 900: 188 and 208; 16,384 at 512 keys: 475 and 456).
+constexpr long long DECODE_WG128_MOST = 1024;
+constexpr int DECODE_WG128_KEYS = 640;
+
 bool attend_split_one_launch(int hd, int ctx_cap, const SplitPlan &p) {
     const int kmax = p.max_keys < ctx_cap ? p.max_keys : ctx_cap;
-    return (hd == 16 || hd == 32 || hd == 64 || hd == 128) && kmax >= 1 && kmax <= 1024;
+    if (kmax < 1 || kmax > 1024) return false;
+    if (hd == 128)
+        return kmax <= decode_wave_keys(hd) || p.row_heads <= DECODE_WG128_MOST || p.mean_keys >= DECODE_WG128_KEYS;
+    return hd == 16 || hd == 32 || hd == 64;
 }
 
 size_t attend_split_partials(const AttnArgs &a, int n_rows, const SplitPlan &p) {
