@@ -810,11 +810,24 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
                 if (EPI == (int)Epi::GeluWide) return (uint32_t)(pl == 0 ? v >> 8 : (v & 255) - 128) & 255;
                 return (uint32_t)v;  // the low byte is packed
             };
-            if (!vec) {  // unaligned output rows: one byte store per output
+            // Unaligned output rows: bytes, or in the 64 x 64 tiles a group of Act in one unaligned store
+            // (256 x 4099 x 6400 32.7 -> 27.9 us). (In 256 x 128 tiles it took 6 to 15% off most products
+            // but made those of just over 256 tiles 5 to 13% slower: 2048 x 4099 x 3000 53 -> 60 us.)
+            if (!vec) {
 #pragma unroll
                 for (int i = 0; i < TI; i++)
 #pragma unroll
-                    for (int j = 0; j < TJ; j++)
+                    for (int j = 0; j < TJ; j++) {
+                        const int n4 = cw + 16 * j + 4 * cg;
+                        if (BM == 64 && EPI == (int)Epi::Act && !g.kv_rows && n4 + 4 <= g.n) {
+                            const int m = rw + 16 * i + rl;
+                            if (m >= M) continue;
+                            uint32_t b = 0;
+#pragma unroll
+                            for (int e = 0; e < 4; e++) b |= (byte_of(acc[i][j][e]) & 255) << (8 * e);
+                            __builtin_memcpy((int8_t *)g.out + (size_t)m * g.ldo + n4, &b, 4);
+                            continue;
+                        }
 #pragma unroll
                         for (int e = 0; e < 4; e++) {
                             const int m = rw + 16 * i + rl, n = cw + 16 * j + 4 * cg + e;
@@ -835,6 +848,7 @@ __global__ __launch_bounds__(64 * gemm_waves(BN)) __attribute__((amdgpu_waves_pe
                                 ((int8_t *)g.out)[panel_off(orow, n, g.out_rows)] = v;
                             }
                         }
+                    }
                 continue;
             }
 #pragma unroll
@@ -941,15 +955,18 @@ static hipError_t launch_gemm_t(const GemmArgs &ga, hipStream_t stream) {
 // 768 (576 tiles) 8.6 -> 6.9, 1536 x 2304 x 768 (864) 8.8 -> 7.5, 2048 x 2304 x 768 (1,152) 9.0
 // -> 9.5; residual 3400 x 768 x 768 (648) 13.9 -> 9.3, 2048 x 768 x 3072 (384) 24.6 -> 17.8,
 // 1536 x 1600 x 6400 (600) 42.3 -> 32.1, 2048 x 1600 x 6400 (800) 42.8 -> 51.7: the line lies
-// lower for long K, where the larger tiles' fewer loads per output count for more.
+// lower for long K, where the larger tiles' fewer loads per output count for more. Rows that are not
+// 16-byte aligned change the stores alone, so the same lines hold for them (256 x 4099 x 6400: 67 us in
+// 256 x 128 tiles, 28 here; 512 x 5000 x 3000 47 -> 18;
+// 1024 x 3001 x 1024 34 -> 10).
 static bool gemm_small_tiles(int m, int n, int k_pad) {
     const long long tiles = ((m + 63) / 64) * (long long)((n + 63) / 64);
     return m <= 2 * GEMM_BM || tiles <= (k_pad <= 1024 ? 900 : 640);
 }
 
 // 256 x 128 tiles (two workgroups per CU, so one's epilogue overlaps the other's main loop),
-// or 256 x 256 (below). Outputs whose rows are not 16-byte aligned take the per-output store
-// path.
+// or 256 x 256 (below). Outputs whose rows are not 16-byte aligned take the store path without staging,
+// in 64 x 64 or 256 x 128 tiles.
 template <int EPI, bool NARROW>
 static hipError_t launch_gemm_w(const GemmArgs &g, hipStream_t stream) {
     {
@@ -960,14 +977,19 @@ static hipError_t launch_gemm_w(const GemmArgs &g, hipStream_t stream) {
         // (the GELU outputs are panels of 64-byte rows: aligned when the base is)
         constexpr bool PANEL_OUT = EPI == (int)Epi::Gelu || EPI == (int)Epi::GeluWide;
         const bool vec = ((uintptr_t)g.out & 15) == 0 && (PANEL_OUT || ((size_t)g.ldo * ES) % 16 == 0);
-        if (!vec) return launch_gemm_t<EPI, NARROW, 128, false>(g, stream);
         if constexpr (EPI == (int)Epi::Act || RESIDUAL || EPI == (int)Epi::Gelu || EPI == (int)Epi::GeluWide ||
                       EPI == (int)Epi::Raw) {
             if (gemm_small_tiles(g.m, g.n, g.k_pad)) {
-                if (g.k_pad >= 1024) return launch_gemm_t<EPI, NARROW, 64, true, 64, true>(g, stream);
-                return launch_gemm_t<EPI, NARROW, 64, true, 64>(g, stream);
+                if constexpr (!PANEL_OUT)
+                    if (!vec)
+                        return g.k_pad >= 1024 ? launch_gemm_t<EPI, NARROW, 64, false, 64, true>(g, stream)
+                                               : launch_gemm_t<EPI, NARROW, 64, false, 64>(g, stream);
+                if (vec)
+                    return g.k_pad >= 1024 ? launch_gemm_t<EPI, NARROW, 64, true, 64, true>(g, stream)
+                                           : launch_gemm_t<EPI, NARROW, 64, true, 64>(g, stream);
             }
         }
+        if (!vec) return launch_gemm_t<EPI, NARROW, 128, false>(g, stream);
         // 256 x 256 tiles (one workgroup per CU, full-line 128-k stages) for long K, where their
         // faster main loop outweighs the lost overlap of a second workgroup per CU and the
         // coarser rounds (measured: GPT-2 small mlp.c_proj, K 3,072, 12% faster; c_attn and the
