@@ -198,13 +198,6 @@ HS_HD float ln_half_dist(float z) {
 #endif
 }
 HS_HD float ln_margin(float max_beta) { return (3.01f * (128.0f + max_beta) + 257.0f) * 0x1p-24f; }
-// One element as an integer, from b = 1/2 + beta with |beta| <= 256 (ln_margin(256) < 2^-13).
-// Returns false (declines) near a half; *out is then unused.
-HS_HD bool ln_elem_f32(int32_t c, float k, float b, int32_t *out) {
-    const float z = ln_elem_z(c, k, b + 127.5f);
-    *out = (int32_t)rintf(z) - 128;
-    return fabsf(ln_half_dist(z)) >= 0x1p-13f;
-}
 
 // floor((c inv gamma m + 2^(s - 1)) / 2^s) (the LayerNorm element rule, layernorm.rs:66-108,
 // s <= 126) in double precision, with kr = ldexp((double)inv * m, -s) of the row:

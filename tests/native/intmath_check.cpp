@@ -238,20 +238,20 @@ int main(int argc, char **argv) {
                 count += 3;
             }
     CHECK(taken > n / 2, "ln_elem_f64 declined too often (%ld of %ld)", declined, declined + taken);
-    // ln_elem_f32 against clamp(floor((c inv gamma m + 2^(s-1)) / 2^s) + beta, +-127) in i128 for
-    // |beta| <= 256, with k and b formed as the kernel forms them: every value it returns is exact.
+    // ln_elem_z with ln_margin against clamp(floor((c inv gamma m + 2^(s-1)) / 2^s) + beta, +-127) in i128
+    // for |beta| <= 256, with k and b formed as the kernel forms them: every value it keeps is exact.
     long declined32 = 0, taken32 = 0;
     auto check_ln32 = [&](int32_t c, uint64_t inv, int32_t g, int32_t m, uint32_t s, int32_t beta) -> bool {
         const float krf = (float)std::ldexp((double)inv * (double)m, -(int)s);
-        int32_t y = 0;
-        if (!hs::ln_elem_f32(c, krf * (float)g, 0.5f + (float)beta, &y)) {
+        const float z = hs::ln_elem_z(c, krf * (float)g, 128.0f + (float)beta);
+        if (std::fabs(hs::ln_half_dist(z)) < hs::ln_margin(256.0f)) {
             declined32++;
             return true;
         }
         taken32++;
         i128 want = exact_ln(c, inv, g, m, s) + beta;
         want = want < -127 ? -127 : (want > 127 ? 127 : want);
-        return (i128)y == want;
+        return (i128)((int32_t)std::rint(z) - 128) == want;
     };
     for (long i = 0; i < n; i++) {
         const int32_t c = (int32_t)(next() >> (33 + next() % 31)) * ((next() & 1) ? -1 : 1);
@@ -264,7 +264,7 @@ int main(int argc, char **argv) {
         if (room < 64) inv = room <= 0 ? 0 : inv & ((1ull << room) - 1);
         const uint32_t s = (uint32_t)(next() % 127);
         const int32_t beta = (int32_t)(next() % 513) - 256;
-        CHECK(check_ln32(c, inv, g, m, s, beta), "ln_elem_f32 c %d inv %llu g %d m %d s %u beta %d", c,
+        CHECK(check_ln32(c, inv, g, m, s, beta), "ln_elem_z c %d inv %llu g %d m %d s %u beta %d", c,
               (unsigned long long)inv, g, m, s, beta);
         count++;
     }
@@ -275,12 +275,12 @@ int main(int argc, char **argv) {
                 const i128 p = (i128)k * ((i128)1 << s) + ((i128)1 << (s - 1)) + delta;
                 if (p <= 0 || p >= ((i128)1 << 64)) continue;
                 for (int32_t beta : {-256, -130, -1, 0, 1, 127, 256}) {
-                    CHECK(check_ln32(1, (uint64_t)p, 1, 1, s, beta), "ln_elem_f32 half s %u k %ld d %d b %d", s, k, delta, beta);
-                    CHECK(check_ln32(-1, (uint64_t)p, 1, 1, s, beta), "ln_elem_f32 -half s %u k %ld d %d b %d", s, k, delta, beta);
+                    CHECK(check_ln32(1, (uint64_t)p, 1, 1, s, beta), "ln_elem_z half s %u k %ld d %d b %d", s, k, delta, beta);
+                    CHECK(check_ln32(-1, (uint64_t)p, 1, 1, s, beta), "ln_elem_z -half s %u k %ld d %d b %d", s, k, delta, beta);
                     count += 2;
                 }
             }
-    CHECK(taken32 > n / 2, "ln_elem_f32 declined too often (%ld of %ld)", declined32, declined32 + taken32);
+    CHECK(taken32 > n / 2, "ln_elem_z declined too often (%ld of %ld)", declined32, declined32 + taken32);
     // softmax_p_of: floor(e 2^P / S) for e <= S, e < 2^31, S < 2^53, P <= 30; random rows and
     // entries on, just below and just above the multiples of S / 2^P
     auto check_p = [&](uint32_t e, uint64_t S, int P) -> bool {
