@@ -1,6 +1,7 @@
 """The LM head of few rows (k_head_rows): row counts at the edges of its 16-row tiles and at its line
-against the tiles (64 and 65 rows), its 8- and 16-wave workgroups (their LDS line at 64 KiB and K past
-the steps in flight), vocabularies that end inside a 4-column group and inside a 64-column tile, and
+against the tiles (64 and 65 rows), its 8- and 16-wave workgroups for 16, 32 and 64 rows (their LDS line at
+64 KiB: widths of 1,088, 2,112 and 4,160 cross it, the last past the LDS for 64 rows; K past the steps in
+flight), vocabularies that end inside a 4-column group and inside a 64-column tile, and
 both rescales (a logits shift of 31 or more, and below), against the CPU fast path."""
 
 import numpy as np
@@ -12,7 +13,8 @@ from tests.conftest import splitmix_tokens
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("heads,vocab,general", [(1, 1502, False), (1, 1502, True), (12, 131, False), (17, 1001, False)])
+@pytest.mark.parametrize("heads,vocab,general", [(1, 1502, False), (1, 1502, True), (12, 131, False), (17, 1001, False),
+                                                 (33, 500, False), (33, 500, True), (65, 333, False), (65, 333, True)])
 def test_few_rows_of_logits(monkeypatch, heads, vocab, general):
     from taco_amd import hip, synth
     d, plain = 64 * heads, synth.shift_for
