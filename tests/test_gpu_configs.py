@@ -247,16 +247,16 @@ def test_layernorm_forms_equal_the_cpu(dev, name, windows, n):
         assert len(bad) == 0, f"{name}, window {w}: {len(bad)} rows differ, first {bad[:8].tolist()}"
 
 
-# Split-K products in decode-shaped passes: passes of at most 512 rows whose mlp.c_proj has
-# K = d_ff > 4,096 run k_gemm<Raw> partials over K slices and the summing pass k_split_epi with
-# the Residual rule (GPT-2 XL's mlp.c_proj, K 6,400, in every unfold pass).
+# Long K in decode-shaped passes: passes of at most 512 rows whose mlp.c_proj has K = d_ff > 4,096
+# split K over the waves of a workgroup, whose partial tiles meet in LDS before the Residual rule
+# (GPT-2 XL's mlp.c_proj, K 6,400, in every unfold pass).
 SPLIT_MODELS = {"d256_f6400": (1, 4, 256, 6400), "d1600_f6400": (1, 25, 1600, 6400)}
 
 
 @pytest.mark.parametrize("name", sorted(SPLIT_MODELS))
 def test_split_k_residual_passes_equal_the_cpu(dev, name):
-    """4 windows of 128 tokens: a first pass of 4 x 96 rows (384 rows, 12 or more K slices),
-    then one row per slot per pass (4-row passes, 16 slices), every interval against the CPU
+    """4 windows of 128 tokens: a first pass of 4 x 96 rows (384 rows: 64 x 32 and 64 x 64 tiles),
+    then one row per slot per pass (4-row passes: 16 x 16 tiles), every interval against the CPU
     fast path's."""
     from taco_amd import hip, synth
     L, H, d, f = SPLIT_MODELS[name]
