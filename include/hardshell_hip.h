@@ -278,8 +278,11 @@ hs_status hs_op_attend_decode_dev(hs_device *dev, const int8_t *q, const int8_t 
  * callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc). The split launches keep their partials in a fixed
  * 64 MiB array per GPU (held until the process ends) instead of stream-ordered allocations;
- * a shape that needs more (row-heads x ctx_cap x 4 bytes plus the chunk partials) is refused
- * with HS_UNSUPPORTED. Calls that overlap on one GPU share that array and race. */
+ * a shape whose partials (row-heads x ctx_cap x 4 bytes plus those of the chunks) are more than
+ * that is refused with HS_UNSUPPORTED. The limit holds at head dims 16, 32, 128 and 256 for every
+ * shape, also one that a single launch serves without partials; at head dim 64 only past 1,024
+ * keys; at other head dims there is none. Split launches that overlap on one GPU share that
+ * array and race. */
 hs_status hs_op_attend_decode_dev_noalloc(hs_device *dev, const int8_t *q, const int8_t *k_cache,
                                           const int8_t *v_cache, const uint32_t *ctx, size_t b,
                                           size_t h, size_t hd, size_t ctx_cap, int32_t score_m,

@@ -1674,8 +1674,9 @@ extern "C" hs_status hs_op_attend_decode_dev_noalloc(hs_device *dev, const int8_
         return HS_OK;
     }
     const hs::SplitPlan plan = hs::attend_split_plan((int)b, (int)h, (int)ctx_cap);
-    // one limit for every key count at head dims other than 64, the split form's, also where the
-    // plan takes one launch: which calls are refused does not depend on the kernel chosen
+    // The limit of the header: the split form's partials, at head dims other than 64 also where the plan
+    // takes one launch, which uses none. Callers sized to the limit see the same refusals whichever
+    // kernel a build or a plan picks; head_dim 64 was always one launch up to 1,024 keys.
     const size_t bytes = hd == 64 ? hs::attend_split_bytes(at, (int)b, plan)
                                   : hs::attend_split_partials(at, (int)b, plan);
     if (bytes > HS_FIXED_SCRATCH_BYTES)

@@ -58,8 +58,8 @@ def _case(seed, B, H, cap, hd):
 
 
 # (streams, heads, positions, head_dim) of the first call, then of the second (smaller) call:
-# split-key kernels (head dims 16 to 256, head_dim 64 past 1,024 keys), the one-launch kernel
-# (head_dim 64, at most 1,024 keys) and the row kernel (head_dim 48).
+# split-key kernels (head_dim 256, head_dim 64 past 1,024 keys), the one-launch kernels (head dims 16, 64
+# and 128, at most 1,024 keys) and the row kernel (head_dim 48).
 SHAPES = [
     ((16, 12, 2048, 64), (3, 12, 1100, 64)),
     ((8, 12, 600, 16), (2, 5, 70, 16)),
@@ -85,20 +85,21 @@ def test_noalloc_equals_the_allocating_entry(dev, first, second):
             assert np.array_equal(got, ref), f"call {i + 1} {shape} against the oracle"
 
 
-def test_noalloc_refuses_partials_beyond_the_fixed_scratch(dev):
+@pytest.mark.parametrize("b,h,cap,hd", [(1, 1, 20_000_000, 16), (1250, 16, 1024, 32)])
+def test_noalloc_refuses_partials_beyond_the_fixed_scratch(dev, b, h, cap, hd):
     """One stream, one head of 16 over 20M positions needs 80 MB of dots: refused with
-    HS_UNSUPPORTED before any launch (the caches are allocated and never read)."""
+    HS_UNSUPPORTED before any launch (the caches are allocated and never read). The limit is the same for
+    20,000 row-heads of 1,024 keys at head_dim 32, which one launch would serve without partials."""
     from taco_amd import hip
     L = hip.lib()
-    cap, hd = 20_000_000, 16
     ptrs = []
-    for nbytes in (hd, cap * hd, cap * hd, 4 * len(TABLE), hd):
+    for nbytes in (b * h * hd, b * h * cap * hd, b * h * cap * hd, 4 * len(TABLE), b * h * hd):
         p = C.c_void_p()
         hip._check(L.hs_device_alloc(dev.h, nbytes, C.byref(p)))
         ptrs.append(p)
-    ctx = _dev_buf(dev, np.array([cap], np.uint32))
+    ctx = _dev_buf(dev, np.full(b, cap, np.uint32))
     try:
-        st = L.hs_op_attend_decode_dev_noalloc(dev.h, ptrs[0], ptrs[1], ptrs[2], ctx, 1, 1, hd,
+        st = L.hs_op_attend_decode_dev_noalloc(dev.h, ptrs[0], ptrs[1], ptrs[2], ctx, b, h, hd,
                                                cap, SCORE_M, SCORE_S, OUT_M, OUT_S, ptrs[3],
                                                len(TABLE), 30, ptrs[4], None)
         assert st == hip.HS_UNSUPPORTED
