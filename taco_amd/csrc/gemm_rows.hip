@@ -260,7 +260,8 @@ static hipError_t launch_rows_t(const GemmArgs &g, hipStream_t stream) {
 // 5.3 -> 4.8), three only where k_gemm's epilogue is a slow one (the residual one: 1024 x 768 x 768
 // 7.2 -> 6.3; the one for products without the i32 bound: 256 x 2304 x 768 8.2 -> 5.9); past that
 // the loads per output decide and k_gemm is faster. With longer K the 64-row tiles take over at one
-// round (512 x 768 x 3072: 12.8 -> 8.2).
+// round (512 x 768 x 3072: 12.8 -> 8.2). What needs more than one round of those takes the 64 x 64 LDS
+// tiles (512 x 4096 x 6400, two slices of K and a summing pass before: 35 -> 29).
 struct RowsTile {
     int mt = 0, nt = 0;
 };
@@ -319,7 +320,8 @@ hipError_t launch_gemm_rows(Epi epi, const GemmArgs &g, hipStream_t stream) {
 // conflicts), and each wave takes 16 columns over all of K with U k-steps of W in flight in
 // registers. Every wave holding A from the caches instead read 4 bytes of it for each byte of W:
 // 18.6 us at 64 rows. A row's tile max meets over the 4 waves of a 64-column tile in LDS.
-// Measured against the tiles of k_gemm, us a launch: width 768 1 row 15.8 -> 8.2, 16 rows 15.9 -> 8.5,
+// Measured against the tiles of k_gemm, us a launch of the head alone, wte in the Infinity Cache (inside a
+// token step 16.1 -> 9.6 us, inside a 64-row decode pass 20.3 -> 14.6): width 768 1 row 15.8 -> 8.2, 16 rows 15.9 -> 8.5,
 // 32 rows 16.5 -> 9.6, 64 rows 17.6 -> 12.2; width 1024 1 row 19.0 -> 11.2, 64 rows 20.5 -> 15.6;
 // width 1600 1 row 29.3 -> 17.3, 64 rows 31.3 -> 22.2. 128 rows (128 accumulated rows a wave): 20.3 ->
 // 19.5 at width 768 but 32.9 -> 41 at 1600, so more than 64 rows stay with the tiles.

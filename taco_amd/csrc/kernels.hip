@@ -1785,9 +1785,6 @@ __device__ __forceinline__ int32_t dot_key(const int *q4, const int8_t *k, int h
     return s;
 }
 
-// The output of row r at column col: row-major (ldo) for the op entries, or the operand panels
-// of the next product (out_rows > 0). Groups of up to 16 columns from a multiple of 16 (of 4
-// for 4-byte groups) lie in one panel.
 __global__ __launch_bounds__(256) void k_attend(AttnArgs a, int n_tasks) {
     __shared__ __attribute__((aligned(16))) int s_q[4][64];  // hd <= 256 bytes per wave
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -2174,9 +2171,10 @@ __device__ __forceinline__ uint64_t wave_sum_dpp(uint64_t v) {
 // loads with no branch around them, K first, so the dots wait for K alone (the compiler counts the
 // in-order loads exactly; with part of V going to LDS by global_load_lds it waited for every
 // load); the dots, the row max, the table sum, the weights p and the sums p v then follow the rules
-// of the split kernels above. 140 VGPRs: three workgroups per CU (768 row-heads in one round). Measured at 1,024 keys and 768 row-heads:
-// 34.2 us with all of V in LDS (two workgroups per CU), 31.0 with half, then 29.8 -> 27.9 with
-// the butterfly reduction.
+// of the split kernels above. 140 VGPRs: three workgroups per CU (768 row-heads in one round). Measured
+// at 768 row-heads over cold caches: 1,024 keys 20.2 us (100.8 MB: 5.0 TB/s), 512 keys 12.4. What the layout
+// rests on, at 1,024 keys with the sums p v still on 24-bit multiplies: 34.2 us with all of V in LDS
+// (two workgroups per CU), 31.0 with half, 29.8 with none.
 template <bool NOCLAMP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_attend_decode64(AttnArgs a,
                                                                                                   int kmax) {
@@ -2588,7 +2586,9 @@ SplitPlan attend_split_plan(int n_rows, int n_head, int max_keys, int mean_keys)
     int want = (int)((4096 + rh - 1) / (rh > 0 ? rh : 1));
     want = want < 1 ? 1 : (want > blocks64 ? blocks64 : want);
     p.chunk_keys = 64 * ((blocks64 + want - 1) / want);
-    p.chunk_keys = p.chunk_keys > 4096 ? 4096 : p.chunk_keys;  // the p values of a chunk in LDS
+    // One wave walks a chunk from end to end, so a chunk holds at most 64 blocks of keys, however many
+    // row-heads there are (the i32 sums of k_split_pv's digit planes would hold 32 times as many).
+    p.chunk_keys = p.chunk_keys > 4096 ? 4096 : p.chunk_keys;
     p.chunks = (max_keys + p.chunk_keys - 1) / p.chunk_keys;
     p.max_keys = max_keys;
     p.row_heads = rh;
@@ -2643,9 +2643,9 @@ hipError_t launch_attend_split(const AttnArgs &a, int n_rows, const SplitPlan &p
     if (!attend_split_ok(a.hd) || p.chunk_keys % 64 != 0 || p.chunk_keys > 4096) return hipErrorInvalidValue;
     const int kmax = p.max_keys < a.ctx_cap ? p.max_keys : a.ctx_cap;
     // one launch and no scratch up to 1,024 keys; of it a wave per (row, head) up to 256 keys at
-    // head_dim 64 (measured, with the butterfly reduction and the branch-free weights in both kernels:
-    // 768 row-heads at 128 keys 10.7 -> 9.6 us per launch against a workgroup per row-head; 4,096
-    // row-heads of a GPT-2-medium decode pass 42 -> 37 us before those changes)
+    // head_dim 64 (768 row-heads at 128 keys 9.6 us a launch where a workgroup per row-head took 10.7, 4,096
+    // row-heads of a GPT-2-medium decode pass 37 against 42, both with the sums p v on 24-bit multiplies;
+    // the wave form now takes 5.8 us for the first)
     if (attend_split_one_launch(a.hd, a.ctx_cap, p))
         return attn_noclamp(a) ? launch_decode_hd<true>(a, n_rows, kmax, stream)
                                : launch_decode_hd<false>(a, n_rows, kmax, stream);

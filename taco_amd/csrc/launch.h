@@ -73,6 +73,9 @@ __device__ __forceinline__ void lds_barrier() {
     asm volatile("" ::: "memory");
 }
 
+// Attention: the output of row r at column col: row-major (ldo) for the op entries, or the operand panels
+// of the next product (out_rows > 0). Groups of up to 16 columns from a multiple of 16 (of 4
+// for 4-byte groups) lie in one panel.
 __device__ __forceinline__ int8_t *attn_out(const AttnArgs &a, int r, int col) {
     return a.out + (a.out_rows ? panel_off(r, col, a.out_rows) : (size_t)r * a.ldo + col);
 }
