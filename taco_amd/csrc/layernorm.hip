@@ -162,7 +162,7 @@ bool layernorm_f32_fits(const LnArgs &a) { return a.gf && a.bits == 8 && a.d % 4
 // or slower). Against the kernels that served these rows before, us a launch of the op alone, its
 // operands still in the caches: 768 columns, 1 row 5.6 -> 2.7, 256 rows 6.0 -> 4.4, 3,400 10.6 -> 7.0,
 // 16,384 21.2 -> 15.7; 1,024 columns, 24,576 rows 48.6 -> 24.6; 1,600 columns, 6,600 rows 27.1 -> 14.9.
-// Inside a fold, 16,384 rows of 768 take 16.2 to 17.1 us (63 MB: 3.7 to 3.9 TB/s). Two rows a wave
+// Inside a fold, 16,384 rows of 768 take 16 to 18 us (63 MB: 3.5 to 3.9 TB/s). Two rows a wave
 // are better only where a row leaves lanes idle and there are many (384 columns, 24,576 rows:
 // 14.1 against 17.9); four rows a wave, the earlier split, nowhere (768 columns, 16,384 rows 18.2).
 hipError_t launch_layernorm_f32(const LnArgs &a, int n_rows, hipStream_t stream) {
